@@ -3,16 +3,11 @@
 // Algorithm: right-looking blocked LU with partial pivoting, outer block width NB.
 // Reference: src/sgetrf/real_lu_blocked_kernel.cpp:1469-1499 (BlockedFactorLaunch::Run:
 // panel, swap+TRSM, trailing product per block). The MI355X design:
-//   * panel: a sequence of register-resident leaf factorizations (leaf_getf2_kernel), one
-//     workgroup of 256/1024 threads holding every active row of W panel columns in VGPRs.
-//     Per column the pivot is a 64-bit (|a|, position) key argmax: DPP within the wave,
-//     then the wave winners through LDS with one barrier; the row swap, the scaling and
-//     the rank-1 update never leave the CU. Pivot rule, zero-pivot info and reciprocal scaling follow
-//     src/sgetrf/real_lu_blocked_kernel.cpp:342-389, :467-482 and
-//     src/utils/kernel/real_lu.hpp:419-437.
-//   * the panel is halved recursively down to leaves; each leaf applies its row
-//     interchanges to the other panel columns itself (a gather/scatter of the <= 2W moved
-//     rows), and every split solves the right half's top rows with the left half's L11
+//   * panel: a sequence of register-resident leaf factorizations (leaf.hip) of up to 64
+//     columns, one workgroup or, for tall panels, several.
+//   * the panel is halved recursively down to leaves; the interchanges of a leaf (a
+//     gather/scatter of the <= 128 moved rows) are applied to the other panel columns, and
+//     every split solves the right half's top rows with the left half's L11
 //     and updates the rest of the right half with one MFMA product.
 //   * after the panel, the composed interchanges of all NB pivots are applied to every
 //     column outside the panel (one coalesced gather/scatter per column), then the NB x NB
@@ -26,6 +21,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "leaf.h"
 #include "lu_kernels.h"
 #include "trsv.h"
 #include "tslu.h"
@@ -36,23 +32,18 @@ namespace ops
 namespace
 {
 
-constexpr int kMaxRows = 16384;  // largest m the register-resident leaf supports
+constexpr int kMaxRows = kLeafMultiRows;  // largest m the register-resident leaves support
 
 // Workspace layout (ints): [0, m) panel row sources; two moved-row lists of 4*NBMAX + 8
 // (panel k uses list k % 2, so the look-ahead panel can build its list while the previous
 // one is still being applied); then the global permutation (m ints).
 constexpr int NBMAX = 512;
 constexpr int kMovedInts = 4 * NBMAX + 8;
-// After the ints (8-byte aligned): the exchange slots of the multi-workgroup leaf and its
-// timeout flag. Slots are tagged 64-bit words, per column parity: the workgroups' keys
-// (one word each: 16-bit tag, 32-bit magnitude, 16-bit position rank; contiguous, so one
-// poll of all keys touches few cache lines), then their candidate rows (kRowWords words
-// each: 32-bit tag, 32-bit value).
-constexpr int kRowWords = 64;        // per workgroup: up to 64 row words
-constexpr int kMaxLeafGroups = 128;  // workgroups of one multi-workgroup leaf
-constexpr int kKeyWords = 2 * kMaxLeafGroups;  // both parities
-constexpr size_t kSlotBytes =
-    (static_cast<size_t>(kKeyWords) + 2ull * kMaxLeafGroups * kRowWords) * sizeof(unsigned long long);
+// After the ints (8-byte aligned): the exchange words of the multi-workgroup leaves, the
+// moved-row list of the one-workgroup leaves, and the timeout flag.
+constexpr size_t kSlotBytes = (256 + 2ull * 128 * 64) * sizeof(unsigned long long);
+static_assert((kLeafSlotWords * 2 + kLeafMoveInts) * sizeof(int) <= kSlotBytes, "leaf words");
+constexpr int kProbeGroups = 8 * 128;  // workgroups of the placement probe
 constexpr size_t kLinvPanelBytes = (NBMAX / 64) * 4096 * sizeof(float);  // block inverses of one panel's L11
 struct Work
 {
@@ -62,6 +53,7 @@ struct Work
     int* composed;  // m ints: composed row map of the deferred interchanges
     int* perm;
     unsigned long long* slots;
+    int* leafMoves;
     int* err;
     unsigned* epoch;       // host counter: tag base of the next multi-workgroup leaf
     float* linvNode;       // block inverses for the panel-internal solves (panel stream only)
@@ -85,6 +77,7 @@ inline Work Layout(void* base, int m)
     uintptr_t q = reinterpret_cast<uintptr_t>(p + WorkInts(m));
     q = (q + 7) & ~static_cast<uintptr_t>(7);
     w.slots = reinterpret_cast<unsigned long long*>(q);
+    w.leafMoves = reinterpret_cast<int*>(w.slots + kLeafSlotWords);
     w.err = reinterpret_cast<int*>(q + kSlotBytes);
     w.epoch = nullptr;
     q = (q + kSlotBytes + 16 + 255) & ~static_cast<uintptr_t>(255);
@@ -94,540 +87,6 @@ inline Work Layout(void* base, int m)
     w.tslu = reinterpret_cast<void*>(q + 3 * kLinvPanelBytes);
     w.tournament = false;
     return w;
-}
-
-// ---------------------------------------------------------------------------------------
-// Leaf factorization: columns [c0, c0 + wact) of rows [c0, m), T threads, R rows per
-// thread (row tid + i*T), W >= wact columns in registers. Pivoting is implicit: each row
-// tracks the position it occupies under the LAPACK interchange sequence, the pivot of
-// column j is the candidate (position >= j) with the largest |a| and, on ties, the lowest
-// position -- the first-row rule of a physical swap. Per column: one 64-bit key argmax
-// per thread, a DPP wave argmax, and one barrier, after which every thread reads the
-// wave winners' keys and the chosen candidate's row from LDS (double-buffered by column
-// parity, so one barrier per column suffices). At the end each row is stored at its final
-// position, which applies the interchanges to the leaf columns.
-// ---------------------------------------------------------------------------------------
-// FULL: wact == W, so no column of the unrolled loop is skipped at run time (a skip path
-// would make the compiler keep two copies of the row registers alive per column).
-template <int T, int R, int W, bool FULL>
-__global__ __launch_bounds__(T) void leaf_getf2_kernel(float* __restrict__ A, int lda, int m, int j0, int c0, int wact,
-                                                       int panelEnd, int pivoting, int newPanel,
-                                                       int* __restrict__ ipiv, int* __restrict__ info,
-                                                       int* __restrict__ rowsrc)
-{
-    constexpr int NW = T / 64;
-    constexpr int MOVES = 2 * W;  // a leaf moves at most 2 * wact rows
-    __shared__ unsigned long long s_key[2][NW];
-    __shared__ float s_row[2][NW][W];
-    __shared__ int s_count;
-    __shared__ int s_mdst[MOVES], s_msrc[MOVES];
-
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int mp = m - c0;
-    float* Ap = A + static_cast<size_t>(c0) * lda + c0;
-
-    float a[R][W];
-    int pos[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        const bool valid = lr < mp;
-#pragma unroll
-        for (int j = 0; j < W; ++j) a[i][j] = (valid && j < wact) ? Ap[static_cast<size_t>(j) * lda + lr] : 0.0f;
-        pos[i] = valid ? lr : -1;  // padding rows: never a candidate, never below a pivot
-    }
-    if (tid == 0) s_count = 0;
-    int zeroCol = 0;
-
-#pragma unroll
-    for (int j = 0; j < W; ++j)
-    {
-        if (FULL || j < wact)  // uniform
-        {
-            const int par = j & 1;
-            // Candidate of this thread: its best row (or, without pivoting, the row at j),
-            // as a 64-bit key (|a| bits + 1, then ~position, so the lowest position wins
-            // magnitude ties). NaN: on the diagonal position it is the pivot (0x7fffffff),
-            // elsewhere it never wins (0) -- src/utils/kernel/real_lu.hpp:59-77, :100-109.
-            unsigned long long best = 0ull;
-            int bi = -1;
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                const bool cand = pivoting ? pos[i] >= j : pos[i] == j;
-                const unsigned ab = __float_as_uint(fabsf(a[i][j]));
-                const unsigned mag = ab <= 0x7f800000u ? ab + 1u : (pos[i] == j ? 0x7fffffffu : 0u);
-                const unsigned long long k =
-                    cand ? (1ull << 63) | (static_cast<unsigned long long>(mag) << 32) | static_cast<unsigned>(~pos[i])
-                         : 0ull;
-                bi = k > best ? i : bi;
-                best = k > best ? k : best;
-            }
-            const unsigned long long wmax = WaveMaxU64Split(best);
-            if (best == wmax && bi >= 0)  // the wave's winner (keys are unique per position)
-            {
-                s_key[par][wid] = wmax;
-                // Selected by a bit of a mask, not by i == bi: the compiler would turn the
-                // equality into a[bi][k], a run-time row index that puts a[][] in scratch.
-                const unsigned bsel = 1u << bi;
-#pragma unroll
-                for (int k = 0; k < W; ++k)
-                {
-                    float v = a[0][k];
-#pragma unroll
-                    for (int i = 1; i < R; ++i) v = (bsel >> i) & 1u ? a[i][k] : v;
-                    s_row[par][wid][k] = v;
-                }
-            }
-            if (lane == 0 && wmax == 0ull) s_key[par][wid] = 0ull;
-            __syncthreads();
-            unsigned long long top = s_key[par][0];
-            int tw = 0;
-#pragma unroll
-            for (int w = 1; w < NW; ++w)
-            {
-                const unsigned long long kw = s_key[par][w];
-                if (kw > top)
-                {
-                    top = kw;
-                    tw = w;
-                }
-            }
-            const int bpos = top == 0ull ? j : static_cast<int>(~static_cast<unsigned>(top & 0xffffffffull));
-            float prow[W];
-#pragma unroll
-            for (int k = 0; k < W; ++k) prow[k] = s_row[par][tw][k];
-            // Positions j and bpos are exchanged.
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                if (pos[i] == bpos)
-                    pos[i] = j;
-                else if (pos[i] == j)
-                    pos[i] = bpos;
-            }
-            if (tid == 0 && ipiv != nullptr) ipiv[c0 + j] = c0 + bpos + 1;
-            // The pivot is the same in every thread: made uniform, the reciprocal / division
-            // choice is a scalar branch and the division sequence runs only for a subnormal
-            // pivot.
-            const float d = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(prow[j])));
-            if (d == 0.0f && zeroCol == 0) zeroCol = c0 + j + 1;
-            // Branch-free update: rows that are not below the pivot take l = 0, for which
-            // the FMA leaves them unchanged (a zero pivot skips the column likewise).
-            const bool recip = fabsf(d) >= FLT_MIN;  // uniform
-            const float r = 1.0f / d;
-            float q[R];
-            if (recip)
-#pragma unroll
-                for (int i = 0; i < R; ++i) q[i] = a[i][j] * r;
-            else
-#pragma unroll
-                for (int i = 0; i < R; ++i) q[i] = a[i][j] / d;
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                const bool below = pos[i] > j && d != 0.0f;
-                const float l = below ? q[i] : 0.0f;
-                a[i][j] = below ? q[i] : a[i][j];
-#pragma unroll
-                for (int k = 1; k < W; ++k)  // constant bounds: unrolled with the j loop
-                    if (k > j) a[i][k] = fmaf(-l, prow[k], a[i][k]);
-            }
-        }
-    }
-
-    // Store each row at its final position and record where the data came from.
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        if (lr < mp)
-        {
-            const int dst = pos[i];
-#pragma unroll
-            for (int j = 0; j < W; ++j)
-                if (j < wact) Ap[static_cast<size_t>(j) * lda + dst] = a[i][j];
-            if (dst != lr)
-            {
-                const int slot = atomicAdd(&s_count, 1);
-                s_mdst[slot] = c0 + dst;
-                s_msrc[slot] = c0 + lr;
-            }
-        }
-    }
-    // Panel-level sources: read before any write (rows only exchange among themselves).
-    int srcv[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        srcv[i] = (lr < mp) ? (newPanel ? c0 + lr : rowsrc[c0 + lr]) : 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        if (lr < mp) rowsrc[c0 + pos[i]] = srcv[i];
-    }
-    if (tid == 0 && zeroCol != 0 && *info == 0) *info = zeroCol;
-
-    // The same interchanges on the other panel columns [j0, c0) and [c0 + wact, panelEnd):
-    // thread t takes moved entry t % MOVES of column t / MOVES of each batch of T / MOVES
-    // columns; every entry of a batch is gathered before any is scattered (rows only
-    // exchange among themselves).
-    const int cnt = s_count;
-    const int left = c0 - j0, others = left + (panelEnd - c0 - wact);
-    constexpr int CPB = T / MOVES;  // columns per batch
-    constexpr int SWB = 8;          // batches gathered per barrier
-    const int e = tid % MOVES;
-    for (int b0 = 0; b0 < others; b0 += CPB * SWB)  // uniform trip count
-    {
-        float v[SWB];
-        int cc[SWB];
-#pragma unroll
-        for (int bb = 0; bb < SWB; ++bb)
-        {
-            const int q = b0 + bb * CPB + tid / MOVES;
-            cc[bb] = -1;
-            v[bb] = 0.0f;
-            if (q < others && e < cnt)
-            {
-                cc[bb] = q < left ? j0 + q : c0 + wact + (q - left);
-                v[bb] = A[static_cast<size_t>(cc[bb]) * lda + s_msrc[e]];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int bb = 0; bb < SWB; ++bb)
-            if (cc[bb] >= 0) A[static_cast<size_t>(cc[bb]) * lda + s_mdst[e]] = v[bb];
-    }
-}
-
-// ---------------------------------------------------------------------------------------
-// Tall leaf over several workgroups: rows [c0, m) are split over P = gridDim.x one-wave
-// workgroups of 64*R consecutive rows, so each CU does 1/P of the per-column work and no
-// workgroup barrier sits on the per-column path. Per column every wave reduces its
-// candidates to one 64-bit key (DPP) and publishes the key, then its candidate's W values,
-// as tagged 64-bit words (relaxed agent-scope atomic stores; tag = this launch's base +
-// column, so each word is valid on its own and no fence or counter is needed); then it
-// polls the P keys, takes the maximum and reads the winning row. The update of columns
-// beyond j+1 by pivot j is deferred to the next column, where it runs between publishing
-// the key and publishing the row, i.e. while the peers' keys are in flight; per element the
-// updates still come in pivot order, so the result equals the unblocked elimination.
-// Slots alternate with the column parity: a workgroup publishes column j+2 only after all
-// have published j+1, i.e. after all have finished reading column j. Pivot choice, scaling
-// and update order are those of leaf_getf2_kernel (a NaN on the diagonal position is the
-// pivot, a NaN elsewhere ranks below every number). Spins are bounded:
-// on a timeout the workgroup raises *err, runs its remaining columns without waiting and
-// stores NaN rows; its peers then time out in turn.
-// SPREAD: the grid holds 8 workgroups per participant and only those with ids = 0 mod 8
-// take part. Workgroups are dispatched to the XCDs round-robin by id, so the participants
-// share one XCD (verified per device by LeafSpreadProbe when a handle is created; without
-// it the leaves run unspread). The exchange words are then stored at workgroup scope --
-// written through the CU's L1 into that XCD's L2 and kept there -- and read with the usual
-// agent-scope loads, which return a line held dirty in the XCD's L2 and fetch clean lines
-// anew: the words never make the trip to the device-coherent memory path (a round trip of
-// ~0.49 us instead of ~0.74 us, measured between two workgroups). Were a participant ever
-// placed on another XCD, it would not see the others' words nor they its: the bounded
-// waits would run out (devInfo -1000), and no stale word passes the tag check.
-// ---------------------------------------------------------------------------------------
-__device__ inline unsigned long long LoadSlot(const unsigned long long* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ inline void StoreWord(unsigned long long* p, unsigned long long v, bool local)
-{
-    if (local)  // uniform
-        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else
-        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ inline void StoreSlot(unsigned long long* p, unsigned tag, unsigned payload, bool local = false)
-{
-    StoreWord(p, (static_cast<unsigned long long>(tag) << 32) | payload, local);
-}
-
-// FULL: wact == W (no column of the unrolled loop is skipped at run time).
-template <int R, int W, bool FULL, bool SPREAD = false>
-__global__ __launch_bounds__(64) void leaf_multi_kernel(float* __restrict__ A, int lda, int m, int j0, int c0, int wact,
-                                                        int panelEnd, int pivoting, int newPanel,
-                                                        int* __restrict__ ipiv, int* __restrict__ info,
-                                                        int* __restrict__ rowsrc, unsigned long long* slots,
-                                                        unsigned tagBase, int* err, unsigned spinLimit)
-{
-    constexpr int T = 64;
-    static_assert(W <= kRowWords && W <= T, "slot layout");
-    constexpr int MOVES = 2 * W;
-    __shared__ float s_row[W];
-    __shared__ float s_prow[2][W];  // pivot rows of columns j (slot j % 2) and j - 1
-    __shared__ int s_bpos[W];
-    __shared__ int s_count;
-    __shared__ int s_mdst[MOVES], s_msrc[MOVES];
-
-    const int lane = threadIdx.x;
-    if (SPREAD && (blockIdx.x & 7) != 0) return;  // not a participant
-    const int P = SPREAD ? static_cast<int>(gridDim.x >> 3) : static_cast<int>(gridDim.x);
-    const int g = SPREAD ? static_cast<int>(blockIdx.x >> 3) : static_cast<int>(blockIdx.x);
-    const int mp = m - c0;
-    float* Ap = A + static_cast<size_t>(c0) * lda + c0;
-    const int rbase = g * T * R;
-    // An earlier leaf of this factorization timed out: its factors are NaN already.
-    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-    bool aborted = false;  // uniform (one wave)
-    // SPREAD: the participants share one XCD (established on the host when the handle was
-    // created), so the exchange words are stored at workgroup scope into its L2.
-    constexpr bool local = SPREAD;
-
-    float a[R][W];
-    int pos[R], srcv[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = rbase + lane + i * T;
-        const bool valid = lr < mp;
-#pragma unroll
-        for (int j = 0; j < W; ++j) a[i][j] = (valid && j < wact) ? Ap[static_cast<size_t>(j) * lda + lr] : 0.0f;
-        pos[i] = valid ? lr : -1;
-        // Panel-level sources, read before any workgroup can store (stores follow the
-        // last column's exchange, which every workgroup enters after these loads).
-        srcv[i] = valid ? (newPanel ? c0 + lr : rowsrc[c0 + lr]) : 0;
-    }
-    if (lane == 0) s_count = 0;
-    int zeroCol = 0;
-    float lprev[R];  // multipliers of the previous pivot (0 for rows not below it)
-#pragma unroll
-    for (int i = 0; i < R; ++i) lprev[i] = 0.0f;
-
-#pragma unroll
-    for (int j = 0; j < W; ++j)
-    {
-        if (FULL || j < wact)  // uniform
-        {
-            const unsigned tag = tagBase + static_cast<unsigned>(j);
-            unsigned long long* keys = slots + (j & 1) * kMaxLeafGroups;
-            unsigned long long* rows = slots + kKeyWords + static_cast<size_t>(j & 1) * kMaxLeafGroups * kRowWords;
-            // Column j is up to date; columns beyond it still lack the previous pivot.
-            // Key: magnitude class in the high word (0: not a candidate, 1: NaN off the
-            // diagonal position, |a| bits + 2, 0x80000000: NaN on it), rank 0xffff - position
-            // (positions are below 16384) in the low word.
-            unsigned long long best = 0ull;
-            int bi = -1;
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                const bool cand = pivoting ? pos[i] >= j : pos[i] == j;
-                const unsigned ab = __float_as_uint(fabsf(a[i][j]));
-                const unsigned mag = ab <= 0x7f800000u ? ab + 2u : (pos[i] == j ? 0x80000000u : 1u);
-                const unsigned long long k =
-                    cand ? (static_cast<unsigned long long>(mag) << 32) | static_cast<unsigned>(0xffff - pos[i]) : 0ull;
-                bi = k > best ? i : bi;
-                best = k > best ? k : best;
-            }
-            const unsigned long long top = WaveMaxU64Split(best);
-            if (lane == 0)
-                StoreWord(keys + g,
-                          (static_cast<unsigned long long>(tag & 0xffffu) << 48) | ((top >> 32) << 16) |
-                              (top & 0xffffull),
-                          local);
-            // Deferred: the previous pivot on columns j+1 .. W-1.
-            if (j > 0)
-#pragma unroll
-                for (int k = j + 1; k < W; ++k)
-                {
-                    const float pk = s_prow[(j - 1) & 1][k];
-#pragma unroll
-                    for (int i = 0; i < R; ++i) a[i][k] = fmaf(-lprev[i], pk, a[i][k]);
-                }
-            // The candidate's row, now complete, through LDS to lanes 0 .. wact-1.
-            if (best == top && bi >= 0)
-#pragma unroll
-                for (int i = 0; i < R; ++i)
-                    if (i == bi)
-#pragma unroll
-                        for (int k = 0; k < W; ++k) s_row[k] = a[i][k];
-            __syncthreads();
-            if (lane < wact)
-                StoreSlot(rows + g * kRowWords + lane, tag, __float_as_uint(s_row[lane < W ? lane : 0]), local);
-            // The P keys: lane l reads the key words of workgroups l and l + 64.
-            unsigned long long key0 = 0ull, key1 = 0ull;
-            bool ok = false;
-            // After a timeout the remaining columns run without waiting (no exchange, no
-            // interchange): the column loop stays one straight unrolled sequence, and the
-            // factors end as NaN.
-            const unsigned lim = aborted ? 0u : spinLimit;
-            const unsigned long long t16 = tag & 0xffffu;
-            for (unsigned spins = 0; spins < lim; ++spins)
-            {
-                const unsigned long long w0 = lane < P ? LoadSlot(keys + lane) : t16 << 48;
-                const unsigned long long w1 = lane + 64 < P ? LoadSlot(keys + lane + 64) : t16 << 48;
-                // (magnitude << 32) | rank, 0 for peers without a candidate
-                key0 = (((w0 >> 16) & 0xffffffffull) << 32) | (w0 & 0xffffull);
-                key1 = (((w1 >> 16) & 0xffffffffull) << 32) | (w1 & 0xffffull);
-                if (__all((w0 >> 48) == t16 && (w1 >> 48) == t16))
-                {
-                    ok = true;
-                    break;
-                }
-            }
-            const unsigned long long gtop = WaveMaxU64Split(key0 > key1 ? key0 : key1);
-            const unsigned long long hit0 = __ballot(ok && lane < P && key0 == gtop);
-            const unsigned long long hit1 = __ballot(ok && lane + 64 < P && key1 == gtop);
-            const int winner = hit0 != 0ull   ? __ffsll(static_cast<long long>(hit0)) - 1
-                               : hit1 != 0ull ? 64 + __ffsll(static_cast<long long>(hit1)) - 1
-                                              : 0;
-            // The winner's row: lane k holds its value in column k.
-            unsigned long long rw = 0ull;
-            for (unsigned spins = 0; ok; ++spins)
-            {
-                rw = lane < wact ? LoadSlot(rows + winner * kRowWords + lane)
-                                 : static_cast<unsigned long long>(tag) << 32;
-                if (__all(static_cast<unsigned>(rw >> 32) == tag)) break;
-                if (spins >= spinLimit) ok = false;
-            }
-            if (!ok)
-            {
-                if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                aborted = true;
-            }
-            if (lane < W) s_prow[j & 1][lane] = __uint_as_float(static_cast<unsigned>(rw));
-            __syncthreads();
-            const int bpos = aborted || gtop == 0ull ? j : 0xffff - static_cast<int>(gtop & 0xffffull);
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                if (pos[i] == bpos)
-                    pos[i] = j;
-                else if (pos[i] == j)
-                    pos[i] = bpos;
-            }
-            if (lane == 0)
-            {
-                s_bpos[j] = bpos;
-                if (g == 0 && ipiv != nullptr) ipiv[c0 + j] = c0 + bpos + 1;
-            }
-            // The pivot, read from lane j of the winner's row into a scalar register: the
-            // reciprocal / division choice is then a scalar branch.
-            const float d = __uint_as_float(__builtin_amdgcn_readlane(static_cast<unsigned>(rw), j));
-            if (d == 0.0f && zeroCol == 0 && !aborted) zeroCol = c0 + j + 1;
-            const bool recip = fabsf(d) >= FLT_MIN;  // uniform
-            const float r = 1.0f / d;
-            float q[R];
-            if (recip)
-#pragma unroll
-                for (int i = 0; i < R; ++i) q[i] = a[i][j] * r;
-            else
-#pragma unroll
-                for (int i = 0; i < R; ++i) q[i] = a[i][j] / d;
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                const bool below = pos[i] > j && d != 0.0f;
-                lprev[i] = below ? q[i] : 0.0f;
-                a[i][j] = below ? q[i] : a[i][j];
-            }
-            // Column j+1 now (the next candidate search needs it); the rest next column.
-            if (j + 1 < W)
-            {
-                const float pk = s_prow[j & 1][j + 1];
-#pragma unroll
-                for (int i = 0; i < R; ++i) a[i][j + 1] = fmaf(-lprev[i], pk, a[i][j + 1]);
-            }
-        }
-    }
-    if (aborted)
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-#pragma unroll
-            for (int j = 0; j < W; ++j) a[i][j] = __builtin_nanf("");
-
-    // Each row to its final position (leaf columns), and its panel-level source.
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = rbase + lane + i * T;
-        if (lr < mp)
-        {
-            const int dst = pos[i];
-#pragma unroll
-            for (int j = 0; j < W; ++j)
-                if (j < wact) Ap[static_cast<size_t>(j) * lda + dst] = a[i][j];
-            rowsrc[c0 + dst] = srcv[i];
-        }
-    }
-    if (g == 0 && lane == 0 && zeroCol != 0 && *info == 0) *info = zeroCol;
-    if (aborted) return;  // uniform
-    __syncthreads();
-
-    // The moved rows, from the interchange sequence (identical in every workgroup): the row
-    // that ends at position p came from the position found by undoing the interchanges in
-    // reverse. Candidates: positions 0..wact-1 (items 0..W-1) and the pivot positions
-    // beyond them (items W..2W-1, first occurrence only).
-    for (int it = lane; it < 2 * W; it += T)
-    {
-        int p = -1;
-        if (it < W)
-            p = it < wact ? it : -1;
-        else if (it - W < wact)
-        {
-            const int jj = it - W;
-            p = s_bpos[jj] >= wact ? s_bpos[jj] : -1;
-            for (int t = 0; t < jj && p >= 0; ++t)
-                if (s_bpos[t] == p) p = -1;
-        }
-        if (p >= 0)
-        {
-            int x = p;
-            for (int jj = wact - 1; jj >= 0; --jj)
-            {
-                const int b = s_bpos[jj];
-                x = x == jj ? b : (x == b ? jj : x);
-            }
-            if (x != p)
-            {
-                const int slot = atomicAdd(&s_count, 1);
-                s_mdst[slot] = c0 + p;
-                s_msrc[slot] = c0 + x;
-            }
-        }
-    }
-    __syncthreads();
-
-    // The same interchanges on the other panel columns [j0, c0) and [c0 + wact, panelEnd),
-    // columns dealt round-robin to the workgroups; each column is gathered completely
-    // before it is scattered.
-    const int cnt = s_count;
-    const int left = c0 - j0, others = left + (panelEnd - c0 - wact);
-    constexpr int SWB = 4, EPL = (MOVES + T - 1) / T;  // moved entries per lane
-    for (int q0 = g; q0 < others; q0 += SWB * P)  // uniform trip count
-    {
-        float v[SWB][EPL];
-        int cc[SWB];
-#pragma unroll
-        for (int bb = 0; bb < SWB; ++bb)
-        {
-            const int q = q0 + bb * P;
-            cc[bb] = q < others ? (q < left ? j0 + q : c0 + wact + (q - left)) : -1;
-#pragma unroll
-            for (int u = 0; u < EPL; ++u)
-            {
-                const int e = lane + u * T;
-                v[bb][u] = (cc[bb] >= 0 && e < cnt) ? A[static_cast<size_t>(cc[bb]) * lda + s_msrc[e]] : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int bb = 0; bb < SWB; ++bb)
-#pragma unroll
-            for (int u = 0; u < EPL; ++u)
-            {
-                const int e = lane + u * T;
-                if (cc[bb] >= 0 && e < cnt) A[static_cast<size_t>(cc[bb]) * lda + s_mdst[e]] = v[bb][u];
-            }
-    }
 }
 
 __global__ void clear_slots_kernel(unsigned long long* slots, int words, int* err)
@@ -746,31 +205,19 @@ __global__ void iota_kernel(int* p, int n)
     if (i < n) p[i] = i;
 }
 
-template <int T, int R, int W>
-hipError_t LaunchLeaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd, int pivoting, int newPanel,
-                      int* ipiv, int* info, const Work& w, hipStream_t stream)
-{
-    if (wact == W)
-        hipLaunchKernelGGL((leaf_getf2_kernel<T, R, W, true>), dim3(1), dim3(T), 0, stream, A, lda, m, j0, c0, wact,
-                           panelEnd, pivoting, newPanel, ipiv, info, w.rowsrc);
-    else
-        hipLaunchKernelGGL((leaf_getf2_kernel<T, R, W, false>), dim3(1), dim3(T), 0, stream, A, lda, m, j0, c0, wact,
-                           panelEnd, pivoting, newPanel, ipiv, info, w.rowsrc);
-    return hipGetLastError();
-}
-
-// Panels with more active rows than this run their leaves over several workgroups
-// (leaf_multi_kernel); OPS_SOLVER_MULTI_LEAF_ROWS overrides it (0: never).
+// Panels with more active rows than this run their leaves over several workgroups;
+// OPS_SOLVER_MULTI_LEAF_ROWS lowers it (a one-workgroup leaf takes at most kLeafSingleRows).
 int MultiLeafRows()
 {
     static const int rows = []
     {
         const char* e = std::getenv("OPS_SOLVER_MULTI_LEAF_ROWS");
-        return e != nullptr ? std::atoi(e) : 2048;
+        const int v = e != nullptr ? std::atoi(e) : 0;
+        return v > 0 ? std::min(v, kLeafSingleRows) : kLeafSingleRows;
     }();
     return rows;
 }
-inline bool UseMultiLeaf(int mp) { return MultiLeafRows() > 0 && mp > MultiLeafRows(); }
+inline bool UseMultiLeaf(int mp) { return mp > MultiLeafRows(); }
 
 // Multi-workgroup leaves by cooperative launch (OPS_SOLVER_LEAF_COOP, default 1).
 bool LeafCooperative()
@@ -783,13 +230,11 @@ bool LeafCooperative()
     return on;
 }
 
-constexpr int kMultiT = 64, kMultiR = 2, kMultiW = 64;  // one wave of 128 rows per workgroup, 64 columns
-
 // Per device: 1 when LeafSpreadProbe found the workgroups with ids = 0 mod 8 of a
 // 1024-workgroup cooperative launch on one XCD, -1 when not, 0 before the probe.
 constexpr int kMaxDevices = 64;
 std::atomic<int> g_spreadOk[kMaxDevices];
-__device__ int g_xccOfGroup[8 * kMaxLeafGroups];
+__device__ int g_xccOfGroup[kProbeGroups];
 
 __global__ void xcc_probe_kernel()
 {
@@ -812,45 +257,6 @@ bool LeafSpread()
 namespace
 {
 
-hipError_t MultiLeaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd, int pivoting, int newPanel,
-                     int* ipiv, int* info, const Work& w, hipStream_t stream)
-{
-    const int mp = m - c0;
-    const int groups = (mp + kMultiT * kMultiR - 1) / (kMultiT * kMultiR);
-    if (groups > kMaxLeafGroups || wact > kMultiW || w.epoch == nullptr) return hipErrorInvalidValue;
-    unsigned tagBase = (*w.epoch)++ * 64u;
-    // Key words carry 16-bit tags: within one factorization (slots cleared at its start)
-    // the tags must not wrap. At most n / 64 <= 256 leaves (plus tournament epochs) use them.
-    if (tagBase + 64u > 0xffffu) return hipErrorInvalidValue;
-    unsigned spinLimit = SpinLimit();
-    // Cooperative launch: the workgroups wait for each other every column, so the runtime
-    // must make all of them resident at once (it refuses a grid that cannot be).
-    int* rowsrc = w.rowsrc;
-    unsigned long long* slots = w.slots;
-    int* err = w.err;
-    void* args[] = {&A, &lda, &m, &j0, &c0, &wact, &panelEnd, &pivoting, &newPanel, &ipiv, &info, &rowsrc, &slots,
-                    &tagBase, &err, &spinLimit};
-    const bool full = wact == kMultiW;
-    if (!LeafCooperative())
-    {
-        if (full)
-            hipLaunchKernelGGL((leaf_multi_kernel<kMultiR, kMultiW, true>), dim3(groups), dim3(kMultiT), 0, stream, A,
-                               lda, m, j0, c0, wact, panelEnd, pivoting, newPanel, ipiv, info, rowsrc, slots, tagBase,
-                               err, spinLimit);
-        else
-            hipLaunchKernelGGL((leaf_multi_kernel<kMultiR, kMultiW, false>), dim3(groups), dim3(kMultiT), 0, stream, A,
-                               lda, m, j0, c0, wact, panelEnd, pivoting, newPanel, ipiv, info, rowsrc, slots, tagBase,
-                               err, spinLimit);
-        return hipGetLastError();
-    }
-    if (full && LeafSpread())
-        return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&leaf_multi_kernel<kMultiR, kMultiW, true, true>),
-                                          dim3(8 * groups), dim3(kMultiT), args, 0, stream);
-    const void* fn = full ? reinterpret_cast<const void*>(&leaf_multi_kernel<kMultiR, kMultiW, true>)
-                          : reinterpret_cast<const void*>(&leaf_multi_kernel<kMultiR, kMultiW, false>);
-    return hipLaunchCooperativeKernel(fn, dim3(groups), dim3(kMultiT), args, 0, stream);
-}
-
 // Panels with more active rows than this take tournament leaves when the caller allows
 // them; OPS_SOLVER_TSLU_ROWS overrides it.
 int TsluRows()
@@ -864,17 +270,7 @@ int TsluRows()
 }
 inline bool UseTslu(const Work& w, int mp) { return w.tournament && mp > TsluRows() && mp <= kTsluMaxRows; }
 
-// Leaf width for a panel of mp active rows: every shape keeps R*W <= 128 values per lane
-// (512-thread workgroups leave up to 256 VGPRs per lane).
-int LeafWidth(int mp, const Work& w)
-{
-    if (UseTslu(w, mp)) return kTsluWidth;
-    if (UseMultiLeaf(mp)) return kMultiW;
-    if (mp <= 512) return 64;
-    if (mp <= 2048) return 32;
-    if (mp <= 8192) return 8;
-    return 4;
-}
+int LeafWidth(int mp, const Work& w) { return UseTslu(w, mp) ? kTsluWidth : kLeafMaxWidth; }
 
 hipError_t Leaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd, int pivoting, int newPanel,
                 int* ipiv, int* info, const Work& w, hipStream_t stream)
@@ -885,17 +281,19 @@ hipError_t Leaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd
     if (pivoting && UseTslu(w, mp))
         return TsluLeaf(A, lda, m, j0, c0, wact, panelEnd, newPanel, ipiv, info, w.rowsrc, w.tslu, (*w.epoch)++,
                         w.err, stream);
-    if (UseMultiLeaf(mp)) return MultiLeaf(A, lda, m, j0, c0, wact, panelEnd, pivoting, newPanel, ipiv, info, w, stream);
-#define LEAF(T, R, W) \
-    LaunchLeaf<T, R, W>(A, lda, m, j0, c0, wact, panelEnd, pivoting, newPanel, ipiv, info, w, stream)
-    if (mp <= 256) return LEAF(256, 1, 64);
-    if (mp <= 512) return LEAF(512, 1, 64);
-    if (mp <= 1024) return LEAF(512, 2, 32);
-    if (mp <= 2048) return LEAF(512, 4, 32);
-    if (mp <= 4096) return LEAF(512, 8, 8);
-    if (mp <= 8192) return LEAF(512, 16, 8);
-    return LEAF(1024, 16, 4);
-#undef LEAF
+    LeafArgs a{A,    lda,      m,         j0,     c0,     wact, panelEnd, pivoting, newPanel, ipiv,
+               info, w.rowsrc, w.leafMoves, w.slots, 0u, w.err, SpinLimit()};
+    if (UseMultiLeaf(mp))
+    {
+        // Key words carry 16-bit tags: within one factorization (slots cleared at its start)
+        // the tags must not wrap. At most n / 64 <= 256 leaves (plus tournament epochs) use them.
+        a.tagBase = (*w.epoch)++ * kLeafMaxWidth;
+        if (a.tagBase + kLeafMaxWidth > 0xffffu) return hipErrorInvalidValue;
+        if (const hipError_t e = LeafMulti(a, LeafCooperative(), LeafSpread(), stream)) return e;
+    }
+    else if (const hipError_t e = LeafSingle(a, stream))
+        return e;
+    return pivoting ? LeafSwap(a, stream) : hipSuccess;
 }
 
 #define RET_IF(e)                          \
@@ -970,7 +368,7 @@ hipError_t RealGetrfPerm(int m, int n, float* a, int lda, int* ipiv, int* info, 
     {
         // The multi-workgroup leaves' exchange slots (when they run) and the timeout flag
         // shared by every bounded wait of the factorization.
-        const int words = UseMultiLeaf(m) ? static_cast<int>(kSlotBytes / sizeof(unsigned long long)) : 0;
+        const int words = UseMultiLeaf(m) ? kLeafSlotWords : 0;
         hipLaunchKernelGGL(clear_slots_kernel, dim3(std::max(1, (words + 255) / 256)), dim3(256), 0, stream, w.slots,
                            words, w.err);
     }
@@ -1303,7 +701,7 @@ hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const
 void LeafSpreadProbe(int device)
 {
     if (device < 0 || device >= kMaxDevices || g_spreadOk[device].load() != 0) return;
-    constexpr int G = 8 * kMaxLeafGroups;
+    constexpr int G = kProbeGroups;
     int result = -1;
     if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&xcc_probe_kernel), dim3(G), dim3(64), nullptr, 0,
                                    nullptr) == hipSuccess &&
@@ -1313,7 +711,7 @@ void LeafSpreadProbe(int device)
         if (hipMemcpyFromSymbol(h, HIP_SYMBOL(g_xccOfGroup), sizeof(h)) == hipSuccess)
         {
             result = 1;
-            for (int k = 1; k < kMaxLeafGroups; ++k)
+            for (int k = 1; k < G / 8; ++k)
                 if (h[8 * k] != h[0]) result = -1;
         }
     }

@@ -95,7 +95,7 @@ void* NoAllocScratch(int device);
 // Once per device at handle creation: may the tall panel leaves exchange through one XCD's
 // L2 (getrf.hip)?
 void LeafSpreadProbe(int device);
-// May the full-width tall leaves of the current device run spread over 8x their grid and
+// May the tall leaves of the current device run spread over 8x their grid and
 // exchange through one XCD's L2 (probe result, OPS_SOLVER_LEAF_XCD)?
 bool LeafSpread();
 
