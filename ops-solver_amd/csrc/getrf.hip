@@ -56,7 +56,8 @@ struct Work
     int* leafMoves;
     int* err;
     unsigned* epoch;       // host counter: tag base of the next multi-workgroup leaf
-    float* linvNode;       // block inverses for the panel-internal solves (panel stream only)
+    float* linvNode;       // tournament panels: block inverses for their internal solves
+    float* panelRows;      // the same space: 64 rows of the panel columns right of a leaf (panel stream only)
     float* linvPanel[2];   // block inverses of panel k's L11 in slot k % 2 (both streams read them)
     void* tslu;            // scratch of the tournament leaves
     bool tournament;       // tall leaves pivot by tournament (TsluLeaf)
@@ -81,7 +82,8 @@ inline Work Layout(void* base, int m)
     w.err = reinterpret_cast<int*>(q + kSlotBytes);
     w.epoch = nullptr;
     q = (q + kSlotBytes + 16 + 255) & ~static_cast<uintptr_t>(255);
-    w.linvNode = reinterpret_cast<float*>(q);
+    w.linvNode = w.panelRows = reinterpret_cast<float*>(q);
+    static_assert(NBMAX * kLeafMaxWidth * sizeof(float) <= kLinvPanelBytes, "panel rows");
     w.linvPanel[0] = reinterpret_cast<float*>(q + kLinvPanelBytes);
     w.linvPanel[1] = reinterpret_cast<float*>(q + 2 * kLinvPanelBytes);
     w.tslu = reinterpret_cast<void*>(q + 3 * kLinvPanelBytes);
@@ -272,28 +274,28 @@ inline bool UseTslu(const Work& w, int mp) { return w.tournament && mp > TsluRow
 
 int LeafWidth(int mp, const Work& w) { return UseTslu(w, mp) ? kTsluWidth : kLeafMaxWidth; }
 
-hipError_t Leaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd, int pivoting, int newPanel,
-                int* ipiv, int* info, const Work& w, hipStream_t stream)
+// The leaf itself; its interchanges (LeafSwap, LeafFinish) are the caller's.
+hipError_t LeafColumns(LeafArgs& a, const Work& w, hipStream_t stream)
 {
-    const int mp = m - c0;
+    const int mp = a.m - a.c0;
     // Algorithmic traffic of a leaf: its panel columns read and written once.
-    ProfileScope prof(ProfileKernel::PanelLeaf, 8.0 * mp * wact, stream);
-    if (pivoting && UseTslu(w, mp))
-        return TsluLeaf(A, lda, m, j0, c0, wact, panelEnd, newPanel, ipiv, info, w.rowsrc, w.tslu, (*w.epoch)++,
-                        w.err, stream);
-    LeafArgs a{A,    lda,      m,         j0,     c0,     wact, panelEnd, pivoting, newPanel, ipiv,
-               info, w.rowsrc, w.leafMoves, w.slots, 0u, w.err, SpinLimit()};
+    ProfileScope prof(ProfileKernel::PanelLeaf, 8.0 * mp * a.wact, stream);
     if (UseMultiLeaf(mp))
     {
         // Key words carry 16-bit tags: within one factorization (slots cleared at its start)
         // the tags must not wrap. At most n / 64 <= 256 leaves (plus tournament epochs) use them.
         a.tagBase = (*w.epoch)++ * kLeafMaxWidth;
         if (a.tagBase + kLeafMaxWidth > 0xffffu) return hipErrorInvalidValue;
-        if (const hipError_t e = LeafMulti(a, LeafCooperative(), LeafSpread(), stream)) return e;
+        return LeafMulti(a, LeafCooperative(), LeafSpread(), stream);
     }
-    else if (const hipError_t e = LeafSingle(a, stream))
-        return e;
-    return pivoting ? LeafSwap(a, stream) : hipSuccess;
+    return LeafSingle(a, stream);
+}
+
+LeafArgs MakeLeaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd, int pivoting, int* ipiv, int* info,
+                  const Work& w)
+{
+    return LeafArgs{A,    lda,      m,           j0,      c0, wact,  panelEnd,   pivoting, c0 == j0, ipiv,
+                    info, w.rowsrc, w.leafMoves, w.slots, 0u, w.err, SpinLimit()};
 }
 
 #define RET_IF(e)                          \
@@ -303,16 +305,48 @@ hipError_t Leaf(float* A, int lda, int m, int j0, int c0, int wact, int panelEnd
         if (_e != hipSuccess) return _e;   \
     } while (0)
 
-// Factors columns [c0, c0 + w) of the outer panel [j0, panelEnd) over rows [c0, m); every
-// panel column already holds the updates of the columns left of c0. The left half is
-// factored first (recursively), its L11 solves the right half's top rows and an MFMA
-// product updates the rest of the right half, then the right half is factored. Each leaf
-// applies its row interchanges to all other panel columns itself.
+// The panel [j0, panelEnd) of rows [j0, m): per 64 columns one leaf, one launch that applies its
+// interchanges to the whole panel and inverts its diagonal block, and one that updates all
+// panel columns to its right. The block inverses (linv, 4096 floats per 64 columns) serve the
+// U12 solves of the trailing columns afterwards.
+// Right-looking by 64 columns rather than recursive: the same number of updates, each one
+// launch instead of two to four, for somewhat more traffic on the panel.
+hipError_t Panel(float* a, int lda, int m, int j0, int panelEnd, int pivoting, int* ipiv, int* info, const Work& wk,
+                 float* linv, hipStream_t stream)
+{
+    for (int c0 = j0; c0 < panelEnd; c0 += kLeafMaxWidth)
+    {
+        const int wact = std::min(kLeafMaxWidth, panelEnd - c0);
+        LeafArgs l = MakeLeaf(a, lda, m, j0, c0, wact, panelEnd, pivoting, ipiv, info, wk);
+        float* const inv = linv + static_cast<size_t>(c0 - j0) * kLeafMaxWidth;
+        RET_IF(LeafColumns(l, wk, stream));
+        RET_IF(LeafFinish(l, inv, wk.panelRows, stream));
+        if (c0 + wact < panelEnd) RET_IF(PanelUpdate(l, inv, wk.panelRows, stream));
+    }
+    return hipSuccess;
+}
+
+// Tournament pivoting: factors columns [c0, c0 + w) of the outer panel [j0, panelEnd) over
+// rows [c0, m); every panel column already holds the updates of the columns left of c0. The
+// left half is factored first (recursively), its L11 solves the right half's top rows and an
+// MFMA product updates the rest of the right half, then the right half is factored. The
+// interchanges of each leaf are applied to all other panel columns.
 hipError_t PanelRec(float* a, int lda, int m, int j0, int panelEnd, int c0, int w, int pivoting, int* ipiv, int* info,
                     const Work& wk, hipStream_t stream)
 {
     const int W = LeafWidth(m - c0, wk);
-    if (w <= W) return Leaf(a, lda, m, j0, c0, w, panelEnd, pivoting, c0 == j0, ipiv, info, wk, stream);
+    if (w <= W)
+    {
+        if (UseTslu(wk, m - c0))
+        {
+            ProfileScope prof(ProfileKernel::PanelLeaf, 8.0 * (m - c0) * w, stream);
+            return TsluLeaf(a, lda, m, j0, c0, w, panelEnd, c0 == j0, ipiv, info, wk.rowsrc, wk.tslu, (*wk.epoch)++,
+                            wk.err, stream);
+        }
+        LeafArgs l = MakeLeaf(a, lda, m, j0, c0, w, panelEnd, pivoting, ipiv, info, wk);
+        RET_IF(LeafColumns(l, wk, stream));
+        return LeafSwap(l, stream);
+    }
     const int h = (w / 2 + W - 1) / W * W;  // whole leaves on the left
     RET_IF(PanelRec(a, lda, m, j0, panelEnd, c0, h, pivoting, ipiv, info, wk, stream));
     const int r = w - h;
@@ -404,13 +438,18 @@ hipError_t RealGetrfPerm(int m, int n, float* a, int lda, int* ipiv, int* info, 
     auto panel = [&](int k) -> hipError_t
     {
         const int j0 = k * NB, nb = std::min(NB, kmax - j0);
-        RET_IF(PanelRec(a, lda, m, j0, j0 + nb, j0, nb, pivoting, ipiv, info, w, s0));
+        float* const linv = w.linvPanel[k & 1];
+        if (w.tournament)
+            RET_IF(PanelRec(a, lda, m, j0, j0 + nb, j0, nb, pivoting, ipiv, info, w, s0));
+        else
+            RET_IF(Panel(a, lda, m, j0, j0 + nb, pivoting, ipiv, info, w, linv, s0));
         if (pivoting)
             hipLaunchKernelGGL(compact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, moved(k),
                                permOut);
         RET_IF(hipGetLastError());
         // The U12 solves of both streams use the block inverses of this panel's L11.
-        return TrsmLowerUnitInverse(nb, a + static_cast<size_t>(j0) * lda + j0, lda, w.linvPanel[k & 1], s0);
+        if (!w.tournament) return hipSuccess;
+        return TrsmLowerUnitInverse(nb, a + static_cast<size_t>(j0) * lda + j0, lda, linv, s0);
     };
     // Applies panel k to the columns [lo, hi) (interchanges, U12 solve, trailing product)
     // and, when leftSwaps, its interchanges to the columns left of the panel.

@@ -30,6 +30,7 @@
 // 1024 rows 104 -> 66 us, 2048 rows 158 -> 89 us, 8192 rows 125 -> 92 us.
 #include "leaf.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 
@@ -682,6 +683,219 @@ __global__ __launch_bounds__(256) void leaf_swap_kernel(float* __restrict__ A, i
     if (m1.x >= 0) col[m1.x] = x1;
 }
 
+// What follows a leaf of 64 columns, in one launch: its interchanges on every panel column
+// and the inverse of its unit-lower 64 x 64 diagonal block. Workgroup 0 takes the leaf's own
+// columns (it needs them in place for the inverse), the others a wave per column left and
+// right of it. The top 64 rows of the right columns go to ub (ld 64) instead of A: the launch
+// that turns them into U writes A while its other workgroups still read them.
+// The inverse is bound by latency: 16 x 16 diagonal blocks by substitution, one lane per
+// column, then two doublings by products on the matrix cores (a substitution over the whole
+// block took 64 dependent steps and 18 us of mostly instruction fetches).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kInvStride = 68;
+
+// D (16 x 16 at d) = sign * A (16 x K at a) * B (K x 16 at b), row-major in LDS, one wave.
+template <int K>
+__device__ inline void Product16(const float* a, const float* b, float* d, float sign, int lane)
+{
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int i = lane & 15, k0 = lane >> 4;
+#pragma unroll
+    for (int k = 0; k < K; k += 4)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i * kInvStride + k + k0], b[(k + k0) * kInvStride + i], acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d[(4 * k0 + r) * kInvStride + i] = sign * acc[r];
+}
+
+__global__ __launch_bounds__(256) void leaf_finish_kernel(float* __restrict__ A, int64_t lda, int j0, int c0, int wact,
+                                                          int hi, const int2* __restrict__ moves,
+                                                          const int* __restrict__ err, float* __restrict__ linv,
+                                                          float* __restrict__ ub)
+{
+    constexpr int W = kLeafMaxWidth;
+    __shared__ __align__(16) float s_l[W * kInvStride], s_i[W * kInvStride], s_t[32 * kInvStride];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (*err != 0) return;  // after a timeout the list is not complete
+    const int2 none = make_int2(-1, -1);
+    const int2 m0 = lane < wact ? moves[lane] : none, m1 = lane < wact ? moves[W + lane] : none;
+    const int from = m0.x >= 0 ? m0.y : c0 + lane;  // the row that ends at position lane
+    if (blockIdx.x > 0)
+    {
+        const int left = c0 - j0, q = static_cast<int>(blockIdx.x - 1) * 4 + wave;
+        const int c = q < left ? j0 + q : c0 + wact + (q - left);
+        if (c >= hi) return;
+        float* const col = A + c * lda;
+        float x0 = 0.0f, x1 = 0.0f;
+        if (lane < wact) x0 = col[from];
+        if (m1.x >= 0) x1 = col[m1.y];
+        if (q >= left)
+            ub[static_cast<size_t>(q - left) * W + lane] = x0;
+        else if (m0.x >= 0)
+            col[m0.x] = x0;
+        if (m1.x >= 0) col[m1.x] = x1;
+        return;
+    }
+    // The leaf's own columns, sixteen per wave, all loads in flight.
+    float x0[16], x1[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+    {
+        const int c = wave * 16 + k;
+        x0[k] = x1[k] = 0.0f;
+        if (c < wact && lane < wact)
+        {
+            const float* const col = A + (c0 + c) * lda;
+            x0[k] = col[from];
+            if (m1.x >= 0) x1[k] = col[m1.y];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+    {
+        const int c = wave * 16 + k;
+        if (c < wact)
+        {
+            float* const col = A + (c0 + c) * lda;
+            if (m0.x >= 0) col[m0.x] = x0[k];
+            if (m1.x >= 0) col[m1.x] = x1[k];
+        }
+        // Unit lower; rows and columns beyond the block are the identity.
+        s_l[lane * kInvStride + c] = lane > c && lane < wact ? x0[k] : 0.0f;
+        s_i[lane * kInvStride + c] = 0.0f;
+    }
+    __syncthreads();
+    if (wave == 0)
+    {
+        // Lane: column lane % 16 of diagonal block lane / 16.
+        const int b = lane & 48;
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+        {
+            float v = i == (lane & 15) ? 1.0f : 0.0f;
+            const float* const row = s_l + (b + i) * kInvStride + b;
+#pragma unroll
+            for (int k = 0; k < i; ++k) v = fmaf(-row[k], x[k], v);
+            x[i] = v;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_i[(b + i) * kInvStride + lane] = x[i];
+    }
+    __syncthreads();
+    // inv [P 0; Q R] = [P' 0; -R' Q P' R'] with 16 x 16, then 32 x 32 blocks.
+    if (wave < 2)
+        Product16<16>(s_l + (32 * wave + 16) * kInvStride + 32 * wave, s_i + 32 * wave * kInvStride + 32 * wave,
+                      s_t + 16 * wave * kInvStride, 1.0f, lane);
+    __syncthreads();
+    if (wave < 2)
+        Product16<16>(s_i + (32 * wave + 16) * kInvStride + 32 * wave + 16, s_t + 16 * wave * kInvStride,
+                      s_i + (32 * wave + 16) * kInvStride + 32 * wave, -1.0f, lane);
+    __syncthreads();
+    const int qr = 16 * (wave >> 1), qc = 16 * (wave & 1);
+    Product16<32>(s_l + (32 + qr) * kInvStride, s_i + qc, s_t + qr * kInvStride + qc, 1.0f, lane);
+    __syncthreads();
+    Product16<32>(s_i + (32 + qr) * kInvStride + 32, s_t + qc, s_i + (32 + qr) * kInvStride + qc, -1.0f, lane);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+    {
+        const int c = wave * 16 + k;
+        linv[c * W + lane] = s_i[lane * kInvStride + c];
+    }
+}
+
+// The panel columns right of a finished leaf: U = inv(L11) B (B: the 64 rows of ub) and
+// C -= L21 U, one workgroup per 32 RT x 64 tile of C, four waves. Every workgroup forms the U
+// of its 64 columns itself (40 products of 16 x 16 x 4 a wave, 0.5 us) rather than wait for a
+// launch that does; those of the first tile row store it. Bound by latency for short panels
+// and by the read and write of C for tall ones. The operands of the update are loaded before
+// U is formed, so the launch waits for memory once.
+template <int RT>
+__global__ __launch_bounds__(256) void panel_update_kernel(float* __restrict__ A, int64_t lda, int m, int c0, int hi,
+                                                           const float* __restrict__ linv, const float* __restrict__ ub)
+{
+    constexpr int W = kLeafMaxWidth;
+    constexpr int BS = W + 4;
+    constexpr int NT = 2 * RT / 4;    // 32 x 32 tiles per wave: 1 (RT = 2) or 2 (RT = 4)
+    static_assert(RT == 2 || RT == 4, "64 or 128 rows");
+    __shared__ __align__(16) float s_b[W * BS];  // [column][row], then U in the same place
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane & 31, lk = lane >> 5;
+    const int col0 = static_cast<int>(blockIdx.y) * W, cols = min(W, hi - (c0 + W) - col0);
+    const int row0 = c0 + W + static_cast<int>(blockIdx.x) * (32 * RT);
+    float* const Ct = A + (c0 + W + col0) * lda;
+    // Wave: rows wr .. wr + 31 of the tile, 32-column strips ws, ws + CT, ...
+    const int row = row0 + (wave % RT) * 32 + li, ws = wave / RT;
+    const bool inRow = row < m;
+    // inv(L11) fragments for this wave's 16 columns of U: all 64 rows, k ascending.
+    const int ui = lane & 15, uk = lane >> 4;
+    float lf[40], l21[32], cv[NT][16];
+#pragma unroll
+    for (int t = 0, x = 0; t < 4; ++t)
+#pragma unroll
+        for (int k = 0; k < 4 * (t + 1); ++k, ++x) lf[x] = linv[(4 * k + uk) * W + 16 * t + ui];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+    {
+        const int c = tid >> 4, r4 = (tid & 15) * 4;
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (c + 16 * t < cols) v = *reinterpret_cast<const float4*>(ub + static_cast<size_t>(col0 + c + 16 * t) * W + r4);
+        *reinterpret_cast<float4*>(s_b + (c + 16 * t) * BS + r4) = v;
+    }
+    const float* lp = A + c0 * lda + row + lk * lda;
+#pragma unroll
+    for (int t = 0; t < 32; ++t)
+    {
+        l21[t] = inRow ? *lp : 0.0f;
+        lp += 2 * lda;
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+        {
+            const int c = (ws + n * (2 / NT)) * 32 + (v & 3) + 8 * (v >> 2) + 4 * lk;
+            cv[n][v] = inRow && c < cols ? Ct[c * lda + row] : 0.0f;
+        }
+    __syncthreads();
+    // U, columns 16 wave .. 16 wave + 15: lane (ui, uk) of product t gets rows 16 t + 4 uk + r.
+    f32x4 uacc[4];
+#pragma unroll
+    for (int t = 0, x = 0; t < 4; ++t)
+    {
+        uacc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 4 * (t + 1); ++k, ++x)
+            uacc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(lf[x], s_b[(16 * wave + ui) * BS + 4 * k + uk], uacc[t], 0, 0, 0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        *reinterpret_cast<f32x4*>(s_b + (16 * wave + ui) * BS + 16 * t + 4 * uk) = uacc[t];
+    __syncthreads();
+    if (blockIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            if (16 * wave + k < cols) Ct[(16 * wave + k) * lda + c0 + lane] = s_b[(16 * wave + k) * BS + lane];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+    {
+        const int strip = (ws + n * (2 / NT)) * 32;
+        f32x16 acc;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 32; ++t)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s_b[(strip + li) * BS + 2 * t + lk], l21[t], acc, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+        {
+            const int c = strip + (v & 3) + 8 * (v >> 2) + 4 * lk;
+            if (inRow && c < cols) Ct[c * lda + row] = cv[n][v] - acc[v];
+        }
+    }
+}
+
 template <int NW, int RP>
 hipError_t Single(const LeafArgs& a, hipStream_t stream)
 {
@@ -744,6 +958,32 @@ hipError_t LeafSwap(const LeafArgs& a, hipStream_t stream)
     const int cols = a.panelEnd - a.j0;
     hipLaunchKernelGGL(leaf_swap_kernel, dim3((cols + 3) / 4), dim3(256), 0, stream, a.A, a.lda, a.j0, a.panelEnd, a.wact,
                        reinterpret_cast<const int2*>(a.moves), a.err);
+    return hipGetLastError();
+}
+
+hipError_t LeafFinish(const LeafArgs& a, float* linv, float* ub, hipStream_t stream)
+{
+    const int others = (a.c0 - a.j0) + (a.panelEnd - a.c0 - a.wact);
+    hipLaunchKernelGGL(leaf_finish_kernel, dim3(1 + (others + 3) / 4), dim3(256), 0, stream, a.A,
+                       static_cast<int64_t>(a.lda), a.j0, a.c0, a.wact, a.panelEnd,
+                       reinterpret_cast<const int2*>(a.moves), a.err, linv, ub);
+    return hipGetLastError();
+}
+
+hipError_t PanelUpdate(const LeafArgs& a, const float* linv, const float* ub, hipStream_t stream)
+{
+    const int cols = a.panelEnd - a.c0 - kLeafMaxWidth, rows = a.m - a.c0 - kLeafMaxWidth;
+    if (a.wact != kLeafMaxWidth) return hipErrorInvalidValue;
+    if (cols <= 0) return hipSuccess;
+    const int nc = (cols + 63) / 64;
+    // 64-row tiles while they leave the chip room (one wave then carries one 32 x 32 tile), 128
+    // above, where the repeated formation of U would cost more.
+    if ((rows + 63) / 64 * nc <= 512)
+        hipLaunchKernelGGL(panel_update_kernel<2>, dim3(std::max(1, (rows + 63) / 64), nc), dim3(256), 0, stream, a.A,
+                           static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, linv, ub);
+    else
+        hipLaunchKernelGGL(panel_update_kernel<4>, dim3((rows + 127) / 128, nc), dim3(256), 0, stream, a.A,
+                           static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, linv, ub);
     return hipGetLastError();
 }
 }  // namespace ops
