@@ -300,10 +300,12 @@ OPS_API aclsolverStatus_t aclsolverSgetrsDevice(aclsolverHandle_t handle, int tr
         arg = 9;
     if (arg) return Invalid(handle, devInfo, 1, arg);
     hipStream_t s = Stream(handle);
-    FillInfo(devInfo, 1, 0, s);
-    if (n == 0 || nrhs == 0) return Launched();
-    void* work = HandleScratch(handle, RealGetrsWorkspaceBytes(n, nrhs));
-    if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
+    void* work = n > 0 && nrhs > 0 ? HandleScratch(handle, RealGetrsWorkspaceBytes(n, nrhs)) : nullptr;
+    if (work == nullptr)
+    {
+        FillInfo(devInfo, 1, 0, s);
+        return n == 0 || nrhs == 0 ? Launched() : ACLSOLVER_STATUS_ALLOC_FAILED;
+    }
     if (RealGetrs(trans, n, nrhs, dA, lda, devIpiv, dB, ldb, work, s, devInfo) != hipSuccess)
         return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();
@@ -373,7 +375,7 @@ OPS_API aclError aclsolverSgetrs(aclsolverHandle_t handle, const uint64_t trans,
 // ---------------------------------------------------------------------------------------
 static size_t GetriWorkBytes(int n)
 {
-    return static_cast<size_t>(n) * n * sizeof(float) + RealGetrsWorkspaceBytes(n, n) + 256;
+    return static_cast<size_t>(n) * n * sizeof(float) + RealGetrsStagingBytes(n, n) + 256;
 }
 
 OPS_API aclsolverStatus_t aclsolverSgetri_bufferSize(aclsolverHandle_t handle, int n, float* A, int lda, int* Lwork)
@@ -427,6 +429,9 @@ OPS_API aclsolverStatus_t aclsolverSgetri(aclsolverHandle_t handle, int n, float
     float* X = Workspace;
     void* work = reinterpret_cast<char*>(Workspace) + static_cast<size_t>(n) * n * sizeof(float);
     work = reinterpret_cast<char*>(work) + (256 - reinterpret_cast<uintptr_t>(work) % 256) % 256;
+    if (RealGetrsWorkspaceBytes(n, n) > RealGetrsStagingBytes(n, n))
+        work = HandleScratch(handle, RealGetrsWorkspaceBytes(n, n));
+    if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
     hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, A, lda, devInfo);
     hipLaunchKernelGGL(set_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, X, n);
     if (RealGetrs(0, n, n, A, lda, devIpiv, X, n, work, s) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;

@@ -23,6 +23,7 @@
 
 #include "leaf.h"
 #include "lu_kernels.h"
+#include "trs.h"
 #include "trsv.h"
 #include "tslu.h"
 #include "wave.h"
@@ -582,18 +583,29 @@ int SolveBlock(int n) { return n >= 4096 ? 256 : 128; }
 
 namespace
 {
-size_t GetrsVectorBytes(int n, int nrhs)
+// Chained substitutions (trs.hip) or, for many right-hand sides of a large system, blocked
+// ones, whose 128 x 128 products then outrun the chain's; also where the chain's padding to 64
+// rows would waste memory, and for the few problems that the no-allocation entry point takes
+// and whose chain does not fit its array (it promises the results of the allocating one).
+bool UseTrs(int n, int nrhs)
 {
-    return ((static_cast<size_t>(n) * std::max(nrhs, 1) + static_cast<size_t>(n) + 64) * sizeof(float) + 255) / 256 *
-           256;
+    if (n > 4096 && nrhs > 256) return false;
+    if (n < 16 && nrhs > 1024) return false;
+    return RealGetrsStagingBytes(n, nrhs) > ACLSOLVER_NOALLOC_SCRATCH_BYTES ||
+           TrsWorkspaceBytes(n, nrhs, true) <= kNoAllocArrayBytes;
 }
-// One right-hand side of at least this order uses the single-launch chained solve.
-constexpr int kChainMinN = 512;
 }  // namespace
+
+size_t RealGetrsStagingBytes(int n, int nrhs)
+{
+    const size_t vectors =
+        ((static_cast<size_t>(n) * std::max(nrhs, 1) + static_cast<size_t>(n) + 64) * sizeof(float) + 255) / 256 * 256;
+    return vectors + TrsvChainStateBytes(std::max(n, 1));
+}
 
 size_t RealGetrsWorkspaceBytes(int n, int nrhs)
 {
-    return GetrsVectorBytes(n, nrhs) + TrsvChainStateBytes(std::max(n, 1));
+    return UseTrs(n, nrhs) ? TrsWorkspaceBytes(n, nrhs, true) : RealGetrsStagingBytes(n, nrhs);
 }
 
 // Triangular solves on a column-major n x nrhs block X (ldx) with packed LU factors.
@@ -704,6 +716,8 @@ hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const
                      void* work, hipStream_t stream, int* info)
 {
     if (n <= 0 || nrhs <= 0) return hipSuccess;
+    if (UseTrs(n, nrhs)) return TrsSolve(trans, n, nrhs, lu, lda, ipiv, b, ldb, b, ldb, info, work, nullptr, stream);
+    if (info != nullptr) FillInfo(info, 1, 0, stream);
     float* x = static_cast<float*>(work);
     int* perm = reinterpret_cast<int*>(x + static_cast<size_t>(n) * nrhs);
     if (ipiv) RET_IF(IpivToPerm(n, ipiv, perm, stream));
@@ -711,16 +725,7 @@ hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const
     if (trans == 0)
     {
         RET_IF(PermuteRows(true, n, nrhs, p, b, ldb, x, n, stream));
-        if (nrhs == 1 && n >= kChainMinN)
-        {
-            TrsvChainState ts = TrsvChainLayout(static_cast<char*>(work) + GetrsVectorBytes(n, nrhs), n);
-            RET_IF(TrsvChainReset(ts, stream));
-            RET_IF(TrsvChain(ts, false, lu, lda, x, stream));
-            RET_IF(TrsvChain(ts, true, lu, lda, x, stream));
-            FoldWaitError(ts.err, info, stream);
-        }
-        else
-            RET_IF(RealLuSolveInPlace(0, n, nrhs, lu, lda, x, n, stream));
+        RET_IF(RealLuSolveInPlace(0, n, nrhs, lu, lda, x, n, stream));
         // copy back
         RET_IF(PermuteRows(true, n, nrhs, nullptr, x, n, b, ldb, stream));
     }

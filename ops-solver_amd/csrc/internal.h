@@ -92,6 +92,9 @@ void* HandleScratch(aclsolverHandle_t h, size_t bytes);
 // Device address of this device's fixed no-allocation scratch array (noalloc.hip), looked
 // up once per device with the device current; nullptr when the lookup fails.
 void* NoAllocScratch(int device);
+// Its size: the documented ACLSOLVER_NOALLOC_SCRATCH_BYTES bound what a solve stages by
+// RealGetrsStagingBytes, the chained solves use up to this much for such problems.
+constexpr size_t kNoAllocArrayBytes = size_t{36} << 20;
 // Once per device at handle creation: may the tall panel leaves exchange through one XCD's
 // L2 (getrf.hip)?
 void LeafSpreadProbe(int device);
@@ -169,7 +172,10 @@ hipError_t RealGetrfPerm(int m, int n, float* a, int lda, int* ipiv, int* info, 
                          int* permOut, hipStream_t stream, void* pack, const LookAhead* la, bool tournament = false);
 // Device column-major getrs from RealGetrf factors (trans 0 / 1). work: RealGetrsWorkspaceBytes.
 size_t RealGetrsWorkspaceBytes(int n, int nrhs);
-// info (optional, Device): set to kInfoWaitTimeout when a bounded wait of the solve gave up.
+// What callers are told a solve stages (the sizes that the no-allocation entry point accepts,
+// the getri workspace query); the chained solves keep their own layout.
+size_t RealGetrsStagingBytes(int n, int nrhs);
+// info (optional, Device): set to 0, or to kInfoWaitTimeout when a bounded wait of the solve gave up.
 hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const int* ipiv, float* b, int ldb,
                      void* work, hipStream_t stream, int* info = nullptr);
 

@@ -35,6 +35,7 @@
 #include <climits>
 
 #include "internal.h"
+#include "trtri64.h"
 #include "wave.h"
 
 namespace ops
@@ -688,25 +689,6 @@ __global__ __launch_bounds__(256) void leaf_swap_kernel(float* __restrict__ A, i
 // columns (it needs them in place for the inverse), the others a wave per column left and
 // right of it. The top 64 rows of the right columns go to ub (ld 64) instead of A: the launch
 // that turns them into U writes A while its other workgroups still read them.
-// The inverse is bound by latency: 16 x 16 diagonal blocks by substitution, one lane per
-// column, then two doublings by products on the matrix cores (a substitution over the whole
-// block took 64 dependent steps and 18 us of mostly instruction fetches).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kInvStride = 68;
-
-// D (16 x 16 at d) = sign * A (16 x K at a) * B (K x 16 at b), row-major in LDS, one wave.
-template <int K>
-__device__ inline void Product16(const float* a, const float* b, float* d, float sign, int lane)
-{
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int i = lane & 15, k0 = lane >> 4;
-#pragma unroll
-    for (int k = 0; k < K; k += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i * kInvStride + k + k0], b[(k + k0) * kInvStride + i], acc, 0, 0, 0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) d[(4 * k0 + r) * kInvStride + i] = sign * acc[r];
-}
-
 __global__ __launch_bounds__(256) void leaf_finish_kernel(float* __restrict__ A, int64_t lda, int j0, int c0, int wact,
                                                           int hi, const int2* __restrict__ moves,
                                                           const int* __restrict__ err, float* __restrict__ linv,
@@ -764,38 +746,7 @@ __global__ __launch_bounds__(256) void leaf_finish_kernel(float* __restrict__ A,
         s_i[lane * kInvStride + c] = 0.0f;
     }
     __syncthreads();
-    if (wave == 0)
-    {
-        // Lane: column lane % 16 of diagonal block lane / 16.
-        const int b = lane & 48;
-        float x[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-        {
-            float v = i == (lane & 15) ? 1.0f : 0.0f;
-            const float* const row = s_l + (b + i) * kInvStride + b;
-#pragma unroll
-            for (int k = 0; k < i; ++k) v = fmaf(-row[k], x[k], v);
-            x[i] = v;
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s_i[(b + i) * kInvStride + lane] = x[i];
-    }
-    __syncthreads();
-    // inv [P 0; Q R] = [P' 0; -R' Q P' R'] with 16 x 16, then 32 x 32 blocks.
-    if (wave < 2)
-        Product16<16>(s_l + (32 * wave + 16) * kInvStride + 32 * wave, s_i + 32 * wave * kInvStride + 32 * wave,
-                      s_t + 16 * wave * kInvStride, 1.0f, lane);
-    __syncthreads();
-    if (wave < 2)
-        Product16<16>(s_i + (32 * wave + 16) * kInvStride + 32 * wave + 16, s_t + 16 * wave * kInvStride,
-                      s_i + (32 * wave + 16) * kInvStride + 32 * wave, -1.0f, lane);
-    __syncthreads();
-    const int qr = 16 * (wave >> 1), qc = 16 * (wave & 1);
-    Product16<32>(s_l + (32 + qr) * kInvStride, s_i + qc, s_t + qr * kInvStride + qc, 1.0f, lane);
-    __syncthreads();
-    Product16<32>(s_i + (32 + qr) * kInvStride + 32, s_t + qc, s_i + (32 + qr) * kInvStride + qc, -1.0f, lane);
-    __syncthreads();
+    InvertLower64<true>(s_l, s_i, s_t, tid);
 #pragma unroll
     for (int k = 0; k < 16; ++k)
     {

@@ -24,7 +24,7 @@ namespace
 constexpr size_t kNoAllocScratchBytes = ACLSOLVER_NOALLOC_SCRATCH_BYTES;
 constexpr int kMaxDevices = 64;
 
-__device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+__device__ __align__(256) unsigned char scratch[kNoAllocArrayBytes];
 
 std::mutex g_mutex;
 void* g_ptr[kMaxDevices] = {};
@@ -61,9 +61,9 @@ OPS_API aclsolverStatus_t aclsolverSgetrsDeviceNoAlloc(aclsolverHandle_t handle,
     int arg = 0;
     if (trans < 0 || trans > 1)
         arg = 1;
-    else if (n < 0 || n > kEngineMaxOrder || RealGetrsWorkspaceBytes(n, 1) > kNoAllocScratchBytes)
+    else if (n < 0 || n > kEngineMaxOrder || RealGetrsStagingBytes(n, 1) > kNoAllocScratchBytes)
         arg = 2;
-    else if (nrhs < 0 || RealGetrsWorkspaceBytes(n, nrhs) > kNoAllocScratchBytes)
+    else if (nrhs < 0 || RealGetrsStagingBytes(n, nrhs) > kNoAllocScratchBytes)
         arg = 3;
     else if (n > 0 && !IsDevice(dA))
         arg = 4;
@@ -87,8 +87,11 @@ OPS_API aclsolverStatus_t aclsolverSgetrsDeviceNoAlloc(aclsolverHandle_t handle,
     void* work = NoAllocScratch(device);
     if (work == nullptr) return ACLSOLVER_STATUS_EXECUTION_FAILED;
     hipStream_t s = Stream(handle);
-    FillInfo(devInfo, 1, 0, s);
-    if (n == 0 || nrhs == 0) return Launched();
+    if (n == 0 || nrhs == 0)
+    {
+        FillInfo(devInfo, 1, 0, s);
+        return Launched();
+    }
     if (RealGetrs(trans, n, nrhs, dA, lda, devIpiv, dB, ldb, work, s, devInfo) != hipSuccess)
         return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();

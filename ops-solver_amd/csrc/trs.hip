@@ -1,0 +1,474 @@
+// Device triangular solves from packed LU factors with any number of right-hand sides, gfx950.
+// Reference: src/sgetrs/real_getrs_kernel.cpp (row permutation, unit-lower and upper solves).
+//
+// One launch per triangle. A workgroup owns 64 rows of up to 64 right-hand sides and walks the
+// blocks it depends on in the order in which they are finished: it waits for X_k, subtracts
+// T(i, k) X_k on the FP32 matrix cores (the next tile of T is loaded meanwhile), and at the end
+// applies the FP64 inverse of its diagonal block on the FP64 matrix cores and publishes X_i as
+// tagged 64-bit words (32-bit tag, value), so that a consumer needs neither a flag nor a fence.
+// Tickets hand out the blocks in dependency order: the block with the lowest unfinished ticket
+// never waits for a workgroup that has not started. With the inverse in FP64 the block solve
+// rounds once; an FP32 inverse, applied once or with a step of refinement in FP32, erred more
+// than the substitution it replaces (Gaussian systems of order 64 to 4096, against 64 bits).
+//
+// What bounds it: the chain, one device-wide trip, two products and a few barriers per 64
+// rows. 64 rows: the longest block whose inverse four waves apply from registers.
+#include "trs.h"
+
+#include <algorithm>
+#include <cfloat>
+#include <climits>
+
+#include "internal.h"
+#include "trtri64.h"
+
+namespace ops
+{
+namespace
+{
+constexpr int NBK = 64;
+
+__device__ inline unsigned long long LoadWord(const unsigned long long* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+struct Trs
+{
+    int trans, n, nrhs, lda, lds, ldb;
+    const float* lu;
+    const int* ipiv;
+    const float* src;  // null: the identity
+    float* B;
+    int* info;
+    unsigned long long* pub;  // X words: [block][strip][row][column], 64 rows, strips of 16 CG columns
+    double* inv;              // inverses of the diagonal blocks of op(L), op(U): row-major 64 x 64
+    int* bad;                 // per diagonal block: its inverse is not finite (2 nb ints)
+    int* perm;
+    unsigned* ticket;         // [2]
+    unsigned spinLimit;
+};
+
+// Preparation, by workgroup: 2 nb diagonal blocks inverted, the permutation (256 positions
+// each), the publication words cleared.
+__global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, size_t words)
+{
+    extern __shared__ __align__(16) double s_mem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int b = blockIdx.x;
+    if (b == 0 && tid == 0)
+    {
+        p.ticket[0] = p.ticket[1] = 0u;
+        if (p.info != nullptr) *p.info = 0;
+    }
+    if (b < 2 * nb)
+    {
+        const bool upper = b >= nb;
+        const int k0 = (upper ? b - nb : b) * NBK, kb = min(NBK, p.n - k0);
+        double* const s_l = s_mem;
+        double* const s_i = s_mem + 64 * kInvStride;
+        double* const s_t = s_i + 64 * kInvStride;
+        const float* const T = p.lu + static_cast<size_t>(k0) * p.lda + k0;
+        // Lower: the block; upper: its transpose. Rows beyond the block are the identity.
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+        {
+            const int c = wave * 16 + k;
+            const float v = lane < kb && c < kb ? T[static_cast<size_t>(c) * p.lda + lane] : (lane == c ? 1.0f : 0.0f);
+            if (!upper)
+                s_l[lane * kInvStride + c] = lane > c ? v : 0.0;
+            else
+                s_l[c * kInvStride + lane] = lane <= c ? v : 0.0;
+            s_i[lane * kInvStride + c] = 0.0;
+        }
+        __syncthreads();
+        if (upper)
+            InvertLower64<false>(s_l, s_i, s_t, tid);
+        else
+            InvertLower64<true>(s_l, s_i, s_t, tid);
+        // Row-major inverse of op(T): L^-1 and (U^T)^-1 as they are, the other two transposed.
+        double* const out = p.inv + static_cast<size_t>(b) * 4096;
+        const bool flip = upper != (p.trans != 0);
+        bool fine = true;
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+        {
+            const int r = wave * 16 + k;
+            const double v = flip ? s_i[lane * kInvStride + r] : s_i[r * kInvStride + lane];
+            fine = fine && fabs(v) <= FLT_MAX;
+            out[r * 64 + lane] = v;
+        }
+        if (!__syncthreads_and(fine))
+        {
+            if (tid == 0) p.bad[b] = 1;
+        }
+        else if (tid == 0)
+            p.bad[b] = 0;
+        return;
+    }
+    b -= 2 * nb;
+    if (b < np)
+    {
+        // perm[i] = source row of row i of P B: position i traced backward through the
+        // interchanges. LAPACK pivots never point above their own row, so position i is first
+        // met by interchange i, and from there on only "x == pivot" can move it; any entry that
+        // does point above takes the general trace.
+        int* const s_piv = reinterpret_cast<int*>(s_mem);
+        const int i = b * 256 + tid, last = min(p.n, b * 256 + 256);
+        bool plain = true;
+        for (int k = tid; k < p.n; k += 256)
+        {
+            int v = p.ipiv[k] - 1;
+            if (v < 0 || v >= p.n) v = k;
+            plain = plain && v >= k;
+            s_piv[k] = v;
+        }
+        plain = __syncthreads_and(plain);
+        int x = i;
+        if (plain)
+        {
+            const int base = b * 256 + wave * 64;  // this wave's first position
+            if (i < p.n) x = s_piv[i];
+            for (int k = min(last, base + 64) - 1; k >= base && k >= 0; --k) x = k < i && s_piv[k] == x ? k : x;
+            int k = base - 1;
+#pragma unroll 1
+            for (; k >= 3; k -= 4)
+            {
+                const int4 v = *reinterpret_cast<const int4*>(s_piv + k - 3);  // k + 1 is a multiple of 64
+                x = v.w == x ? k : x;
+                x = v.z == x ? k - 1 : x;
+                x = v.y == x ? k - 2 : x;
+                x = v.x == x ? k - 3 : x;
+            }
+        }
+        else
+            for (int k = p.n - 1; k >= 0; --k)
+            {
+                const int v = s_piv[k];
+                x = x == k ? v : (x == v ? k : x);
+            }
+        if (i < p.n) p.perm[i] = x;
+        return;
+    }
+    b -= np;
+    const size_t step = static_cast<size_t>(gridDim.x - 2 * nb - np) * 256;
+    for (size_t w = static_cast<size_t>(b) * 256 + tid; w < words; w += step) p.pub[w] = 0ull;
+}
+
+// SECOND: the second substitution of the solve (reads the first one's words, writes B).
+// TRANS: op(T) = T^T. CG: 16-column groups per strip.
+// Tile operand: lane (li, g) holds row 16 wave + li of the tile and its columns 16 q + 4 g + t,
+// q, t = 0..3, so that the four columns of a lane are consecutive; the other operand is read
+// from LDS in the same order.
+template <bool TRANS, bool SECOND, int CG>
+__global__ __launch_bounds__(256) void trs_chain_kernel(Trs p, int nb, int strips)
+{
+    constexpr bool UPPER = TRANS != SECOND;  // N: L then U; T: U^T then L^T
+    constexpr bool BACK = SECOND;            // both second substitutions run upward
+    constexpr int NS = 16 * CG, S = NS + 4;
+    constexpr int PER = 64 * NS / 256;
+    constexpr unsigned TAG = SECOND ? 2u : 1u;
+    __shared__ __align__(16) float s_x[2][64 * S];
+    __shared__ unsigned s_id;
+    __shared__ int s_fail;  // a wait of this workgroup ran out
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, g = lane >> 4;
+    if (tid == 0)
+    {
+        s_id = atomicAdd(p.ticket + (SECOND ? 1 : 0), 1u);
+        s_fail = 0;
+    }
+    __syncthreads();
+    const int id = static_cast<int>(s_id);
+    const int step = id / strips, strip = id - step * strips;
+    const int ib = BACK ? nb - 1 - step : step;
+    const int r0 = ib * NBK, c0 = strip * NS;
+    const int row = r0 + 16 * wave + li;
+    const bool inRow = row < p.n;
+    const bool vec = TRANS && p.lda % 4 == 0 && (reinterpret_cast<uintptr_t>(p.lu) & 15) == 0;
+
+    auto loadTile = [&](int kb, float (&t)[16])
+    {
+        const int k0 = kb * NBK;
+        if (TRANS)
+        {
+            const float* const col = p.lu + static_cast<size_t>(inRow ? row : 0) * p.lda + k0 + 4 * g;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (vec && k0 + NBK <= p.n)  // uniform
+                {
+                    const float4 v = inRow ? *reinterpret_cast<const float4*>(col + 16 * q) : make_float4(0, 0, 0, 0);
+                    t[4 * q] = v.x;
+                    t[4 * q + 1] = v.y;
+                    t[4 * q + 2] = v.z;
+                    t[4 * q + 3] = v.w;
+                }
+                else
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        t[4 * q + e] = inRow && k0 + 16 * q + 4 * g + e < p.n ? col[16 * q + e] : 0.0f;
+        }
+        else
+        {
+            const float* const col = p.lu + static_cast<size_t>(k0) * p.lda + row;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const int k = 16 * q + 4 * g + e;
+                    t[4 * q + e] = inRow && k0 + k < p.n ? col[static_cast<size_t>(k) * p.lda] : 0.0f;
+                }
+        }
+    };
+    auto multiply = [&](const float* s, const float (&t)[16], f32x4 (&acc)[CG])
+    {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < CG; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[(16 * q + 4 * g + e) * S + 16 * c + li],
+                                                                  t[4 * q + e], acc[c], 0, 0, 0);
+    };
+
+    // Right-hand side: lane (li, g) holds row li of its wave, columns 16 c + 4 g + r.
+    f32x4 rhs[CG];
+    {
+        int from = row;
+        if (!SECOND && !TRANS && p.ipiv != nullptr && inRow) from = p.perm[row];
+        const unsigned long long* const mine =
+            p.pub + (static_cast<size_t>(ib) * strips + strip) * (64 * NS) + (16 * wave + li) * NS;
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+            {
+                const int col = 16 * c + 4 * g + r;
+                float v = 0.0f;
+                if (SECOND)
+                    v = __uint_as_float(static_cast<unsigned>(mine[col]));
+                else if (inRow && c0 + col < p.nrhs)
+                    v = p.src == nullptr ? (from == c0 + col ? 1.0f : 0.0f)
+                                         : p.src[static_cast<size_t>(c0 + col) * p.lds + from];
+                rhs[c][r] = v;
+            }
+    }
+    float cur[16], nxt[16];
+    double iv[16];
+    if (step > 0) loadTile(BACK ? nb - 1 : 0, cur);
+    {
+        const double* const in = p.inv + static_cast<size_t>(UPPER ? nb + ib : ib) * 4096 + (16 * wave + li) * 64 + 4 * g;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) iv[4 * q + e] = in[16 * q + e];
+    }
+    const int bad = p.bad[UPPER ? nb + ib : ib];
+    bool failed = false;  // uniform over the workgroup
+    for (int s = 0; s < step; ++s)
+    {
+        const int kb = BACK ? nb - 1 - s : s;
+        if (s + 1 < step) loadTile(BACK ? kb - 1 : kb + 1, nxt);
+        const unsigned long long* const words = p.pub + (static_cast<size_t>(kb) * strips + strip) * (64 * NS);
+        unsigned long long w[PER];
+        bool ok = false;
+        const unsigned lim = failed ? 0u : p.spinLimit;
+        for (unsigned spins = 0; spins < lim && !ok; ++spins)
+        {
+            // One word per lane until it is there, then all.
+            w[0] = LoadWord(words + tid);
+            ok = __all(static_cast<unsigned>(w[0] >> 32) == TAG);
+            if (ok)
+            {
+#pragma unroll
+                for (int i = 1; i < PER; ++i) w[i] = LoadWord(words + tid + 256 * i);
+                bool all = true;
+#pragma unroll
+                for (int i = 1; i < PER; ++i) all = all && static_cast<unsigned>(w[i] >> 32) == TAG;
+                ok = __all(all);
+            }
+            if (!ok) __builtin_amdgcn_s_sleep(1);
+        }
+        float* const x = s_x[s & 1];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+        {
+            const int at = tid + 256 * i;
+            x[(at / NS) * S + at % NS] = __uint_as_float(static_cast<unsigned>(w[i]));
+        }
+        if (!ok && lane == 0) s_fail = 1;
+        __syncthreads();
+        failed = s_fail != 0;
+        // Each block's product is summed from zero and subtracted once: one long sum over the
+        // row would round more.
+        f32x4 acc[CG];
+#pragma unroll
+        for (int c = 0; c < CG; ++c) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        multiply(x, cur, acc);
+#pragma unroll
+        for (int c = 0; c < CG; ++c) rhs[c] = rhs[c] - acc[c];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) cur[e] = nxt[e];
+    }
+    __syncthreads();
+    float* const s_r = s_x[0];
+    float* const s_y = s_x[1];
+    f32x4 x0[CG];
+#pragma unroll
+    for (int c = 0; c < CG; ++c)
+        *reinterpret_cast<f32x4*>(s_r + (16 * wave + li) * S + 16 * c + 4 * g) = rhs[c];
+    __syncthreads();
+    if (__builtin_expect(bad == 0, 1))  // uniform
+    {
+        // The FP64 matrix cores return row 4 r + g in element r: fed with the columns in the order
+        // 4 (i mod 4) + i / 4, lane (li, g) gets columns 4 g + r as everywhere else.
+        f64x4 wide[CG];
+#pragma unroll
+        for (int c = 0; c < CG; ++c) wide[c] = f64x4{0.0, 0.0, 0.0, 0.0};
+        const int sig = 4 * (li & 3) + (li >> 2);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < CG; ++c)
+                    wide[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        static_cast<double>(s_r[(16 * q + 4 * g + e) * S + 16 * c + sig]), iv[4 * q + e], wide[c], 0, 0,
+                        0);
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x0[c][r] = static_cast<float>(wide[c][r]);
+    }
+    else
+    {
+        // A zero pivot (or an inverse beyond the range): plain substitution, as LAPACK's.
+        for (int e = 0; e < 64; ++e)
+        {
+            const int k = BACK ? 63 - e : e;
+            if (r0 + k >= p.n) continue;  // uniform
+            const float d = p.lu[static_cast<size_t>(r0 + k) * p.lda + r0 + k];
+            __syncthreads();
+            for (int at = tid; at < 64 * NS; at += 256)
+            {
+                const int r = at / NS, c = at - r * NS;
+                if (r == k) s_y[k * S + c] = UPPER ? s_r[k * S + c] / d : s_r[k * S + c];
+            }
+            __syncthreads();
+            for (int at = tid; at < 64 * NS; at += 256)
+            {
+                const int r = at / NS, c = at - r * NS;
+                if (r0 + r < p.n && (BACK ? r < k : r > k))
+                {
+                    const float t = TRANS ? p.lu[static_cast<size_t>(r0 + r) * p.lda + r0 + k]
+                                          : p.lu[static_cast<size_t>(r0 + k) * p.lda + r0 + r];
+                    s_r[r * S + c] = fmaf(-t, s_y[k * S + c], s_r[r * S + c]);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < CG; ++c) x0[c] = *reinterpret_cast<const f32x4*>(s_y + (16 * wave + li) * S + 16 * c + 4 * g);
+    }
+    if (failed)
+    {
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x0[c][r] = __builtin_nanf("");
+        if (tid == 0 && p.info != nullptr) *p.info = kInfoWaitTimeout;
+    }
+    unsigned long long* const words =
+        p.pub + (static_cast<size_t>(ib) * strips + strip) * (64 * NS) + (16 * wave + li) * NS;
+    int to = row;
+    if (SECOND && TRANS && p.ipiv != nullptr && inRow) to = p.perm[row];
+#pragma unroll
+    for (int c = 0; c < CG; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const int col = 16 * c + 4 * g + r;
+            __hip_atomic_store(words + col,
+                               (static_cast<unsigned long long>(TAG) << 32) | __float_as_uint(inRow ? x0[c][r] : 0.0f),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    if (SECOND)
+#pragma unroll
+        for (int c = 0; c < CG; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+            {
+                const int col = 16 * c + 4 * g + r;
+                if (inRow && c0 + col < p.nrhs) p.B[static_cast<size_t>(c0 + col) * p.ldb + to] = x0[c][r];
+            }
+}
+
+// 16 columns per strip for up to 32 right-hand sides, else 64.
+int GroupsPerStrip(int nrhs) { return nrhs <= 32 ? 1 : 4; }
+
+template <bool TRANS, int CG>
+void Chains(const Trs& p, int nb, int strips, hipStream_t stream)
+{
+    hipLaunchKernelGGL((trs_chain_kernel<TRANS, false, CG>), dim3(nb * strips), dim3(256), 0, stream, p, nb, strips);
+    hipLaunchKernelGGL((trs_chain_kernel<TRANS, true, CG>), dim3(nb * strips), dim3(256), 0, stream, p, nb, strips);
+}
+
+size_t Up(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
+}  // namespace
+
+size_t TrsPublicationBytes(int n, int nrhs)
+{
+    const int ns = 16 * GroupsPerStrip(nrhs);
+    return static_cast<size_t>((n + NBK - 1) / NBK) * NBK * ((nrhs + ns - 1) / ns * ns) * sizeof(unsigned long long);
+}
+
+size_t TrsWorkspaceBytes(int n, int nrhs, bool withPublication)
+{
+    const size_t nb = (n + NBK - 1) / NBK;
+    return Up(2 * nb * 4096 * sizeof(double)) + Up(2 * nb * sizeof(int)) + Up(n * sizeof(int)) + 256 +
+           (withPublication ? Up(TrsPublicationBytes(n, nrhs)) : 0) + 256;
+}
+
+hipError_t TrsSolve(int trans, int n, int nrhs, const float* lu, int lda, const int* ipiv, const float* src, int lds,
+                    float* B, int ldb, int* info, void* work, void* pub, hipStream_t stream)
+{
+    if (n <= 0 || nrhs <= 0) return hipSuccess;
+    if (n > kEngineMaxOrder) return hipErrorInvalidValue;
+    const int nb = (n + NBK - 1) / NBK, cg = GroupsPerStrip(nrhs), strips = (nrhs + 16 * cg - 1) / (16 * cg);
+    char* q = reinterpret_cast<char*>(Up(reinterpret_cast<uintptr_t>(work)));
+    auto take = [&](size_t bytes) {
+        char* const at = q;
+        q += Up(bytes);
+        return at;
+    };
+    Trs p{};
+    p.trans = trans;
+    p.n = n;
+    p.nrhs = nrhs;
+    p.lda = lda;
+    p.lds = lds;
+    p.ldb = ldb;
+    p.lu = lu;
+    p.ipiv = ipiv;
+    p.src = src;
+    p.B = B;
+    p.info = info;
+    p.inv = reinterpret_cast<double*>(take(static_cast<size_t>(2 * nb) * 4096 * sizeof(double)));
+    p.bad = reinterpret_cast<int*>(take(static_cast<size_t>(2 * nb) * sizeof(int)));
+    p.perm = reinterpret_cast<int*>(take(static_cast<size_t>(n) * sizeof(int)));
+    p.ticket = reinterpret_cast<unsigned*>(take(256));
+    const size_t words = TrsPublicationBytes(n, nrhs) / sizeof(unsigned long long);
+    p.pub = reinterpret_cast<unsigned long long*>(pub != nullptr ? pub : take(words * sizeof(unsigned long long)));
+    p.spinLimit = SpinLimit();
+    const int np = ipiv != nullptr ? (n + 255) / 256 : 0;
+    const int nz = static_cast<int>(std::min<size_t>((words + 1023) / 1024, 1024));
+    const size_t ldsBytes = std::max<size_t>((2 * 64 + 32) * kInvStride * sizeof(double), ipiv ? ((n + 3) & ~3) * sizeof(int) : 0);
+    hipLaunchKernelGGL(trs_prep_kernel, dim3(2 * nb + np + nz), dim3(256), ldsBytes, stream, p, nb, np, words);
+    if (trans == 0)
+        cg == 1 ? Chains<false, 1>(p, nb, strips, stream) : Chains<false, 4>(p, nb, strips, stream);
+    else
+        cg == 1 ? Chains<true, 1>(p, nb, strips, stream) : Chains<true, 4>(p, nb, strips, stream);
+    return hipGetLastError();
+}
+}  // namespace ops

@@ -22,8 +22,7 @@ TrsvChainState TrsvChainLayout(void* base, int n);
 hipError_t TrsvChainReset(TrsvChainState& s, hipStream_t stream);
 // x <- T^{-1} x for the unit lower (upper = false) or non-unit upper (upper = true)
 // triangle of the packed LU factors T (n x n, column-major, ldt). The upper solve divides
-// through a rounded reciprocal of each pivot. The double overload carries the whole
-// substitution in FP64 on the FP32 factors.
-hipError_t TrsvChain(TrsvChainState& s, bool upper, const float* T, int ldt, float* x, hipStream_t stream);
+// through a rounded reciprocal of each pivot. The whole substitution runs in FP64 on the FP32
+// factors.
 hipError_t TrsvChain(TrsvChainState& s, bool upper, const float* T, int ldt, double* x, hipStream_t stream);
 }  // namespace ops

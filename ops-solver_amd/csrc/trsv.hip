@@ -1,4 +1,5 @@
-// Single-launch triangular solve of one right-hand side with packed LU factors.
+// Single-launch triangular solve of one FP64 right-hand side with packed FP32 LU factors (the
+// preconditioner of the refined solvers; FP32 right-hand sides go through trs.hip).
 //
 // The blocked solve (a diagonal TRSM and a GEMV per block row, two launches per block)
 // is bound by launch latency for one vector: n = 16384 with 128-row blocks is 256
@@ -8,7 +9,7 @@
 // solves its own diagonal block and publishes x_b. The only serial part left is the chain
 // of diagonal solves plus one device-scope round trip per block.
 //
-// Publication: every solved entry is written as one 64-bit word (epoch << 32 | float
+// Publication: every solved entry is written as two 64-bit words (epoch << 32 | half of its
 // bits) with a relaxed agent-scope atomic store, and readers poll the words themselves, so
 // no separate flag or fence is needed and a stale word can never pass as current. Block
 // order comes from a ticket counter (a workgroup that draws ticket t only waits for
@@ -36,18 +37,6 @@ __device__ inline unsigned long long PollWord(const unsigned long long* p)
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Publication words of one solved entry: a float takes one word (epoch << 32 | bits), a
-// double two (low and high halves, each tagged with the epoch).
-template <typename V>
-struct Words
-{
-    static constexpr int count = sizeof(V) / 4;
-};
-
-__device__ inline float Broadcast(float v, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
 __device__ inline double Broadcast(double v, int lane)
 {
     const long long b = __double_as_longlong(v);
@@ -57,17 +46,18 @@ __device__ inline double Broadcast(double v, int lane)
 }
 
 // NB rows per block, 256 threads: wave w streams columns [w*NB/4, (w+1)*NB/4) of every
-// off-diagonal tile, lane l owns rows l, l+64, ... of the block. V is the vector type
-// (float, or double for a solve carried out in FP64 on FP32 factors).
-template <int NB, bool UPPER, typename V>
+// off-diagonal tile, lane l owns rows l, l+64, ... of the block. The vector is FP64, on FP32
+// factors: each entry takes two words (low and high half, each tagged with the epoch).
+template <int NB, bool UPPER>
 __global__ __launch_bounds__(256) void trsv_chain_kernel(int n, const float* __restrict__ T, int ldt,
-                                                         V* __restrict__ x, unsigned long long* __restrict__ pub,
+                                                         double* __restrict__ x, unsigned long long* __restrict__ pub,
                                                          unsigned* __restrict__ ticket, unsigned base, unsigned epoch,
                                                          int* __restrict__ err, unsigned spinLimit)
 {
     constexpr int RPL = NB / 64;  // rows per lane
     constexpr int CPW = NB / 4;   // tile columns per wave
-    constexpr int NW = Words<V>::count;
+    constexpr int NW = 2;
+    using V = double;
     __shared__ float s_diag[NB][NB + 1];
     __shared__ V s_part[4][NB];
     __shared__ V s_rinv[NB];
@@ -143,11 +133,7 @@ __global__ __launch_bounds__(256) void trsv_chain_kernel(int n, const float* __r
             }
             __builtin_amdgcn_s_sleep(2);
         }
-        V yv;
-        if constexpr (NW == 1)
-            yv = __uint_as_float(static_cast<unsigned>(w[0]));
-        else
-            yv = __longlong_as_double(static_cast<long long>((w[1] << 32) | (w[0] & 0xffffffffull)));
+        const V yv = __longlong_as_double(static_cast<long long>((w[1] << 32) | (w[0] & 0xffffffffull)));
 #pragma unroll
         for (int c = 0; c < CPW; ++c)
         {
@@ -227,19 +213,11 @@ __global__ __launch_bounds__(256) void trsv_chain_kernel(int n, const float* __r
         {
             x[r0 + r] = xv[q];
             const unsigned long long tag = static_cast<unsigned long long>(epoch) << 32;
-            if constexpr (NW == 1)
-            {
-                const unsigned long long word = tag | __float_as_uint(xv[q]);
-                __hip_atomic_store(pub + r0 + r, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            else
-            {
-                const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(xv[q]));
-                __hip_atomic_store(pub + 2 * static_cast<size_t>(r0 + r), tag | (b & 0xffffffffull), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(pub + 2 * static_cast<size_t>(r0 + r) + 1, tag | (b >> 32), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            }
+            const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(xv[q]));
+            __hip_atomic_store(pub + 2 * static_cast<size_t>(r0 + r), tag | (b & 0xffffffffull), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(pub + 2 * static_cast<size_t>(r0 + r) + 1, tag | (b >> 32), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
@@ -292,8 +270,7 @@ hipError_t TrsvChainReset(TrsvChainState& s, hipStream_t stream)
     return hipGetLastError();
 }
 
-template <typename V>
-hipError_t LaunchChain(TrsvChainState& s, bool upper, const float* T, int ldt, V* x, hipStream_t stream)
+hipError_t TrsvChain(TrsvChainState& s, bool upper, const float* T, int ldt, double* x, hipStream_t stream)
 {
     const int n = s.n;
     if (n <= 0) return hipSuccess;
@@ -309,7 +286,7 @@ hipError_t LaunchChain(TrsvChainState& s, bool upper, const float* T, int ldt, V
     const unsigned base = static_cast<unsigned>(s.launches) * static_cast<unsigned>(nblk);
     const unsigned spinLimit = SpinLimit();
 #define CHAIN(NB, UP)                                                                                             \
-    hipLaunchKernelGGL((trsv_chain_kernel<NB, UP, V>), dim3(nblk), dim3(256), 0, stream, n, T, ldt, x, s.pub, s.ticket, \
+    hipLaunchKernelGGL((trsv_chain_kernel<NB, UP>), dim3(nblk), dim3(256), 0, stream, n, T, ldt, x, s.pub, s.ticket, \
                        base, epoch, s.err, spinLimit)
     if (nb == 128)
     {
@@ -328,16 +305,6 @@ hipError_t LaunchChain(TrsvChainState& s, bool upper, const float* T, int ldt, V
 #undef CHAIN
     ++s.launches;
     return hipGetLastError();
-}
-
-hipError_t TrsvChain(TrsvChainState& s, bool upper, const float* T, int ldt, float* x, hipStream_t stream)
-{
-    return LaunchChain<float>(s, upper, T, ldt, x, stream);
-}
-
-hipError_t TrsvChain(TrsvChainState& s, bool upper, const float* T, int ldt, double* x, hipStream_t stream)
-{
-    return LaunchChain<double>(s, upper, T, ldt, x, stream);
 }
 
 }  // namespace ops
