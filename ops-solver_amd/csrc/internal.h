@@ -113,8 +113,10 @@ aclsolverStatus_t Launched();
 // Synchronizes the stream (reference src/utils/real_lu_common.h:90-132).
 bool AllFinite(aclsolverHandle_t h, const float* a, int rows, int cols, int lda, int64_t batchStride, int batch,
                bool* ok);
-bool AllFiniteArrays(aclsolverHandle_t h, const float* const* arrays, int rows, int cols, int lda, int batch,
-                     bool* ok);
+// piv (optional, rows * batch ints): also checks that pivot k of every matrix lies in k + 1 ..
+// rows (*pivOk).
+bool AllFiniteArrays(aclsolverHandle_t h, const float* const* arrays, int rows, int cols, int lda, int batch, bool* ok,
+                     const int* piv = nullptr, bool* pivOk = nullptr);
 
 // ---- optional launch timing (profile.hip) ----
 enum class ProfileKernel

@@ -175,6 +175,15 @@ __global__ __launch_bounds__(256) void finite_arrays_small_kernel(const float* c
     if (__any(bad) && (threadIdx.x % warpSize) == 0) atomicOr(flag, 1);
 }
 
+// flag |= 2 when a pivot of the batch lies outside k + 1 .. n.
+__global__ __launch_bounds__(256) void pivot_range_kernel(const int* piv, int n, size_t total, int* flag)
+{
+    int bad = 0;
+    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < total; i += static_cast<size_t>(gridDim.x) * 256)
+        bad |= piv[i] < static_cast<int>(i % n) + 1 || piv[i] > n;
+    if (__any(bad) && (threadIdx.x % warpSize) == 0) atomicOr(flag, 2);
+}
+
 static bool ReadFlag(int* dflag, int* hflag, hipStream_t stream, bool* ok)
 {
     *hflag = 0;
@@ -199,8 +208,8 @@ bool AllFinite(aclsolverHandle_t h, const float* a, int rows, int cols, int lda,
     return ReadFlag(dflag, H(h)->hflag, stream, ok);
 }
 
-bool AllFiniteArrays(aclsolverHandle_t h, const float* const* arrays, int rows, int cols, int lda, int batch,
-                     bool* ok)
+bool AllFiniteArrays(aclsolverHandle_t h, const float* const* arrays, int rows, int cols, int lda, int batch, bool* ok,
+                     const int* piv, bool* pivOk)
 {
     *ok = true;
     if (rows <= 0 || cols <= 0 || batch <= 0) return true;
@@ -212,12 +221,21 @@ bool AllFiniteArrays(aclsolverHandle_t h, const float* const* arrays, int rows, 
         const int blocks = std::min((batch + 3) / 4, 65536);
         hipLaunchKernelGGL(finite_arrays_small_kernel, dim3(blocks), dim3(256), 0, stream, arrays, rows * cols, batch,
                            dflag);
-        return ReadFlag(dflag, H(h)->hflag, stream, ok);
     }
-    int per = (rows * cols + 255) / 256;
-    dim3 grid(std::min(per, 64), std::min(batch, 4096));
-    hipLaunchKernelGGL(finite_arrays_kernel, grid, dim3(256), 0, stream, arrays, rows, cols, lda, batch, dflag);
-    return ReadFlag(dflag, H(h)->hflag, stream, ok);
+    else
+    {
+        int per = (rows * cols + 255) / 256;
+        dim3 grid(std::min(per, 64), std::min(batch, 4096));
+        hipLaunchKernelGGL(finite_arrays_kernel, grid, dim3(256), 0, stream, arrays, rows, cols, lda, batch, dflag);
+    }
+    const size_t pivots = piv != nullptr ? static_cast<size_t>(rows) * batch : 0;
+    if (pivots > 0)
+        hipLaunchKernelGGL(pivot_range_kernel, dim3(static_cast<unsigned>(std::min<size_t>((pivots + 1023) / 1024, 4096))),
+                           dim3(256), 0, stream, piv, rows, pivots, dflag);
+    if (!ReadFlag(dflag, H(h)->hflag, stream, ok)) return false;
+    *ok = (*H(h)->hflag & 1) == 0;
+    if (pivOk != nullptr) *pivOk = (*H(h)->hflag & 2) == 0;
+    return true;
 }
 
 }  // namespace ops

@@ -20,6 +20,7 @@
 #include <climits>
 
 #include "internal.h"
+#include "permute.h"
 #include "trtri64.h"
 
 namespace ops
@@ -109,12 +110,8 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
     b -= 2 * nb;
     if (b < np)
     {
-        // perm[i] = source row of row i of P B: position i traced backward through the
-        // interchanges. LAPACK pivots never point above their own row, so position i is first
-        // met by interchange i, and from there on only "x == pivot" can move it; any entry that
-        // does point above takes the general trace.
         int* const s_piv = reinterpret_cast<int*>(s_mem);
-        const int i = b * 256 + tid, last = min(p.n, b * 256 + 256);
+        const int i = b * 256 + tid;
         bool plain = true;
         for (int k = tid; k < p.n; k += 256)
         {
@@ -124,29 +121,7 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
             s_piv[k] = v;
         }
         plain = __syncthreads_and(plain);
-        int x = i;
-        if (plain)
-        {
-            const int base = b * 256 + wave * 64;  // this wave's first position
-            if (i < p.n) x = s_piv[i];
-            for (int k = min(last, base + 64) - 1; k >= base && k >= 0; --k) x = k < i && s_piv[k] == x ? k : x;
-            int k = base - 1;
-#pragma unroll 1
-            for (; k >= 3; k -= 4)
-            {
-                const int4 v = *reinterpret_cast<const int4*>(s_piv + k - 3);  // k + 1 is a multiple of 64
-                x = v.w == x ? k : x;
-                x = v.z == x ? k - 1 : x;
-                x = v.y == x ? k - 2 : x;
-                x = v.x == x ? k - 3 : x;
-            }
-        }
-        else
-            for (int k = p.n - 1; k >= 0; --k)
-            {
-                const int v = s_piv[k];
-                x = x == k ? v : (x == v ? k : x);
-            }
+        const int x = TracePosition(s_piv, p.n, i, b * 256 + wave * 64, plain);
         if (i < p.n) p.perm[i] = x;
         return;
     }
