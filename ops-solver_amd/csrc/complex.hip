@@ -18,10 +18,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cfloat>
 #include <climits>
 #include <cstdint>
 
+#include "cleaf.h"
+#include "complex_math.h"
 #include "internal.h"
 
 namespace ops
@@ -29,510 +30,6 @@ namespace ops
 namespace
 {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ inline uint32_t PivotScore(float2 v)
-{
-    const float r = fabsf(v.x), i = fabsf(v.y);
-    float s = r + i;
-    if (!(s >= 0.0f)) return 0u;
-    if (s == 0.0f) return 1u;
-    if (s > FLT_MAX)
-    {
-        s = r * 0.5f + i * 0.5f;
-        return __float_as_uint(s) + 0x00800001u;
-    }
-    return __float_as_uint(s) + 1u;
-}
-
-__device__ inline float2 SubMul(float2 x, float2 a, float2 b)
-{
-    return make_float2(fmaf(a.y, b.y, fmaf(-a.x, b.x, x.x)), fmaf(-a.y, b.x, fmaf(-a.x, b.y, x.y)));
-}
-
-// 1/d in FP64 (exact enough that a * (1/d) rounds within one ulp of a / d).
-__device__ inline double2 Recip64(float2 d)
-{
-    const double dr = d.x, di = d.y;
-    const double den = dr * dr + di * di;
-    return make_double2(dr / den, -di / den);
-}
-
-__device__ inline float2 Mul64(float2 a, double2 r)
-{
-    const double ar = a.x, ai = a.y;
-    return make_float2(static_cast<float>(ar * r.x - ai * r.y), static_cast<float>(ar * r.y + ai * r.x));
-}
-
-__device__ inline float2 Conj(float2 v, bool c) { return c ? make_float2(v.x, -v.y) : v; }
-
-// ---------------------------------------------------------------------------------------
-// Leaf (see getrf.hip for the real counterpart): W complex columns, R rows per thread.
-// ---------------------------------------------------------------------------------------
-template <int T, int R, int W>
-__global__ __launch_bounds__(T) void cleaf_kernel(float2* __restrict__ A, int lda, int m, int j0, int c0, int wact,
-                                                  int pivoting, int newPanel, int* __restrict__ ipiv,
-                                                  int* __restrict__ info, int* __restrict__ rowsrc,
-                                                  int* __restrict__ leafmap)
-{
-    constexpr int NW = T / 64;
-    __shared__ float2 s_prow[W];
-    __shared__ uint32_t s_best[NW];
-    __shared__ int s_bpos[NW];
-    __shared__ int s_count;
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int mp = m - c0;
-    float2* Ap = A + static_cast<size_t>(c0) * lda + c0;
-    float2 a[R][W];
-    int pos[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        const bool valid = lr < mp;
-#pragma unroll
-        for (int j = 0; j < W; ++j)
-            a[i][j] = (valid && j < wact) ? Ap[static_cast<size_t>(j) * lda + lr] : make_float2(0.0f, 0.0f);
-        pos[i] = valid ? lr : INT_MAX;
-    }
-    if (tid == 0) s_count = 0;
-    int zeroCol = 0;
-#pragma unroll
-    for (int j = 0; j < W; ++j)
-    {
-        if (j < wact)
-        {
-            int bpos = j;
-            if (pivoting)
-            {
-                uint32_t best = 0;
-                int bp = INT_MAX;
-#pragma unroll
-                for (int i = 0; i < R; ++i)
-                    if (pos[i] >= j && pos[i] != INT_MAX)
-                    {
-                        const uint32_t s = PivotScore(a[i][j]);
-                        if (s > best || (s == best && pos[i] < bp))
-                        {
-                            best = s;
-                            bp = pos[i];
-                        }
-                    }
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1)
-                {
-                    const uint32_t ob = __shfl_xor(best, off);
-                    const int op = __shfl_xor(bp, off);
-                    if (ob > best || (ob == best && op < bp))
-                    {
-                        best = ob;
-                        bp = op;
-                    }
-                }
-                if (lane == 0)
-                {
-                    s_best[wid] = best;
-                    s_bpos[wid] = bp;
-                }
-                __syncthreads();
-                best = s_best[0];
-                bp = s_bpos[0];
-#pragma unroll
-                for (int w = 1; w < NW; ++w)
-                {
-                    const uint32_t ob = s_best[w];
-                    const int op = s_bpos[w];
-                    if (ob > best || (ob == best && op < bp))
-                    {
-                        best = ob;
-                        bp = op;
-                    }
-                }
-                bpos = bp == INT_MAX ? j : bp;
-            }
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-                if (pos[i] == bpos)
-                {
-#pragma unroll
-                    for (int k = 0; k < W; ++k) s_prow[k] = a[i][k];
-                }
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                if (pos[i] == bpos)
-                    pos[i] = j;
-                else if (pos[i] == j)
-                    pos[i] = bpos;
-            }
-            if (tid == 0 && ipiv != nullptr) ipiv[c0 + j] = c0 + bpos + 1;
-            __syncthreads();
-            const float2 d = s_prow[j];
-            const bool zero = d.x == 0.0f && d.y == 0.0f;
-            if (zero && zeroCol == 0) zeroCol = c0 + j + 1;
-            const double2 rinv = Recip64(zero ? make_float2(1.0f, 0.0f) : d);
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                const bool below = pos[i] > j && pos[i] != INT_MAX && !zero;
-                const float2 q = Mul64(a[i][j], rinv);
-                const float2 l = below ? q : make_float2(0.0f, 0.0f);
-                a[i][j] = below ? q : a[i][j];
-#pragma unroll
-                for (int k = 1; k < W; ++k)  // constant bounds: unrolled with the j loop
-                    if (k > j) a[i][k] = SubMul(a[i][k], l, s_prow[k]);
-            }
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        if (lr < mp)
-        {
-            const int dst = pos[i];
-#pragma unroll
-            for (int j = 0; j < W; ++j)
-                if (j < wact) Ap[static_cast<size_t>(j) * lda + dst] = a[i][j];
-            if (dst != lr)
-            {
-                const int slot = atomicAdd(&s_count, 1);
-                leafmap[1 + 2 * slot] = c0 + dst;
-                leafmap[2 + 2 * slot] = c0 + lr;
-            }
-        }
-    }
-    int srcv[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        srcv[i] = (lr < mp) ? (newPanel ? c0 + lr : rowsrc[c0 + lr]) : 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = tid + i * T;
-        if (lr < mp) rowsrc[c0 + pos[i]] = srcv[i];
-    }
-    if (tid == 0)
-    {
-        leafmap[0] = s_count;
-        if (zeroCol != 0 && *info == 0) *info = zeroCol;
-    }
-}
-
-__global__ __launch_bounds__(128) void cpanel_swap_trsm_kernel(float2* __restrict__ A, int lda, int j0, int c0,
-                                                               int wact, const int* __restrict__ leafmap)
-{
-    __shared__ float2 s_x[64];
-    const int left = c0 - j0;
-    const int idx = blockIdx.x;
-    const int c = idx < left ? j0 + idx : c0 + wact + (idx - left);
-    float2* col = A + static_cast<size_t>(c) * lda;
-    const int cnt = leafmap[0];
-    const int t = threadIdx.x;
-    float2 v = make_float2(0.0f, 0.0f);
-    int dst = -1;
-    if (t < cnt)
-    {
-        dst = leafmap[1 + 2 * t];
-        v = col[leafmap[2 + 2 * t]];
-    }
-    __syncthreads();
-    if (dst >= 0) col[dst] = v;
-    __syncthreads();
-    if (c < c0) return;
-    if (t < wact) s_x[t] = col[c0 + t];
-    __syncthreads();
-    const float2* L = A + static_cast<size_t>(c0) * lda + c0;
-    for (int s = 0; s < wact - 1; ++s)
-    {
-        if (t > s && t < wact) s_x[t] = SubMul(s_x[t], L[static_cast<size_t>(s) * lda + t], s_x[s]);
-        __syncthreads();
-    }
-    if (t < wact) col[c0 + t] = s_x[t];
-}
-
-// ---------------------------------------------------------------------------------------
-// Tall complex leaf over several one-wave workgroups (the design of leaf_multi_kernel in
-// getrf.hip): rows [c0, m) split over P = gridDim.x workgroups of 64*R rows; per column each
-// wave reduces its candidates to one 64-bit key (pivot score, then the lowest position),
-// publishes its candidate's row (two tagged 64-bit words per complex value: real, imag) and
-// the key, polls the P keys, fetches the winning row and eliminates with the FP64
-// reciprocal and SubMul order of cleaf_kernel. The interchanges are written to leafmap for
-// cpanel_swap_trsm_kernel, exactly as cleaf_kernel does. Spins are bounded; on a timeout the
-// workgroup raises *err and fills its rows with NaN.
-// ---------------------------------------------------------------------------------------
-// Slots, per column parity: the workgroups' keys (one word each: 16-bit tag, 32-bit pivot
-// score, 16-bit position rank; contiguous, so one poll of all keys touches few cache lines),
-// then their candidate rows (kCRowWords words each: 32-bit tag, 32-bit value).
-constexpr int kCRowWords = 64;  // 2 words per complex column (W <= 32)
-constexpr int kCMaxGroups = 128;
-constexpr int kCKeyWords = 2 * kCMaxGroups;  // both parities
-constexpr size_t kCSlotBytes =
-    (static_cast<size_t>(kCKeyWords) + 2ull * kCMaxGroups * kCRowWords) * sizeof(unsigned long long);
-
-template <int CTRL>
-__device__ inline unsigned CDppU32(unsigned v)
-{
-    return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, false));
-}
-__device__ inline unsigned CWaveMaxU32(unsigned v)
-{
-    auto mx = [](unsigned a, unsigned b) { return a > b ? a : b; };
-    v = mx(v, CDppU32<0xB1>(v));   // quad_perm [1,0,3,2]
-    v = mx(v, CDppU32<0x4E>(v));   // quad_perm [2,3,0,1]
-    v = mx(v, CDppU32<0x124>(v));  // row_ror:4
-    v = mx(v, CDppU32<0x128>(v));  // row_ror:8
-    const unsigned r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
-    const unsigned r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
-    return mx(mx(r0, r1), mx(r2, r3));
-}
-// Wave-wide maximum of a 64-bit key, reduced word by word: the high words first (one 32-bit
-// DPP max per step), then, only when several lanes hold that high word, their low words
-// (the keys hold a pivot score in the high word and a position in the low one, so the
-// second pass runs only on exact score ties).
-__device__ inline unsigned long long CWaveMax64(unsigned long long v)
-{
-    const unsigned hi = static_cast<unsigned>(v >> 32), lo = static_cast<unsigned>(v);
-    const unsigned mh = CWaveMaxU32(hi);
-    const unsigned long long tie = __ballot(hi == mh);
-    unsigned ml;
-    if (__popcll(tie) == 1)  // uniform
-        ml = __builtin_amdgcn_readlane(lo, __builtin_ctzll(tie));
-    else
-        ml = CWaveMaxU32(hi == mh ? lo : 0u);
-    return (static_cast<unsigned long long>(mh) << 32) | ml;
-}
-__device__ inline unsigned long long CLoadSlot(const unsigned long long* p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <bool LOCAL = false>
-__device__ inline void CStoreSlot(unsigned long long* p, unsigned tag, unsigned payload)
-{
-    __hip_atomic_store(p, (static_cast<unsigned long long>(tag) << 32) | payload, __ATOMIC_RELAXED,
-                       LOCAL ? __HIP_MEMORY_SCOPE_WORKGROUP : __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// FULL: wact == W (no column of the unrolled loop is skipped at run time). SPREAD: 8
-// workgroups per participant, only ids = 0 mod 8 take part, all on one XCD, and the exchange
-// words are stored at workgroup scope into its L2 (as leaf_multi_kernel's SPREAD).
-template <int R, int W, bool FULL, bool SPREAD = false>
-__global__ __launch_bounds__(64) void cleaf_multi_kernel(float2* __restrict__ A, int lda, int m, int c0, int wact,
-                                                         int pivoting, int newPanel, int* __restrict__ ipiv,
-                                                         int* __restrict__ info, int* __restrict__ rowsrc,
-                                                         int* __restrict__ leafmap, unsigned long long* slots,
-                                                         unsigned tagBase, int* err, unsigned spinLimit)
-{
-    constexpr int T = 64;
-    static_assert(2 * W <= kCRowWords && 2 * W <= T, "slot layout");
-    __shared__ float s_row[2 * W];   // this wave's candidate row (re, im interleaved)
-    __shared__ float s_prow[2 * W];  // the pivot row
-    __shared__ int s_bpos[W];
-    __shared__ int s_count;
-    const int lane = threadIdx.x;
-    if (SPREAD && (blockIdx.x & 7) != 0) return;  // not a participant
-    const int P = SPREAD ? static_cast<int>(gridDim.x >> 3) : static_cast<int>(gridDim.x);
-    const int g = SPREAD ? static_cast<int>(blockIdx.x >> 3) : static_cast<int>(blockIdx.x);
-    const int mp = m - c0;
-    float2* Ap = A + static_cast<size_t>(c0) * lda + c0;
-    const int rbase = g * T * R;
-    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-
-    float2 a[R][W];
-    int pos[R], srcv[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = rbase + lane + i * T;
-        const bool valid = lr < mp;
-#pragma unroll
-        for (int j = 0; j < W; ++j)
-            a[i][j] = (valid && j < wact) ? Ap[static_cast<size_t>(j) * lda + lr] : make_float2(0.0f, 0.0f);
-        pos[i] = valid ? lr : INT_MAX;
-        // read before any workgroup stores (stores follow the last column's exchange)
-        srcv[i] = valid ? (newPanel ? c0 + lr : rowsrc[c0 + lr]) : 0;
-    }
-    if (lane == 0) s_count = 0;
-    int zeroCol = 0;
-    bool aborted = false;
-
-#pragma unroll
-    for (int j = 0; j < W; ++j)
-    {
-        if (FULL || j < wact)  // uniform (one wave)
-        {
-            const unsigned tag = tagBase + static_cast<unsigned>(j);
-            unsigned long long* keys = slots + (j & 1) * kCMaxGroups;
-            unsigned long long* rows = slots + kCKeyWords + static_cast<size_t>(j & 1) * kCMaxGroups * kCRowWords;
-            // After a timeout the remaining columns run without waiting (no exchange, no
-            // interchange): the column loop stays one straight unrolled sequence, and the
-            // factors end as NaN.
-            const unsigned lim = aborted ? 0u : spinLimit;
-            unsigned long long best = 0ull;
-            int bi = -1;
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                // (score << 32) | (0xffff - position): positions are below 16384, so a
-                // candidate's key is never 0, even with score 0 (NaN)
-                const bool cand = pos[i] != INT_MAX && (pivoting ? pos[i] >= j : pos[i] == j);
-                const unsigned long long k =
-                    cand ? (static_cast<unsigned long long>(PivotScore(a[i][j])) << 32) |
-                               static_cast<unsigned>(0xffff - pos[i])
-                         : 0ull;
-                bi = k > best ? i : bi;
-                best = k > best ? k : best;
-            }
-            const unsigned long long top = CWaveMax64(best);
-            if (best == top && bi >= 0)
-#pragma unroll
-                for (int i = 0; i < R; ++i)
-                    if (i == bi)
-#pragma unroll
-                        for (int k = 0; k < W; ++k)
-                        {
-                            s_row[2 * k] = a[i][k].x;
-                            s_row[2 * k + 1] = a[i][k].y;
-                        }
-            __syncthreads();
-            if (lane < 2 * wact)
-                CStoreSlot<SPREAD>(rows + g * kCRowWords + lane, tag,
-                                   __float_as_uint(s_row[lane < 2 * W ? lane : 0]));
-            if (lane == 0)
-                __hip_atomic_store(keys + g,
-                                   (static_cast<unsigned long long>(tag & 0xffffu) << 48) | ((top >> 32) << 16) |
-                                       (top & 0xffffull),
-                                   __ATOMIC_RELAXED, SPREAD ? __HIP_MEMORY_SCOPE_WORKGROUP : __HIP_MEMORY_SCOPE_AGENT);
-            // the P keys: lane l reads workgroups l and l + 64
-            unsigned long long key0 = 0ull, key1 = 0ull;
-            bool ok = false;
-            const unsigned long long t16 = tag & 0xffffu;
-            for (unsigned spins = 0; spins < lim; ++spins)
-            {
-                const unsigned long long w0 = lane < P ? CLoadSlot(keys + lane) : t16 << 48;
-                const unsigned long long w1 = lane + 64 < P ? CLoadSlot(keys + lane + 64) : t16 << 48;
-                key0 = (((w0 >> 16) & 0xffffffffull) << 32) | (w0 & 0xffffull);
-                key1 = (((w1 >> 16) & 0xffffffffull) << 32) | (w1 & 0xffffull);
-                if (__all((w0 >> 48) == t16 && (w1 >> 48) == t16))
-                {
-                    ok = true;
-                    break;
-                }
-            }
-            const unsigned long long gtop = CWaveMax64(key0 > key1 ? key0 : key1);
-            const unsigned long long hit0 = __ballot(ok && lane < P && key0 == gtop);
-            const unsigned long long hit1 = __ballot(ok && lane + 64 < P && key1 == gtop);
-            const int winner = hit0 != 0ull   ? __ffsll(static_cast<long long>(hit0)) - 1
-                               : hit1 != 0ull ? 64 + __ffsll(static_cast<long long>(hit1)) - 1
-                                              : 0;
-            unsigned long long rw = 0ull;
-            for (unsigned spins = 0; ok; ++spins)
-            {
-                rw = lane < 2 * wact ? CLoadSlot(rows + winner * kCRowWords + lane)
-                                     : static_cast<unsigned long long>(tag) << 32;
-                if (__all(static_cast<unsigned>(rw >> 32) == tag)) break;
-                if (spins >= spinLimit) ok = false;
-            }
-            if (!ok)
-            {
-                if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                aborted = true;
-            }
-            if (lane < 2 * W) s_prow[lane] = __uint_as_float(static_cast<unsigned>(rw));
-            __syncthreads();
-            const int bpos = aborted || gtop == 0ull ? j : 0xffff - static_cast<int>(gtop & 0xffffull);
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                if (pos[i] == bpos)
-                    pos[i] = j;
-                else if (pos[i] == j)
-                    pos[i] = bpos;
-            }
-            if (lane == 0)
-            {
-                s_bpos[j] = bpos;
-                if (g == 0 && ipiv != nullptr) ipiv[c0 + j] = c0 + bpos + 1;
-            }
-            const float2 d = make_float2(s_prow[2 * j], s_prow[2 * j + 1]);
-            const bool zero = d.x == 0.0f && d.y == 0.0f;
-            if (zero && zeroCol == 0 && !aborted) zeroCol = c0 + j + 1;
-            const double2 rinv = Recip64(zero ? make_float2(1.0f, 0.0f) : d);
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-            {
-                const bool below = pos[i] > j && pos[i] != INT_MAX && !zero;
-                const float2 q = Mul64(a[i][j], rinv);
-                const float2 l = below ? q : make_float2(0.0f, 0.0f);
-                a[i][j] = below ? q : a[i][j];
-#pragma unroll
-                for (int k = 1; k < W; ++k)  // constant bounds: unrolled with the j loop
-                    if (k > j) a[i][k] = SubMul(a[i][k], l, make_float2(s_prow[2 * k], s_prow[2 * k + 1]));
-            }
-        }
-    }
-    if (aborted)
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-#pragma unroll
-            for (int j = 0; j < W; ++j) a[i][j] = make_float2(__builtin_nanf(""), __builtin_nanf(""));
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-    {
-        const int lr = rbase + lane + i * T;
-        if (lr < mp)
-        {
-            const int dst = pos[i];
-#pragma unroll
-            for (int j = 0; j < W; ++j)
-                if (j < wact) Ap[static_cast<size_t>(j) * lda + dst] = a[i][j];
-            rowsrc[c0 + dst] = srcv[i];
-        }
-    }
-    if (g != 0) return;
-    if (lane == 0 && zeroCol != 0 && *info == 0) *info = zeroCol;
-    if (aborted)
-    {
-        if (lane == 0) leafmap[0] = 0;
-        return;
-    }
-    __syncthreads();
-    // workgroup 0 lists the moved rows for cpanel_swap_trsm_kernel (undoing the interchange
-    // sequence from each touched position, as leaf_multi_kernel does)
-    {
-        int p = -1;
-        if (lane < W)
-            p = lane < wact ? lane : -1;
-        else if (lane - W < wact)
-        {
-            const int jj = lane - W;
-            p = s_bpos[jj] >= wact ? s_bpos[jj] : -1;
-            for (int t = 0; t < jj && p >= 0; ++t)
-                if (s_bpos[t] == p) p = -1;
-        }
-        if (p >= 0)
-        {
-            int x = p;
-            for (int jj = wact - 1; jj >= 0; --jj)
-            {
-                const int b = s_bpos[jj];
-                x = x == jj ? b : (x == b ? jj : x);
-            }
-            if (x != p)
-            {
-                const int slot = atomicAdd(&s_count, 1);
-                leafmap[1 + 2 * slot] = c0 + p;
-                leafmap[2 + 2 * slot] = c0 + x;
-            }
-        }
-    }
-    __syncthreads();
-    if (lane == 0) leafmap[0] = s_count;
-}
 
 __global__ void cclear_slots_kernel(unsigned long long* slots, int words, int* err)
 {
@@ -561,7 +58,7 @@ __global__ __launch_bounds__(1024) void ccompact_moves_kernel(int m, int j0, con
     if (threadIdx.x == 0) moved[0] = s_count;
 }
 
-constexpr int CNB = 128;  // complex outer block
+constexpr int CNB = 512;  // complex outer block
 
 // Applies a panel's moved-row list to the columns [lo1, hi1) and [lo2, hi2): one wave64 per
 // column gathers every source row, then scatters.
@@ -594,92 +91,128 @@ __global__ __launch_bounds__(256) void couter_swap_kernel(float2* __restrict__ A
         if (d[q] >= 0) col[d[q]] = v[q];
 }
 
-// C (MxN) -= op(A) (MxK) * B (KxN), complex64, 4 real MFMA products per block.
-// op(A): transA 0 = A, 1 = A^T, 2 = A^H. Tile 64x64 per workgroup, one 32x32 block per wave.
-template <int TRANSA>
-__global__ __launch_bounds__(256) void cgemm_sub_kernel(int M, int N, int K, const float2* __restrict__ A, int lda,
-                                                        const float2* __restrict__ B, int ldb, float2* __restrict__ C,
-                                                        int ldc, int tilesM)
+// C (MxN) -= op(A) (MxK) * B (KxN), complex64, four real FP32 MFMA products per block; op(A):
+// transA 0 = A, 1 = A^T, 2 = A^H. Tiles of 64 Q x 64 Q per workgroup, 32 Q x 32 Q per wave, k
+// chunks of 16 staged through LDS (parts apart) with the next chunk prefetched into registers;
+// formed as C^T, so that an accumulator register holds 32 consecutive rows of C.
+template <int TRANSA, int Q>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void cgemm_sub_kernel(
+    int M, int N, int K, const float2* __restrict__ A, int64_t lda, const float2* __restrict__ B, int64_t ldb,
+    float2* __restrict__ C, int64_t ldc, int tilesM, int tilesN)
 {
-    __shared__ float Ar[16][64 + 4], Ai[16][64 + 4], Br[16][64 + 4], Bi[16][64 + 4];
-    const int tm = blockIdx.x % tilesM, tn = blockIdx.x / tilesM;
-    const int row0 = tm * 64, col0 = tn * 64;
+    constexpr int KC = 16, TS = 64 * Q, E = 4 * Q;
+    __shared__ float Ar[2][KC][TS + 4], Ai[2][KC][TS + 4], Br[2][KC][TS + 4], Bi[2][KC][TS + 4];
+    int id = blockIdx.x;
+    const int total = tilesM * tilesN;
+    // Workgroups go round the XCDs: each XCD gets a run of tiles, so that neighbours share L2.
+    if (total >= 64) id = id < (total & ~7) ? (id & 7) * (total >> 3) + (id >> 3) : id;
+    const int row0 = id % tilesM * TS, col0 = id / tilesM * TS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    f32x16 accR, accI;
+    const int wm = (wave & 1) * 32 * Q + (lane & 31), wn = (wave >> 1) * 32 * Q + (lane & 31), lk = lane >> 5;
+    f32x16 accR[Q][Q], accI[Q][Q];
 #pragma unroll
-    for (int v = 0; v < 16; ++v)
+    for (int i = 0; i < Q; ++i)
+#pragma unroll
+        for (int j = 0; j < Q; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) accR[i][j][v] = accI[i][j][v] = 0.0f;
+    // Rows and columns beyond the edge repeat the last one: their products are not stored. Sixteen
+    // lanes read the 128 bytes of a chunk of one column of B (of one row of op(A) when
+    // transposed), so that a line is fetched by one load, not by eight.
+    const int ar = TRANSA ? tid >> 4 : tid % TS, ak = TRANSA ? tid & 15 : tid / TS * E;
+    const int bj = tid >> 4, bk = tid & 15;
+    const float2* const Arow = A + static_cast<int64_t>(min(row0 + ar, M - 1)) * (TRANSA ? lda : 1);
+    const float2* const Bcol = B + static_cast<int64_t>(min(col0 + bj, N - 1)) * ldb;
+    float2 ra[E], rb[E];
+    auto gload = [&](int k0)
     {
-        accR[v] = 0.0f;
-        accI[v] = 0.0f;
-    }
-    for (int k0 = 0; k0 < K; k0 += 16)
+        const int kb = k0 + bk;
+        const float2* pa = Arow + (TRANSA ? min(kb, K - 1) : 0);
+        const float2* pb = Bcol + min(kb, K - 1);
+#pragma unroll
+        for (int q = 0; q < E; ++q)
+        {
+            const int ka = TRANSA ? kb : k0 + ak + q;
+            ra[q] = TRANSA ? *pa : pa[static_cast<int64_t>(min(ka, K - 1)) * lda];
+            rb[q] = *pb;
+            if (ka >= K) ra[q] = make_float2(0.0f, 0.0f);
+            if (kb >= K) rb[q] = make_float2(0.0f, 0.0f);
+            if (TRANSA) pa += row0 + ar + 16 * (q + 1) < M ? 16 * lda : 0;
+            pb += col0 + bj + 16 * (q + 1) < N ? 16 * ldb : 0;
+        }
+    };
+    auto lstore = [&](int buf)
     {
-        // A tile: 64 rows x 16 k
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < E; ++q)
         {
-            const int e = tid + q * 256;  // 1024 elements
-            int r, k;
-            if (TRANSA == 0)
-            {
-                r = e & 63;
-                k = e >> 6;
-            }
-            else
-            {
-                k = e & 15;
-                r = e >> 4;
-            }
-            float2 v = make_float2(0.0f, 0.0f);
-            if (row0 + r < M && k0 + k < K)
-            {
-                v = TRANSA == 0 ? A[static_cast<size_t>(k0 + k) * lda + row0 + r]
-                                : A[static_cast<size_t>(row0 + r) * lda + k0 + k];
-                if (TRANSA == 2) v.y = -v.y;
-            }
-            Ar[k][r] = v.x;
-            Ai[k][r] = v.y;
+            const int k = TRANSA ? ak : ak + q, r = TRANSA ? ar + 16 * q : ar;
+            Ar[buf][k][r] = ra[q].x;
+            Ai[buf][k][r] = TRANSA == 2 ? -ra[q].y : ra[q].y;
+            Br[buf][bk][bj + 16 * q] = rb[q].x;
+            Bi[buf][bk][bj + 16 * q] = rb[q].y;
         }
+    };
+    const int chunks = (K + KC - 1) / KC;
+    gload(0);
+    lstore(0);
+    __syncthreads();
+    for (int c = 0; c < chunks; ++c)
+    {
+        const int buf = c & 1;
+        if (c + 1 < chunks) gload((c + 1) * KC);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int kk = 0; kk < KC; kk += 2)
         {
-            const int e = tid + q * 256;
-            const int k = e & 15, j = e >> 4;
-            float2 v = make_float2(0.0f, 0.0f);
-            if (col0 + j < N && k0 + k < K) v = B[static_cast<size_t>(col0 + j) * ldb + k0 + k];
-            Br[k][j] = v.x;
-            Bi[k][j] = v.y;
+            float xr[Q], xi[Q], yr[Q], yi[Q];
+#pragma unroll
+            for (int i = 0; i < Q; ++i)
+            {
+                xr[i] = Ar[buf][kk + lk][wm + 32 * i];
+                xi[i] = Ai[buf][kk + lk][wm + 32 * i];
+                yr[i] = Br[buf][kk + lk][wn + 32 * i];
+                yi[i] = Bi[buf][kk + lk][wn + 32 * i];
+            }
+#pragma unroll
+            for (int i = 0; i < Q; ++i)
+#pragma unroll
+                for (int j = 0; j < Q; ++j)
+                {
+                    accR[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(yr[j], xr[i], accR[i][j], 0, 0, 0);
+                    accI[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(yi[j], xr[i], accI[i][j], 0, 0, 0);
+                }
+#pragma unroll
+            for (int i = 0; i < Q; ++i)
+#pragma unroll
+                for (int j = 0; j < Q; ++j)
+                {
+                    accR[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(-yi[j], xi[i], accR[i][j], 0, 0, 0);
+                    accI[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(yr[j], xi[i], accI[i][j], 0, 0, 0);
+                }
         }
+        if (c + 1 < chunks) lstore(buf ^ 1);
         __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 16; kk += 2)
-        {
-            const int k = kk + (lane >> 5);
-            const float ar = Ar[k][wm * 32 + (lane & 31)], ai = Ai[k][wm * 32 + (lane & 31)];
-            const float br = Br[k][wn * 32 + (lane & 31)], bi = Bi[k][wn * 32 + (lane & 31)];
-            accR = __builtin_amdgcn_mfma_f32_32x32x2f32(ar, br, accR, 0, 0, 0);
-            accR = __builtin_amdgcn_mfma_f32_32x32x2f32(-ai, bi, accR, 0, 0, 0);
-            accI = __builtin_amdgcn_mfma_f32_32x32x2f32(ar, bi, accI, 0, 0, 0);
-            accI = __builtin_amdgcn_mfma_f32_32x32x2f32(ai, br, accI, 0, 0, 0);
-        }
-        __syncthreads();
     }
-    const int j = col0 + wn * 32 + (lane & 31);
-    if (j >= N) return;
-    float2* cj = C + static_cast<size_t>(j) * ldc;
+    // All loads of a 32 x 32 tile before its first store (a load under its own condition waits by
+    // itself: 128 trips in a row took longer than the product of 512 columns).
 #pragma unroll
-    for (int v = 0; v < 16; ++v)
-    {
-        const int i = row0 + wm * 32 + (v & 3) + 8 * (v >> 2) + 4 * (lane >> 5);
-        if (i < M)
+    for (int bi = 0; bi < Q; ++bi)
+#pragma unroll
+        for (int bc = 0; bc < Q; ++bc)
         {
-            float2 c = cj[i];
-            c.x -= accR[v];
-            c.y -= accI[v];
-            cj[i] = c;
+            const int i = row0 + wm + 32 * bi, j0 = col0 + (wave >> 1) * 32 * Q + bc * 32 + 4 * lk;
+            float2 x[16];
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                x[v] = C[static_cast<int64_t>(min(j0 + (v & 3) + 8 * (v >> 2), N - 1)) * ldc + min(i, M - 1)];
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+            {
+                const int j = j0 + (v & 3) + 8 * (v >> 2);
+                if (i < M && j < N)
+                    C[j * ldc + i] = make_float2(x[v].x - accR[bi][bc][v], x[v].y - accI[bi][bc][v]);
+            }
         }
-    }
 }
 
 template <int CTRL>
@@ -749,19 +282,32 @@ __global__ __launch_bounds__(256) void ctrsm_diag64_kernel(int kb, int N, const 
         if (live && 16 * q + t < kb) b[16 * q + t] = x[t];
 }
 
+template <int Q>
+hipError_t LaunchCGemm(int M, int N, int K, const float2* A, int lda, int transA, const float2* B, int ldb, float2* C,
+                       int ldc, hipStream_t stream)
+{
+    const int tilesM = (M + 64 * Q - 1) / (64 * Q), tilesN = (N + 64 * Q - 1) / (64 * Q);
+    const dim3 grid(tilesM * tilesN);
+#define CG_CASE(TR)                                                                                                  \
+    hipLaunchKernelGGL((cgemm_sub_kernel<TR, Q>), grid, dim3(256), 0, stream, M, N, K, A, static_cast<int64_t>(lda), \
+                       B, static_cast<int64_t>(ldb), C, static_cast<int64_t>(ldc), tilesM, tilesN)
+    if (transA == 0)
+        CG_CASE(0);
+    else if (transA == 1)
+        CG_CASE(1);
+    else
+        CG_CASE(2);
+#undef CG_CASE
+    return hipGetLastError();
+}
+
 hipError_t CGemmSub(int M, int N, int K, const float2* A, int lda, int transA, const float2* B, int ldb, float2* C,
                     int ldc, hipStream_t stream)
 {
     if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
-    const int tilesM = (M + 63) / 64, tilesN = (N + 63) / 64;
-    const dim3 grid(tilesM * tilesN);
-    if (transA == 0)
-        hipLaunchKernelGGL(cgemm_sub_kernel<0>, grid, dim3(256), 0, stream, M, N, K, A, lda, B, ldb, C, ldc, tilesM);
-    else if (transA == 1)
-        hipLaunchKernelGGL(cgemm_sub_kernel<1>, grid, dim3(256), 0, stream, M, N, K, A, lda, B, ldb, C, ldc, tilesM);
-    else
-        hipLaunchKernelGGL(cgemm_sub_kernel<2>, grid, dim3(256), 0, stream, M, N, K, A, lda, B, ldb, C, ldc, tilesM);
-    return hipGetLastError();
+    const int64_t big = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
+    if (big >= 256) return LaunchCGemm<2>(M, N, K, A, lda, transA, B, ldb, C, ldc, stream);
+    return LaunchCGemm<1>(M, N, K, A, lda, transA, B, ldb, C, ldc, stream);
 }
 
 template <bool FWD, bool UNIT, int TRANS>
@@ -825,93 +371,42 @@ hipError_t CTrsmBlock(int K, int N, const float2* T, int ldt, bool lower, bool u
 
 // Workspace: ints [0, m) row sources, two moved-row lists of 4 CNB + 8 (panel k uses list
 // k % 2, so the look-ahead panel can build its list while the previous one is still being
-// applied), the leaf's map (136); then, 8-byte aligned, the exchange slots of the
-// multi-workgroup leaf and its timeout flag.
-constexpr int kCLeafMultiRows = 2048;  // panels taller than this spread their leaves
+// applied), the leaf's moved rows; then, 8-byte aligned, the exchange words of the
+// multi-workgroup leaves, the rows a leaf's update takes, two panels' diagonal-block inverses and
+// the timeout flag.
 constexpr int kCMovedInts = 4 * CNB + 8;
+inline int CPanelBlocks(int m) { return (std::min(m, CNB) + 63) / 64; }
 struct CWork
 {
     int* rowsrc;
     int* moved[2];
-    int* leafmap;
+    int* moves;
     unsigned long long* slots;
+    float2* panelRows;
+    float* linv[2];
     int* err;
-    unsigned* epoch;  // host counter: tag base of the next multi-workgroup leaf
 };
-inline size_t CWorkInts(int m) { return static_cast<size_t>(m) + 2 * kCMovedInts + 1 + 2 * 64 + 7; }
+inline size_t CWorkInts(int m) { return static_cast<size_t>(m) + 2 * kCMovedInts + 4 * kCLeafWidth + 2; }
+inline size_t CWorkWords(int m)  // 8-byte words behind the ints
+{
+    const size_t blocks = static_cast<size_t>(CPanelBlocks(m));
+    return kCLeafSlotWords + blocks * 64 * 64 + 2 * blocks * (kCInverseBlock / 2) + 1;
+}
 CWork CLayout(void* base, int m)
 {
-    int* p = static_cast<int*>(base);
+    const size_t blocks = static_cast<size_t>(CPanelBlocks(m));
     CWork w;
-    w.rowsrc = p;
-    w.moved[0] = p + m;
-    w.moved[1] = w.moved[0] + kCMovedInts;
-    w.leafmap = w.moved[1] + kCMovedInts;
-    uintptr_t q = reinterpret_cast<uintptr_t>(p + CWorkInts(m));
-    q = (q + 7) & ~static_cast<uintptr_t>(7);
+    uintptr_t q = (reinterpret_cast<uintptr_t>(base) + 7) & ~static_cast<uintptr_t>(7);
     w.slots = reinterpret_cast<unsigned long long*>(q);
-    w.err = reinterpret_cast<int*>(q + kCSlotBytes);
-    w.epoch = nullptr;
+    w.panelRows = reinterpret_cast<float2*>(w.slots + kCLeafSlotWords);
+    w.linv[0] = reinterpret_cast<float*>(w.panelRows + blocks * 64 * 64);
+    w.linv[1] = w.linv[0] + blocks * kCInverseBlock;
+    w.err = reinterpret_cast<int*>(w.linv[1] + blocks * kCInverseBlock);
+    w.moves = w.err + 2;
+    w.moved[0] = w.moves + 4 * kCLeafWidth;
+    w.moved[1] = w.moved[0] + kCMovedInts;
+    w.rowsrc = w.moved[1] + kCMovedInts;
     return w;
-}
-
-template <int T, int R, int W>
-hipError_t LaunchCLeaf(float2* A, int lda, int m, int j0, int c0, int wact, int pivoting, int newPanel, int* ipiv,
-                       int* info, const CWork& w, hipStream_t stream)
-{
-    hipLaunchKernelGGL((cleaf_kernel<T, R, W>), dim3(1), dim3(T), 0, stream, A, lda, m, j0, c0, wact, pivoting,
-                       newPanel, ipiv, info, w.rowsrc, w.leafmap);
-    return hipGetLastError();
-}
-
-int CLeafWidth(int mp)
-{
-    if (mp > kCLeafMultiRows) return 32;
-    if (mp <= 512) return 32;
-    if (mp <= 2048) return 16;
-    if (mp <= 4096) return 8;
-    if (mp <= 8192) return 4;
-    return 2;
-}
-
-hipError_t CLeaf(float2* A, int lda, int m, int j0, int c0, int wact, int pivoting, int newPanel, int* ipiv, int* info,
-                 const CWork& w, hipStream_t stream)
-{
-    const int mp = m - c0;
-    if (mp > kCLeafMultiRows)
-    {
-        constexpr int R = 2, W = 32;
-        const int groups = (mp + 64 * R - 1) / (64 * R);
-        if (groups > kCMaxGroups || wact > W || w.epoch == nullptr) return hipErrorInvalidValue;
-        // Tags: W per leaf; key words carry 16 bits of them, which must not wrap within one
-        // factorization (slots cleared at its start): at most n / W leaves.
-        unsigned tagBase = (*w.epoch)++ * static_cast<unsigned>(W);
-        if (tagBase + W > 0xffffu) return hipErrorInvalidValue;
-        unsigned spinLimit = SpinLimit();
-        // Cooperative launch: the workgroups wait for each other every column, so all of
-        // them must be resident at once.
-        int* rowsrc = w.rowsrc;
-        int* leafmap = w.leafmap;
-        unsigned long long* slots = w.slots;
-        int* err = w.err;
-        void* args[] = {&A, &lda, &m, &c0, &wact, &pivoting, &newPanel, &ipiv, &info, &rowsrc, &leafmap, &slots,
-                        &tagBase, &err, &spinLimit};
-        if (wact == W && LeafSpread())
-            return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&cleaf_multi_kernel<R, W, true, true>),
-                                              dim3(8 * groups), dim3(64), args, 0, stream);
-        const void* fn = wact == W ? reinterpret_cast<const void*>(&cleaf_multi_kernel<R, W, true>)
-                                   : reinterpret_cast<const void*>(&cleaf_multi_kernel<R, W, false>);
-        return hipLaunchCooperativeKernel(fn, dim3(groups), dim3(64), args, 0, stream);
-    }
-#define CLEAF(T, R, W) LaunchCLeaf<T, R, W>(A, lda, m, j0, c0, wact, pivoting, newPanel, ipiv, info, w, stream)
-    if (mp <= 256) return CLEAF(256, 1, 32);
-    if (mp <= 512) return CLEAF(512, 1, 32);
-    if (mp <= 1024) return CLEAF(512, 2, 16);
-    if (mp <= 2048) return CLEAF(512, 4, 16);
-    if (mp <= 4096) return CLEAF(512, 8, 8);
-    if (mp <= 8192) return CLEAF(512, 16, 4);
-    return CLEAF(512, 32, 2);
-#undef CLEAF
 }
 
 #define CRET(e)                          \
@@ -926,21 +421,21 @@ hipError_t CLeaf(float2* A, int lda, int m, int j0, int c0, int wact, int pivoti
 size_t ComplexGetrfWorkspaceBytes(int m, int n)
 {
     (void)n;
-    return CWorkInts(std::max(m, 1)) * sizeof(int) + 8 + kCSlotBytes + 16;
+    m = std::max(m, 1);
+    return CWorkInts(m) * sizeof(int) + CWorkWords(m) * 8 + 16;
 }
 
 hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, void* work, hipStream_t stream,
                         const LookAhead* la)
 {
-    if (m > 16384) return hipErrorInvalidValue;
+    if (m > kCLeafMaxRows) return hipErrorInvalidValue;
     CWork w = CLayout(work, m);
-    unsigned epoch = 1;
-    w.epoch = &epoch;
     FillInfo(info, 1, 0, stream);
-    if (m > kCLeafMultiRows)
+    const bool multi = m > kCLeafSingleRows;
     {
-        constexpr int words = static_cast<int>(kCSlotBytes / sizeof(unsigned long long));
-        hipLaunchKernelGGL(cclear_slots_kernel, dim3((words + 255) / 256), dim3(256), 0, stream, w.slots, words, w.err);
+        const int words = multi ? kCLeafSlotWords : 0;
+        hipLaunchKernelGGL(cclear_slots_kernel, dim3(std::max(1, (words + 255) / 256)), dim3(256), 0, stream, w.slots,
+                           words, w.err);
     }
     const int kmax = std::min(m, n);
     if (kmax == 0) return hipGetLastError();
@@ -958,35 +453,39 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
         CRET(hipStreamWaitEvent(s1, la->fork, 0));
     }
 
-    // Panel k: its leaves (each followed by the update of the panel's remaining columns),
-    // then the list of its interchanges.
+    // Panel k: per 64 columns one leaf, one launch that applies its interchanges to the whole
+    // panel and inverts its diagonal block, one that updates the panel columns to its right;
+    // then the list of the panel's interchanges.
     auto panel = [&](int k) -> hipError_t
     {
-        const int j0 = k * CNB, nb = std::min(CNB, kmax - j0), panelEnd = j0 + nb;
-        for (int c0 = j0; c0 < panelEnd;)
+        const int j0 = k * CNB, panelEnd = std::min(j0 + CNB, kmax);
+        for (int c0 = j0; c0 < panelEnd; c0 += kCLeafWidth)
         {
-            const int W = CLeafWidth(m - c0);
-            const int wact = std::min(W, panelEnd - c0);
-            CRET(CLeaf(a, lda, m, j0, c0, wact, pivoting, c0 == j0, ipiv, info, w, s0));
-            const int others = nb - wact;
-            if (others > 0)
-            {
-                if (pivoting)
-                    hipLaunchKernelGGL(cpanel_swap_trsm_kernel, dim3(others), dim3(128), 0, s0, a, lda, j0, c0, wact,
-                                       w.leafmap);
-                else if (panelEnd - c0 - wact > 0)
-                    CRET(CTrsmBlock(wact, panelEnd - c0 - wact, a + static_cast<size_t>(c0) * lda + c0, lda, true,
-                                    true, 0, a + static_cast<size_t>(c0 + wact) * lda + c0, lda, s0));
-                CRET(hipGetLastError());
-                const int right = panelEnd - c0 - wact;
-                if (right > 0 && m - c0 - wact > 0)
-                    CRET(CGemmSub(m - c0 - wact, right, wact, a + static_cast<size_t>(c0) * lda + c0 + wact, lda, 0,
-                                  a + static_cast<size_t>(c0 + wact) * lda + c0, lda,
-                                  a + static_cast<size_t>(c0 + wact) * lda + c0 + wact, lda, s0));
-            }
-            c0 += wact;
+            CLeafArgs l;
+            l.A = a;
+            l.lda = lda;
+            l.m = m;
+            l.j0 = j0;
+            l.c0 = c0;
+            l.wact = std::min(kCLeafWidth, panelEnd - c0);
+            l.panelEnd = panelEnd;
+            l.pivoting = pivoting;
+            l.newPanel = c0 == j0;
+            l.ipiv = ipiv;
+            l.info = info;
+            l.rowsrc = w.rowsrc;
+            l.moves = w.moves;
+            l.slots = w.slots;
+            // The key words carry 16 bits of a tag: at most 256 leaves of 64 tags and the first.
+            l.tagBase = static_cast<unsigned>(c0 + kCLeafWidth);
+            l.err = w.err;
+            l.spinLimit = SpinLimit();
+            float* const linv = w.linv[k & 1] + static_cast<size_t>((c0 - j0) / 64) * kCInverseBlock;
+            CRET(CLeafColumns(l, LeafSpread(), s0));
+            CRET(CLeafFinish(l, linv, w.panelRows, s0));
+            if (c0 + l.wact < panelEnd) CRET(CPanelUpdate(l, linv, w.panelRows, s0));
         }
-        if (pivoting)
+        if (pivoting && (k > 0 || panelEnd < n))
             hipLaunchKernelGGL(ccompact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, w.moved[k & 1]);
         return hipGetLastError();
     };
@@ -1001,8 +500,8 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
                                hi, w.moved[k & 1]);
         CRET(hipGetLastError());
         if (cols <= 0) return hipSuccess;
-        CRET(CTrsmBlock(nb, cols, a + static_cast<size_t>(j0) * lda + j0, lda, true, true, 0,
-                        a + static_cast<size_t>(lo) * lda + j0, lda, st));
+        CRET(CTrsmLowerUnit(nb, cols, a + static_cast<size_t>(j0) * lda + j0, lda, w.linv[k & 1],
+                            a + static_cast<size_t>(lo) * lda + j0, lda, st));
         if (m - pe <= 0) return hipSuccess;
         ProfileScope prof(ProfileKernel::ComplexGemm, 8.0 * (m - pe) * cols * nb, st);
         return CGemmSub(m - pe, cols, nb, a + static_cast<size_t>(j0) * lda + pe, lda, 0,
@@ -1030,7 +529,7 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
         }
     }
     if (two) CRET(hipStreamWaitEvent(s0, la->bulk[(npanel - 1) & 1], 0));
-    if (m > kCLeafMultiRows) FoldWaitError(w.err, info, s0);
+    if (multi) FoldWaitError(w.err, info, s0);
     return hipGetLastError();
 }
 
