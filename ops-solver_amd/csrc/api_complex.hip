@@ -200,7 +200,7 @@ aclsolverStatus_t InverseByFactor(aclsolverHandle_t h, int n, const float2* a, i
     hipStream_t s = Stream(h);
     const size_t luBytes = static_cast<size_t>(n) * n * sizeof(float2);
     const size_t need = luBytes + static_cast<size_t>(n) * sizeof(int) + ComplexGetrfWorkspaceBytes(n, n) +
-                        ComplexGetrsWorkspaceBytes(n, n) + 1024;
+                        ComplexGetrsWorkspaceBytes(n, n, true) + 1024;
     char* base = static_cast<char*>(HandleScratch(h, need));
     if (base == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
     float2* lu = reinterpret_cast<float2*>(base);
@@ -217,7 +217,7 @@ aclsolverStatus_t InverseByFactor(aclsolverHandle_t h, int n, const float2* a, i
     else
         hipLaunchKernelGGL(c_first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, lu, n, info);
     hipLaunchKernelGGL(c_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, c, ldc);
-    if (ComplexGetrs(0, n, n, lu, n, p, c, ldc, sw, s) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
+    if (ComplexGetrs(0, n, n, lu, n, p, c, ldc, sw, s, info, true) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();
 }
 }  // namespace
@@ -292,10 +292,10 @@ OPS_API aclsolverStatus_t aclsolverCgetrsDevice(aclsolverHandle_t handle, int tr
     hipStream_t s = Stream(handle);
     FillInfo(devInfo, 1, 0, s);
     if (n == 0 || nrhs == 0) return Launched();
-    void* work = HandleScratch(handle, ComplexGetrsWorkspaceBytes(n, nrhs));
+    void* work = HandleScratch(handle, ComplexGetrsWorkspaceBytes(n, nrhs, true));
     if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
     if (ComplexGetrs(trans, n, nrhs, reinterpret_cast<const float2*>(dA), lda, devIpiv, reinterpret_cast<float2*>(dB),
-                     ldb, work, s) != hipSuccess)
+                     ldb, work, s, devInfo, true) != hipSuccess)
         return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();
 }
@@ -325,7 +325,7 @@ struct ComplexStagingRuntime
         return hipGetLastError() != hipSuccess;
     }
     int Synchronize() { return hipStreamSynchronize(s) != hipSuccess; }
-    size_t WorkBytes(int nn, int rr) { return ComplexGetrsWorkspaceBytes(nn, rr); }
+    size_t WorkBytes(int nn, int rr) { return ComplexGetrsWorkspaceBytes(nn, rr, true); }
     int Solve(const hoststage::Staging& st)
     {
         float2* aRow = static_cast<float2*>(st.aRow);
@@ -334,7 +334,7 @@ struct ComplexStagingRuntime
         float2* bCol = static_cast<float2*>(st.bCol);
         hipError_t e = CTransposeRM(n, n, aRow, lda, aCol, n, s);
         if (e == hipSuccess) e = CTransposeRM(n, nrhs, bRow, ldb, bCol, n, s);
-        if (e == hipSuccess) e = ComplexGetrs(trans, n, nrhs, aCol, n, st.piv, bCol, n, st.work, s);
+        if (e == hipSuccess) e = ComplexGetrs(trans, n, nrhs, aCol, n, st.piv, bCol, n, st.work, s, nullptr, true);
         if (e == hipSuccess) e = CTransposeRM(nrhs, n, bCol, n, bRow, ldb, s);
         return e != hipSuccess;
     }
@@ -355,7 +355,7 @@ OPS_API aclError aclsolverCgetrs(aclsolverHandle_t handle, const uint64_t trans,
 
 static size_t CGetriWorkBytes(int n)
 {
-    return static_cast<size_t>(n) * n * sizeof(float2) + ComplexGetrsWorkspaceBytes(n, n) + 256;
+    return static_cast<size_t>(n) * n * sizeof(float2) + ComplexGetrsWorkspaceBytes(n, n, false) + 256;
 }
 
 OPS_API aclsolverStatus_t aclsolverCgetri_bufferSize(aclsolverHandle_t handle, int n, aclFloatComplex* A, int lda,
@@ -411,7 +411,7 @@ OPS_API aclsolverStatus_t aclsolverCgetri(aclsolverHandle_t handle, int n, aclFl
     float2* a = reinterpret_cast<float2*>(A);
     hipLaunchKernelGGL(c_first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, a, lda, devInfo);
     hipLaunchKernelGGL(c_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, X, n);
-    if (ComplexGetrs(0, n, n, a, lda, devIpiv, X, n, w, s) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
+    if (ComplexGetrs(0, n, n, a, lda, devIpiv, X, n, w, s, nullptr, false) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
     hipLaunchKernelGGL(c_copy_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, n, X, n, a, lda, devInfo);
     return Launched();
 }

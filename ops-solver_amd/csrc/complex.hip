@@ -23,6 +23,7 @@
 
 #include "cleaf.h"
 #include "complex_math.h"
+#include "ctrs.h"
 #include "internal.h"
 
 namespace ops
@@ -553,16 +554,27 @@ __global__ void cpermute_kernel(int n, int nrhs, const int* __restrict__ perm, c
 }
 }  // namespace
 
-size_t ComplexGetrsWorkspaceBytes(int n, int nrhs)
+namespace
 {
+// The chain up to 2048 right-hand sides; n = 8192: 1 rhs 10.5 and 2.1 ms (per-block launches, chain),
+// 256 12.0 and 3.1, 2048 22.1 and 13.0 (transposed 20.9 and 19.1); n = 400, 2048 rhs: 539 and 191
+// us. Beyond, its published words (16 bytes an element) and the re-reading of the factors per 16
+// columns outweigh the launches.
+bool UseChain(int nrhs) { return nrhs <= kCTrsMaxRhs; }
+}  // namespace
+
+size_t ComplexGetrsWorkspaceBytes(int n, int nrhs, bool chain)
+{
+    if (chain && UseChain(nrhs)) return CTrsWorkspaceBytes(n, nrhs);
     return static_cast<size_t>(n) * std::max(nrhs, 1) * sizeof(float2) + (static_cast<size_t>(n) + 64) * sizeof(int);
 }
 
 hipError_t ComplexGetrs(int trans, int n, int nrhs, const float2* lu, int lda, const int* ipiv, float2* b, int ldb,
-                        void* work, hipStream_t stream)
+                        void* work, hipStream_t stream, int* info, bool chain)
 {
     if (n <= 0 || nrhs <= 0) return hipSuccess;
     if (n > 16384) return hipErrorInvalidValue;
+    if (chain && UseChain(nrhs)) return CTrsSolve(trans, n, nrhs, lu, lda, ipiv, b, ldb, info, work, stream);
     float2* x = static_cast<float2*>(work);
     int* perm = reinterpret_cast<int*>(x + static_cast<size_t>(n) * nrhs);
     if (ipiv) CRET(IpivToPerm(n, ipiv, perm, stream, true));

@@ -190,8 +190,9 @@ size_t ComplexGetrfWorkspaceBytes(int m, int n);
 // on la->side beside the next panel).
 hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, void* work, hipStream_t stream,
                         const LookAhead* la = nullptr);
-size_t ComplexGetrsWorkspaceBytes(int n, int nrhs);
+// chain: the chained solve may be taken (its workspace is larger); info as in CTrsSolve.
+size_t ComplexGetrsWorkspaceBytes(int n, int nrhs, bool chain);
 hipError_t ComplexGetrs(int trans, int n, int nrhs, const float2* lu, int lda, const int* ipiv, float2* b, int ldb,
-                        void* work, hipStream_t stream);
+                        void* work, hipStream_t stream, int* info, bool chain);
 
 }  // namespace ops
