@@ -643,26 +643,6 @@ __device__ inline void CGroupArgmax(uint32_t val, int key, uint32_t* bestVal, in
     *bestKey = k;
 }
 
-// Column k of a register row (k uniform but not a compile-time constant): a select chain,
-// so register arrays stay in registers when the loop over k is not unrolled.
-template <int NL>
-__device__ inline float2 GetCol(const float2 (&S)[NL], int k)
-{
-    float2 v = S[0];
-#pragma unroll
-    for (int j = 1; j < NL; ++j) v = (j == k) ? S[j] : v;
-    return v;
-}
-template <int NL>
-__device__ inline void SetCol(float2 (&S)[NL], int k, float2 v)
-{
-#pragma unroll
-    for (int j = 0; j < NL; ++j) S[j] = (j == k) ? v : S[j];
-}
-// Up to 32 columns the loops over k are unrolled (k becomes a constant and the selects
-// fold away); at 64 they stay loops, which keeps those kernels small enough to compile
-// quickly and to fit the instruction cache.
-
 // Gauss-Jordan with implicit pivoting (see batched.hip for the real derivation).
 template <int NL>
 __global__ __launch_bounds__(256) void cmatinv_gj_kernel(int n, const float2* const* __restrict__ Aarr,
@@ -696,7 +676,7 @@ __global__ __launch_bounds__(256) void cmatinv_gj_kernel(int n, const float2* co
     // Slot j of S holds column (j + steps done) % NL: each step pivots slot 0 and rotates the
     // slots down by one (the processed column moves to the last slot), so no slot is ever
     // addressed by a run-time index, also where the step loop is not unrolled.
-#pragma unroll(NL <= 32 ? NL : 1)
+#pragma unroll
     for (int k = 0; k < NL; ++k)
     {
         if (k < n)
@@ -888,8 +868,7 @@ hipError_t CMatinvBatched(int n, const float2* const* Aarr, const float2* Abase,
         return LaunchCMatinv<16>(n, Aarr, Abase, lda, strideA, Carr, Cbase, ldc, strideC, info, batch, stream);
     if (n <= 32)
         return LaunchCMatinv<32>(n, Aarr, Abase, lda, strideA, Carr, Cbase, ldc, strideC, info, batch, stream);
-    if (n <= 64)
-        return LaunchCMatinv<64>(n, Aarr, Abase, lda, strideA, Carr, Cbase, ldc, strideC, info, batch, stream);
+    if (n <= 64) return CMatinvRows64(n, Aarr, Abase, lda, strideA, Carr, Cbase, ldc, strideC, info, batch, stream);
     return hipErrorNotSupported;  // 64 < n: the caller takes the factor-and-solve route
 }
 

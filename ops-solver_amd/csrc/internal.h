@@ -190,6 +190,10 @@ size_t ComplexGetrfWorkspaceBytes(int m, int n);
 // on la->side beside the next panel).
 hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, void* work, hipStream_t stream,
                         const LookAhead* la = nullptr);
+// Orders up to 64 (cmatinv.hip); info receives the first zero pivot's step.
+hipError_t CMatinvRows64(int n, const float2* const* Aarr, const float2* Abase, int lda, int64_t strideA,
+                         float2* const* Carr, float2* Cbase, int ldc, int64_t strideC, int* info, int batch,
+                         hipStream_t stream);
 // chain: the chained solve may be taken (its workspace is larger); info as in CTrsSolve.
 size_t ComplexGetrsWorkspaceBytes(int n, int nrhs, bool chain);
 hipError_t ComplexGetrs(int trans, int n, int nrhs, const float2* lu, int lda, const int* ipiv, float2* b, int ldb,

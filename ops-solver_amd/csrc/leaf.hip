@@ -35,6 +35,7 @@
 #include <climits>
 
 #include "internal.h"
+#include "lanes.h"
 #include "trtri64.h"
 #include "wave.h"
 
@@ -61,25 +62,6 @@ __device__ inline void StoreWord(unsigned long long* p, unsigned long long v, bo
 __device__ inline void StoreTagged(unsigned long long* p, unsigned tag, float v, bool local)
 {
     StoreWord(p, (static_cast<unsigned long long>(tag) << 32) | __float_as_uint(v), local);
-}
-
-// The upper 32 lanes of x and the lower 32 lanes of y change places.
-__device__ inline void SwapHalves(float& x, float& y)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-    x = __uint_as_float(r[0]);
-    y = __uint_as_float(r[1]);
-}
-__device__ inline void SwapHalves(int& x, int& y)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(static_cast<unsigned>(x), static_cast<unsigned>(y), false, false);
-    x = static_cast<int>(r[0]);
-    y = static_cast<int>(r[1]);
-}
-
-__device__ inline float ReadLane(float v, int lane)
-{
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
 }
 
 // Maximum over the NW values that the lanes hold cyclically (lane l: value l % NW).
