@@ -457,7 +457,7 @@ def complex_solve(A, torch, h, n=8192, nrhs=16, steps=2):
 def uneven_batched(A, torch, h, steps=5):
     """20000 FP32 systems, n_i ~ U{8..256} (seeded), A_i = N(0,1)/sqrt(n_i) + 2I, 4 RHS:
     getrf + getrs of every system through one plan execution: four size-class launches
-    (plan built and autotuned once, untimed). Inputs are restored between steps outside the
+    (plan built once, untimed). Inputs are restored between steps outside the
     timed events."""
     import numpy as np
 
@@ -513,8 +513,8 @@ def uneven_batched(A, torch, h, steps=5):
         r = (Bi - Ai @ Xi).abs().max() / (Ai.abs().sum(1).max() * Xi.abs().max() + Bi.abs().max())
         worst = max(worst, r.item())
     return {"workload": "20000 FP32 systems, n_i ~ U{8..256}, A_i = N(0,1)/sqrt(n_i) + 2I, 4 RHS; getrf+getrs "
-                        "through one plan, one persistent launch: n<=64 one wave per system, 65..256 column-cyclic "
-                        "wave groups (configuration per 16-wide size bin from the autotuner)",
+                        "through one plan, one launch per size class: n<=64 one wave per system, 65..256 one "
+                        "workgroup of 2 to 4 waves per system",
             "schedule": {f"{65 + 16 * b}..{80 + 16 * b}": cfg_names.get(int(c), str(int(c))) for b, c in enumerate(sched)},
             "ms": round(ms, 4), "solves_per_s": round(count / ms * 1e3, 1),
             "GB_per_s": round(bytes_ / ms / 1e6, 1), "hbm_frac": round(bytes_ / (ms * 1e-3) / PEAK_HBM, 4),

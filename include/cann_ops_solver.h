@@ -166,13 +166,13 @@ extern "C"
      * pivoting, as sgetrf. SS always uses partial pivoting. */
     aclsolverStatus_t aclsolverSetTournamentPivoting(aclsolverHandle_t handle, int on);
 
-    /* ---- EXTENSION: uneven batched LU solve (getrf + getrs) in one persistent launch ----
+    /* ---- EXTENSION: uneven batched LU solve (getrf + getrs) ----
      * nArray (HOST, batchSize entries) holds each order n_i; dAarray / dBarray are Device
      * arrays of Device pointers to column-major A_i (n_i x n_i, lda = n_i) and B_i
      * (n_i x nrhs, ldb = n_i); A_i is overwritten by its packed LU, B_i by X_i. dIpiv holds
      * sum(n_i) pivots, matrix i's at offset sum_{j<i} n_j. dInfo gets one info per matrix.
-     * A plan bins the matrices by size and holds the tuned per-bin schedule; executing a
-     * plan allocates nothing, synchronizes nothing and may be captured into a hipGraph. */
+     * A plan sorts the matrices into size classes; executing it is one launch per class (at
+     * most four), allocates nothing, synchronizes nothing and may be captured into a hipGraph. */
     typedef void* aclsolverVbatchedPlan_t;
     aclsolverStatus_t aclsolverSgesvVbatched_createPlan(aclsolverHandle_t handle, int batchSize, const int* nArray,
                                                         int nrhs, aclsolverVbatchedPlan_t* plan);
@@ -184,9 +184,10 @@ extern "C"
      * the configuration that solves its matrices, as an id: 1 = 2 rows per lane, 4 waves per
      * matrix (n <= 128); 2 = 2 rows, 8 waves (n <= 128); 3 = 3 rows, 8 waves (n <= 192);
      * 4 = 3 rows, 16 waves (n <= 192); 5 = 4 rows, 16 waves (n <= 256). Orders <= 64 always
-     * take one wave per matrix. createPlan takes the autotuned schedule of the device;
-     * createPlanWithSchedule takes the caller's (INVALID_VALUE for an id outside 1..5 or one
-     * whose largest order is below its bin's); getSchedule reports a plan's. */
+     * take one wave per matrix. createPlanWithSchedule takes the caller's (INVALID_VALUE for an
+     * id outside 1..5 or one whose largest order is below its bin's). createPlan needs none: orders
+     * above 64 take one workgroup of 2 to 4 waves per matrix. getSchedule reports a plan's (for
+     * createPlan's the first id that fits each bin). */
     aclsolverStatus_t aclsolverSgesvVbatched_createPlanWithSchedule(aclsolverHandle_t handle, int batchSize,
                                                                     const int* nArray, int nrhs, const int* schedule,
                                                                     aclsolverVbatchedPlan_t* plan);

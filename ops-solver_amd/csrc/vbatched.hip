@@ -1,7 +1,7 @@
 // Uneven batched LU solve (getrf + getrs per matrix), EXTENSION: the reference has no
 // batched getrf/getrs.
 //
-// One persistent launch: a grid of one 1024-thread workgroup per CU pulls items from a
+// A persistent launch: a grid of one 1024-thread workgroup per CU pulls items from a
 // device queue (largest orders first: longest-processing-time order). An item is a group of
 // matrices of similar order and one configuration, which splits the workgroup's 16 waves:
 //   W64   n <= 64:  one wave per matrix, 16 matrices per item;
@@ -10,11 +10,10 @@
 //   C3x8  n <= 192: column-cyclic, 3 rows per lane, 8 waves per matrix, 2 per item;
 //   C3x16 n <= 192: column-cyclic, 3 rows per lane, 16 waves, 1 per item;
 //   C4x16 n <= 256: column-cyclic, 4 rows per lane, 16 waves, 1 per item.
-// The configuration of each 16-wide size bin above 64 is chosen per device by an autotuner
-// that times every configuration that fits the bin on one item per CU of synthetic systems
-// of the bin's largest order (at most ~80 MB of samples, generated on the device) and keeps the
-// one with the least time per matrix; a plan may also be given the schedule explicitly.
-// The last workgroup to leave re-arms the queue, so executing a plan is one kernel launch.
+// Orders above 64 take vbrows.hip's kernels (one workgroup per matrix: outputs the same, 20000
+// systems of orders 1..256 in 4.8 instead of 8.2 ms) unless the plan's caller gives a schedule,
+// the configuration of each 16-wide size bin above 64: those go through the queue here.
+// The last workgroup to leave re-arms the queue, so the queue needs no reset between launches.
 //
 // Column-cyclic kernel (one matrix per workgroup): lane l of every wave holds rows
 // l, l + 64, ... of the matrix; wave w holds columns w, w + NW, w + 2 NW, ... of the augmented
@@ -35,15 +34,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cfloat>
 #include <climits>
-#include <map>
-#include <mutex>
 #include <new>
 #include <vector>
 
+#include "backsub.h"
 #include "internal.h"
+#include "vbrows.h"
 
 namespace ops
 {
@@ -434,11 +432,6 @@ __device__ inline bool Aborted(int& flag, int it)
     return true;
 }
 
-__device__ inline float Rl(float v, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
 // The pivot row's values in this wave's column slots, written to the wave's LDS row buffer
 // by the lane that holds the row (lane lp, slot sp; call under lane == lp) for the chunks of
 // four slots below nv; every lane then reads them back as a broadcast. This replaces one
@@ -622,55 +615,6 @@ __device__ __attribute__((always_inline)) inline void PivotColumn(float (&col)[R
     }
 #pragma unroll
     for (int i = 0; i < RPL; ++i) col[i] = (below[i] & (l[i] != 0.0f)) ? l[i] : col[i];
-}
-
-// Back substitution over the columns k of position segment S (64 S <= k < 64 S + 64, k < n),
-// last to first, then the segments below. Lane l holds y at positions l + 64 i; column k of
-// U (rows 0 .. 64 S + 63, slots 0..S) is read from the stored LU with a prefetch of D columns
-// in registers. x_k = y_k * (1 / U_kk): the reciprocal depends only on U, so it stays off
-// the dependent chain that runs through the y values.
-template <int S, int RPL, int Q>
-__device__ __attribute__((always_inline)) inline void BackSubSeg(const float* __restrict__ A, int n, int lane,
-                                                                 float (&y)[Q][RPL])
-{
-    constexpr int D = 8;
-    const int kLo = 64 * S;
-    const int kHi = min(n, 64 * S + 64) - 1;
-    float u[D][S + 1];
-#pragma unroll
-    for (int t = 0; t < D; ++t)
-    {
-        const int k = kHi - t;
-#pragma unroll
-        for (int i = 0; i <= S; ++i)
-            u[t][i] = (k >= kLo && lane + 64 * i < n) ? A[static_cast<size_t>(k) * n + lane + 64 * i] : 0.0f;
-    }
-    for (int k0 = kHi; k0 >= kLo; k0 -= D)
-    {
-#pragma unroll
-        for (int t = 0; t < D; ++t)
-        {
-            const int k = k0 - t;
-            if (k >= kLo)
-            {
-                const int kl = k - kLo;
-                const float r = 1.0f / Rl(u[t][S], kl);
-#pragma unroll
-                for (int q = 0; q < Q; ++q)
-                {
-                    const float x = Rl(y[q][S], kl) * r;
-#pragma unroll
-                    for (int i = 0; i < S; ++i) y[q][i] = fmaf(-u[t][i], x, y[q][i]);
-                    y[q][S] = lane < kl ? fmaf(-u[t][S], x, y[q][S]) : (lane == kl ? x : y[q][S]);
-                }
-            }
-            const int kn = k - D;
-#pragma unroll
-            for (int i = 0; i <= S; ++i)
-                u[t][i] = (kn >= kLo && lane + 64 * i < n) ? A[static_cast<size_t>(kn) * n + lane + 64 * i] : 0.0f;
-        }
-    }
-    if constexpr (S > 0) BackSubSeg<S - 1, RPL, Q>(A, n, lane, y);
 }
 
 // Column slots per wave of the column-cyclic solve (a multiple of 4).
@@ -1022,29 +966,6 @@ __global__ __launch_bounds__(1024) void vb_persistent_kernel(const Item* __restr
     }
 }
 
-// Synthetic systems for the autotuner: count matrices of order n at A + i * n * n (diagonally
-// dominant, deterministic), right-hand sides of ones, pointer arrays.
-__global__ void tune_fill_kernel(int n, int count, int nrhs, float* A, float* B, float** Ap, float** Bp)
-{
-    const size_t per = static_cast<size_t>(n) * n, total = per * count;
-    for (size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
-         e += static_cast<size_t>(gridDim.x) * blockDim.x)
-    {
-        const int i = static_cast<int>(e / per);
-        const int c = static_cast<int>((e % per) / n), r = static_cast<int>(e % n);
-        const float off = 0.25f * static_cast<float>(((r * 7 + c * 13 + i) % 17) - 8) / (8.0f * n);
-        A[e] = (r == c ? 2.0f : 0.0f) + off;
-    }
-    for (size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-         e < static_cast<size_t>(count) * n * (nrhs > 0 ? nrhs : 1); e += static_cast<size_t>(gridDim.x) * blockDim.x)
-        B[e] = 1.0f;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x)
-    {
-        Ap[i] = A + static_cast<size_t>(i) * n * n;
-        Bp[i] = B + static_cast<size_t>(i) * n * (nrhs > 0 ? nrhs : 1);
-    }
-}
-
 }  // namespace
 
 struct VbatchedPlan
@@ -1055,6 +976,8 @@ struct VbatchedPlan
     int numItems = 0;
     int grid = 0;                // one workgroup per CU
     int schedule[kNumBins] = {}; // configuration of each size bin above 64
+    int rowsFirst[3] = {};       // matrices of vbrows.hip's classes (4, 3, 2 waves) in the order
+    int rowsCount[3] = {};
     Item* dItems = nullptr;
     int* dOrder = nullptr;
     int* dN = nullptr;
@@ -1074,30 +997,30 @@ static void FreePlan(VbatchedPlan* p)
     delete p;
 }
 
-static hipError_t LaunchItems(const Item* items, int numItems, int grid, const int* order, const int* nArr,
-                              const long long* pivOff, int nrhs, float* const* dA, float* const* dB, int* dIpiv,
-                              int* dInfo, int* counters, hipStream_t s)
+// Up to four launches; capturable into a hipGraph from the caller's stream.
+hipError_t VbatchedLaunch(VbatchedPlan* p, float* const* dA, float* const* dB, int* dIpiv, int* dInfo, hipStream_t s)
 {
-    hipLaunchKernelGGL(vb_persistent_kernel, dim3(grid), dim3(1024), 0, s, items, numItems, order, nArr, pivOff, nrhs,
-                       dA, dB, dIpiv, dInfo, counters);
+    for (int c = 0; c < 3; ++c)
+    {
+        const hipError_t e = VbRowsLaunch(4 - c, p->rowsCount[c], p->dOrder + p->rowsFirst[c], p->dN, p->dPivOff,
+                                          p->nrhs, dA, dB, dIpiv, dInfo, s);
+        if (e != hipSuccess) return e;
+    }
+    if (p->numItems == 0) return hipSuccess;
+    hipLaunchKernelGGL(vb_persistent_kernel, dim3(p->grid), dim3(1024), 0, s, p->dItems, p->numItems, p->dOrder, p->dN,
+                       p->dPivOff, p->nrhs, dA, dB, dIpiv, dInfo, p->dCounter);
     return hipGetLastError();
 }
 
-// One launch; capturable into a hipGraph from the caller's stream.
-hipError_t VbatchedLaunch(VbatchedPlan* p, float* const* dA, float* const* dB, int* dIpiv, int* dInfo, hipStream_t s)
-{
-    return LaunchItems(p->dItems, p->numItems, p->grid, p->dOrder, p->dN, p->dPivOff, p->nrhs, dA, dB, dIpiv, dInfo,
-                       p->dCounter, s);
-}
-
-// Items of the plan: matrices in decreasing order of n, each group of up to kCfgCap[cfg]
+// Items of the plan: matrices from order[first] on in decreasing order of n, each group of up to kCfgCap[cfg]
 // consecutive matrices of one configuration an item (longest-processing-time order).
-static std::vector<Item> BuildItems(const std::vector<int>& ns, const std::vector<int>& order, const int* schedule)
+static std::vector<Item> BuildItems(const std::vector<int>& ns, const std::vector<int>& order, int first,
+                                    const int* schedule)
 {
     std::vector<Item> items;
     Item open[kNumCfg];
     for (int c = 0; c < kNumCfg; ++c) open[c] = {0, 0, c, 0};
-    for (int i = 0; i < static_cast<int>(order.size()); ++i)
+    for (int i = first; i < static_cast<int>(order.size()); ++i)
     {
         const int n = ns[order[i]];
         const int c = n <= 64 ? kW64 : schedule[BinOf(n)];
@@ -1117,109 +1040,6 @@ static std::vector<Item> BuildItems(const std::vector<int>& ns, const std::vecto
     return items;
 }
 
-// Autotuner (per device, once per process): for each bin above 64 and each configuration
-// that fits it, one launch of numCUs items (one per CU) of synthetic systems of the bin's
-// largest order; the configuration with the least time per matrix wins. Bins whose only
-// fitting configuration is C4x16 are not timed.
-static std::mutex g_tuneMutex;
-static std::map<int, std::array<int, kNumBins>> g_tuned;
-
-static hipError_t Autotune(int device, int numCUs, int nrhs, int* schedule, hipStream_t s)
-{
-    std::lock_guard<std::mutex> lock(g_tuneMutex);
-    auto hit = g_tuned.find(device);
-    if (hit != g_tuned.end())
-    {
-        std::copy(hit->second.begin(), hit->second.end(), schedule);
-        return hipSuccess;
-    }
-    size_t maxMats = 0, maxElems = 0;
-    for (int c = 1; c < kNumCfg; ++c)
-    {
-        maxMats = std::max<size_t>(maxMats, static_cast<size_t>(numCUs) * kCfgCap[c]);
-        maxElems = std::max<size_t>(maxElems, static_cast<size_t>(numCUs) * kCfgCap[c] * kCfgMaxN[c] * kCfgMaxN[c]);
-    }
-    float *dA = nullptr, *dB = nullptr;
-    float **dAp = nullptr, **dBp = nullptr;
-    int *dPiv = nullptr, *dInfo = nullptr, *dOrder = nullptr, *dN = nullptr, *dCnt = nullptr;
-    long long* dOff = nullptr;
-    Item* dItems = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    hipError_t e = hipMalloc(&dA, maxElems * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&dB, maxMats * 256 * kNrhsMax * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&dAp, maxMats * sizeof(float*));
-    if (e == hipSuccess) e = hipMalloc(&dBp, maxMats * sizeof(float*));
-    if (e == hipSuccess) e = hipMalloc(&dPiv, maxMats * 256 * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&dInfo, maxMats * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&dOrder, maxMats * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&dN, maxMats * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc(&dOff, maxMats * sizeof(long long));
-    if (e == hipSuccess) e = hipMalloc(&dItems, static_cast<size_t>(numCUs) * sizeof(Item));
-    if (e == hipSuccess) e = hipMalloc(&dCnt, 256);
-    if (e == hipSuccess) e = hipMemset(dCnt, 0, 256);
-    if (e == hipSuccess) e = hipEventCreate(&e0);
-    if (e == hipSuccess) e = hipEventCreate(&e1);
-    std::vector<int> iota(maxMats);
-    for (size_t i = 0; i < maxMats; ++i) iota[i] = static_cast<int>(i);
-    if (e == hipSuccess) e = hipMemcpy(dOrder, iota.data(), maxMats * sizeof(int), hipMemcpyHostToDevice);
-    std::array<int, kNumBins> best{};
-    for (int b = 0; b < kNumBins && e == hipSuccess; ++b)
-    {
-        const int n = 64 + kBinW * (b + 1);
-        double bestT = 1e30;
-        best[b] = kC4x16;
-        for (int c = 1; c < kNumCfg && e == hipSuccess; ++c)
-        {
-            if (kCfgMaxN[c] < n || (n > 192 && c == kC4x16)) continue;  // does not fit / nothing to compare
-            const int cap = kCfgCap[c], mats = numCUs * cap;
-            std::vector<Item> items(numCUs);
-            for (int i = 0; i < numCUs; ++i) items[i] = {i * cap, cap, c, 0};
-            std::vector<int> nv(mats, n);
-            std::vector<long long> off(mats);
-            for (int i = 0; i < mats; ++i) off[i] = static_cast<long long>(i) * n;
-            e = hipMemcpy(dItems, items.data(), items.size() * sizeof(Item), hipMemcpyHostToDevice);
-            if (e == hipSuccess) e = hipMemcpy(dN, nv.data(), mats * sizeof(int), hipMemcpyHostToDevice);
-            if (e == hipSuccess) e = hipMemcpy(dOff, off.data(), mats * sizeof(long long), hipMemcpyHostToDevice);
-            float t = 1e30f;
-            for (int rep = 0; rep < 2 && e == hipSuccess; ++rep)
-            {
-                hipLaunchKernelGGL(tune_fill_kernel, dim3(1024), dim3(256), 0, s, n, mats, nrhs, dA, dB, dAp, dBp);
-                e = hipEventRecord(e0, s);
-                if (e == hipSuccess)
-                    e = LaunchItems(dItems, numCUs, numCUs, dOrder, dN, dOff, nrhs, dAp, dBp, dPiv, dInfo, dCnt, s);
-                if (e == hipSuccess) e = hipEventRecord(e1, s);
-                if (e == hipSuccess) e = hipEventSynchronize(e1);
-                float ms = 0.0f;
-                if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
-                t = std::min(t, ms);
-            }
-            const double perMatrix = static_cast<double>(t) / cap;
-            if (e == hipSuccess && perMatrix < bestT)
-            {
-                bestT = perMatrix;
-                best[b] = c;
-            }
-        }
-    }
-    (void)hipFree(dA);
-    (void)hipFree(dB);
-    (void)hipFree(dAp);
-    (void)hipFree(dBp);
-    (void)hipFree(dPiv);
-    (void)hipFree(dInfo);
-    (void)hipFree(dOrder);
-    (void)hipFree(dN);
-    (void)hipFree(dOff);
-    (void)hipFree(dItems);
-    (void)hipFree(dCnt);
-    if (e0) (void)hipEventDestroy(e0);
-    if (e1) (void)hipEventDestroy(e1);
-    if (e != hipSuccess) return e;
-    g_tuned[device] = best;
-    std::copy(best.begin(), best.end(), schedule);
-    return hipSuccess;
-}
-
 }  // namespace ops
 
 using namespace ops;
@@ -1227,7 +1047,7 @@ using namespace ops;
 namespace
 {
 // schedule: kNumBins configuration ids (1..5) for the bins 65..80, ..., 241..256, or null
-// to take the autotuned schedule.
+// (orders above 64 by vbrows.hip).
 aclsolverStatus_t CreatePlan(aclsolverHandle_t handle, int batchSize, const int* nArray, int nrhs,
                              const int* schedule, aclsolverVbatchedPlan_t* plan)
 {
@@ -1247,16 +1067,26 @@ aclsolverStatus_t CreatePlan(aclsolverHandle_t handle, int batchSize, const int*
     p->nrhs = nrhs;
     (void)hipGetDevice(&p->device);
     p->grid = H(handle)->numCUs;
-    hipStream_t s = Stream(handle);
     hipError_t e = hipSuccess;
-    if (schedule != nullptr)
-        std::copy(schedule, schedule + kNumBins, p->schedule);
-    else
-        e = Autotune(p->device, p->grid, kNrhsMax, p->schedule, s);
+    // Without a schedule of the caller's the orders above 64 take vbrows.hip's kernels, and the
+    // schedule reported is the first configuration that fits each bin.
+    for (int b = 0; b < kNumBins; ++b)
+    {
+        const int top = 64 + kBinW * (b + 1);
+        p->schedule[b] = schedule != nullptr ? schedule[b] : (top <= 128 ? kC2x4 : (top <= 192 ? kC3x8 : kC4x16));
+    }
     std::vector<int> order(batchSize);
     for (int i = 0; i < batchSize; ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ns[x] > ns[y]; });
-    const std::vector<Item> items = BuildItems(ns, order, p->schedule);
+    int first = 0;
+    if (schedule == nullptr)
+        for (int c = 0; c < 3; ++c)
+        {
+            p->rowsFirst[c] = first;
+            while (first < batchSize && ns[order[first]] > 64 * (3 - c)) ++first;
+            p->rowsCount[c] = first - p->rowsFirst[c];
+        }
+    const std::vector<Item> items = BuildItems(ns, order, first, p->schedule);
     std::vector<long long> pivOff(batchSize + 1, 0);
     for (int i = 0; i < batchSize; ++i)
     {
