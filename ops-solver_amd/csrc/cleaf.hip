@@ -65,6 +65,7 @@ __device__ inline unsigned CyclicMaxU32(unsigned v)
 template <int NW, bool MULTI, bool SPREAD>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MULTI && !SPREAD && NW == 4 ? 1 : 2))) void cpanel_leaf_kernel(CLeafArgs p)
 {
+    __builtin_amdgcn_s_setprio(3);  // before the trailing product's waves on the same SIMD
     constexpr int T = 64 * NW, W = kCLeafWidth;
     constexpr int US = W + 28;
     __shared__ uint2 s_key[2][NW];
@@ -616,6 +617,7 @@ __global__ __launch_bounds__(256) void cleaf_finish_kernel(float2* __restrict__ 
                                                            const int* __restrict__ err, float* __restrict__ linv,
                                                            float2* __restrict__ ub)
 {
+    __builtin_amdgcn_s_setprio(3);  // before the trailing product's waves on the same SIMD
     constexpr int W = kCLeafWidth;
     __shared__ __align__(16) float s_l[2 * kC];  // the block, then its inverse
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -706,6 +708,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     float2* __restrict__ A, int64_t lda, int m, int c0, int hi, const float* __restrict__ linv,
     const float2* __restrict__ ub)
 {
+    __builtin_amdgcn_s_setprio(3);  // before the trailing product's waves on the same SIMD
     constexpr int W = kCLeafWidth;
     constexpr int BS = W + 4;
     __shared__ __align__(16) float s_r[W * BS], s_i[W * BS];  // [column][row] of B, then of U

@@ -93,15 +93,17 @@ __global__ __launch_bounds__(256) void couter_swap_kernel(float2* __restrict__ A
 }
 
 // C (MxN) -= op(A) (MxK) * B (KxN), complex64, four real FP32 MFMA products per block; op(A):
-// transA 0 = A, 1 = A^T, 2 = A^H. Tiles of 64 Q x 64 Q per workgroup, 32 Q x 32 Q per wave, k
-// chunks of 16 staged through LDS (parts apart) with the next chunk prefetched into registers;
-// formed as C^T, so that an accumulator register holds 32 consecutive rows of C.
+// transA 0 = A, 1 = A^T, 2 = A^H. Tiles of 64 Q x 64 Q per workgroup of 4 Q waves, 32 Q x 32 per
+// wave, k chunks of 16 staged through LDS (parts apart) with the next chunk prefetched into
+// registers; formed as C^T, so that an accumulator register holds 32 consecutive rows of C. Bound
+// by the matrix cores and, beside a panel, by what the panel takes: 78 to 82 TF at 7680 x 7168 x 512
+// (64 x 64 tiles without prefetch before: 67).
 template <int TRANSA, int Q>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void cgemm_sub_kernel(
+__global__ __launch_bounds__(256 * Q) __attribute__((amdgpu_waves_per_eu(4))) void cgemm_sub_kernel(
     int M, int N, int K, const float2* __restrict__ A, int64_t lda, const float2* __restrict__ B, int64_t ldb,
     float2* __restrict__ C, int64_t ldc, int tilesM, int tilesN)
 {
-    constexpr int KC = 16, TS = 64 * Q, E = 4 * Q;
+    constexpr int KC = 16, TS = 64 * Q, E = 4;
     __shared__ float Ar[2][KC][TS + 4], Ai[2][KC][TS + 4], Br[2][KC][TS + 4], Bi[2][KC][TS + 4];
     int id = blockIdx.x;
     const int total = tilesM * tilesN;
@@ -109,14 +111,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     if (total >= 64) id = id < (total & ~7) ? (id & 7) * (total >> 3) + (id >> 3) : id;
     const int row0 = id % tilesM * TS, col0 = id / tilesM * TS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave & 1) * 32 * Q + (lane & 31), wn = (wave >> 1) * 32 * Q + (lane & 31), lk = lane >> 5;
-    f32x16 accR[Q][Q], accI[Q][Q];
+    const int wm = (wave & 1) * 32 * Q + (lane & 31), wn = (wave >> 1) * 32 + (lane & 31), lk = lane >> 5;
+    f32x16 accR[Q], accI[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i)
 #pragma unroll
-        for (int j = 0; j < Q; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) accR[i][j][v] = accI[i][j][v] = 0.0f;
+        for (int v = 0; v < 16; ++v) accR[i][v] = accI[i][v] = 0.0f;
     // Rows and columns beyond the edge repeat the last one: their products are not stored. Sixteen
     // lanes read the 128 bytes of a chunk of one column of B (of one row of op(A) when
     // transposed), so that a line is fetched by one load, not by eight.
@@ -138,8 +138,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
             rb[q] = *pb;
             if (ka >= K) ra[q] = make_float2(0.0f, 0.0f);
             if (kb >= K) rb[q] = make_float2(0.0f, 0.0f);
-            if (TRANSA) pa += row0 + ar + 16 * (q + 1) < M ? 16 * lda : 0;
-            pb += col0 + bj + 16 * (q + 1) < N ? 16 * ldb : 0;
+            if (TRANSA) pa += row0 + ar + 16 * Q * (q + 1) < M ? 16 * Q * lda : 0;
+            pb += col0 + bj + 16 * Q * (q + 1) < N ? 16 * Q * ldb : 0;
         }
     };
     auto lstore = [&](int buf)
@@ -147,11 +147,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
         for (int q = 0; q < E; ++q)
         {
-            const int k = TRANSA ? ak : ak + q, r = TRANSA ? ar + 16 * q : ar;
+            const int k = TRANSA ? ak : ak + q, r = TRANSA ? ar + 16 * Q * q : ar;
             Ar[buf][k][r] = ra[q].x;
             Ai[buf][k][r] = TRANSA == 2 ? -ra[q].y : ra[q].y;
-            Br[buf][bk][bj + 16 * q] = rb[q].x;
-            Bi[buf][bk][bj + 16 * q] = rb[q].y;
+            Br[buf][bk][bj + 16 * Q * q] = rb[q].x;
+            Bi[buf][bk][bj + 16 * Q * q] = rb[q].y;
         }
     };
     const int chunks = (K + KC - 1) / KC;
@@ -165,53 +165,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 #pragma unroll
         for (int kk = 0; kk < KC; kk += 2)
         {
-            float xr[Q], xi[Q], yr[Q], yi[Q];
+            const float yr = Br[buf][kk + lk][wn], yi = Bi[buf][kk + lk][wn];
+            float xr[Q], xi[Q];
 #pragma unroll
             for (int i = 0; i < Q; ++i)
             {
                 xr[i] = Ar[buf][kk + lk][wm + 32 * i];
                 xi[i] = Ai[buf][kk + lk][wm + 32 * i];
-                yr[i] = Br[buf][kk + lk][wn + 32 * i];
-                yi[i] = Bi[buf][kk + lk][wn + 32 * i];
             }
 #pragma unroll
             for (int i = 0; i < Q; ++i)
-#pragma unroll
-                for (int j = 0; j < Q; ++j)
-                {
-                    accR[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(yr[j], xr[i], accR[i][j], 0, 0, 0);
-                    accI[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(yi[j], xr[i], accI[i][j], 0, 0, 0);
-                }
+            {
+                accR[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(yr, xr[i], accR[i], 0, 0, 0);
+                accI[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(yi, xr[i], accI[i], 0, 0, 0);
+            }
 #pragma unroll
             for (int i = 0; i < Q; ++i)
-#pragma unroll
-                for (int j = 0; j < Q; ++j)
-                {
-                    accR[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(-yi[j], xi[i], accR[i][j], 0, 0, 0);
-                    accI[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(yr[j], xi[i], accI[i][j], 0, 0, 0);
-                }
+            {
+                accR[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(-yi, xi[i], accR[i], 0, 0, 0);
+                accI[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(yr, xi[i], accI[i], 0, 0, 0);
+            }
         }
         if (c + 1 < chunks) lstore(buf ^ 1);
         __syncthreads();
     }
-    // All loads of a 32 x 32 tile before its first store (a load under its own condition waits by
-    // itself: 128 trips in a row took longer than the product of 512 columns).
+    // Loads before stores, eight at a time (a load under its own condition waits by itself).
 #pragma unroll
     for (int bi = 0; bi < Q; ++bi)
 #pragma unroll
-        for (int bc = 0; bc < Q; ++bc)
+        for (int h = 0; h < 2; ++h)
         {
-            const int i = row0 + wm + 32 * bi, j0 = col0 + (wave >> 1) * 32 * Q + bc * 32 + 4 * lk;
-            float2 x[16];
+            const int i = row0 + wm + 32 * bi, j0 = col0 + (wave >> 1) * 32 + 4 * lk + 16 * h;
+            float2 x[8];
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
+            for (int v = 0; v < 8; ++v)
                 x[v] = C[static_cast<int64_t>(min(j0 + (v & 3) + 8 * (v >> 2), N - 1)) * ldc + min(i, M - 1)];
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
+            for (int v = 0; v < 8; ++v)
             {
                 const int j = j0 + (v & 3) + 8 * (v >> 2);
                 if (i < M && j < N)
-                    C[j * ldc + i] = make_float2(x[v].x - accR[bi][bc][v], x[v].y - accI[bi][bc][v]);
+                    C[j * ldc + i] = make_float2(x[v].x - accR[bi][8 * h + v], x[v].y - accI[bi][8 * h + v]);
             }
         }
 }
@@ -289,9 +283,14 @@ hipError_t LaunchCGemm(int M, int N, int K, const float2* A, int lda, int transA
 {
     const int tilesM = (M + 64 * Q - 1) / (64 * Q), tilesN = (N + 64 * Q - 1) / (64 * Q);
     const dim3 grid(tilesM * tilesN);
-#define CG_CASE(TR)                                                                                                  \
-    hipLaunchKernelGGL((cgemm_sub_kernel<TR, Q>), grid, dim3(256), 0, stream, M, N, K, A, static_cast<int64_t>(lda), \
-                       B, static_cast<int64_t>(ldb), C, static_cast<int64_t>(ldc), tilesM, tilesN)
+    // LDS for one workgroup of the large tiles per compute unit: with its 128 registers a lane on
+    // eight waves the other half of the registers stays free for the panel beside it, whose leaves
+    // otherwise wait for a tile to end (n = 8192: 37.9 ms with two workgroups of four waves, 37.2).
+    const int pad = Q == 2 ? 16384 : 0;
+#define CG_CASE(TR)                                                                                           \
+    hipLaunchKernelGGL((cgemm_sub_kernel<TR, Q>), grid, dim3(256 * Q), pad, stream, M, N, K, A,               \
+                       static_cast<int64_t>(lda), B, static_cast<int64_t>(ldb), C, static_cast<int64_t>(ldc), \
+                       tilesM, tilesN)
     if (transA == 0)
         CG_CASE(0);
     else if (transA == 1)
@@ -307,6 +306,7 @@ hipError_t CGemmSub(int M, int N, int K, const float2* A, int lda, int transA, c
 {
     if (M <= 0 || N <= 0 || K <= 0) return hipSuccess;
     const int64_t big = static_cast<int64_t>((M + 127) / 128) * ((N + 127) / 128);
+    // At least a tile per compute unit: below, the small tiles spread the work further.
     if (big >= 256) return LaunchCGemm<2>(M, N, K, A, lda, transA, B, ldb, C, ldc, stream);
     return LaunchCGemm<1>(M, N, K, A, lda, transA, B, ldb, C, ldc, stream);
 }

@@ -23,9 +23,9 @@
 // What bounds it: the latency of the chain, one column about 0.35 us on one workgroup (24 us
 // of 64 columns) and 1.2 us over several (two trips through the XCD's L2 included), far from
 // any rate of the chip. Eight columns per block: the block's own columns cost up to seven
-// FMAs per row on the chain and the exchanged pivot row stays at eight words; the rolled
-// block loop (about 1500 instructions) stays in the instruction cache, where the unrolled
-// column loop it replaces (about 17000, each fetched once) waited for its instructions. 64
+// FMAs per row on the chain and the exchanged pivot row stays at eight words. A wave issues about
+// one instruction in five clocks here, so their number is the time: about 190 a column, where
+// the unrolled leaf this replaces had 265 and passed whole pivot rows through LDS. 64
 // columns, alone on the GPU, before and after: 64 rows 56 -> 26 us, 512 rows 104 -> 48 us,
 // 1024 rows 104 -> 66 us, 2048 rows 158 -> 89 us, 8192 rows 125 -> 92 us.
 #include "leaf.h"
