@@ -158,6 +158,13 @@ inline int TilesPerXcd(int tilesM, int tilesN)
     return tilesN < kXcds ? (tilesM * tilesN + kXcds - 1) / kXcds : tilesM * ((tilesN + kXcds - 1) / kXcds);
 }
 
+// Dynamic LDS of the three-part product: with it two workgroups instead of three share a compute
+// unit, and 208 of the 512 registers stay free, enough for a wave of the tall leaves (164), which
+// otherwise wait for the whole product (the second leaf of a panel 1.3 ms at order 16384). SB at
+// 16384: 67.3 ms without, 64.2 with two workgroups, 65.2 with one; the two-part product (SH 4700:
+// 11.50, 11.58) does not run long enough.
+constexpr int kPanelRoom = 8192;
+
 // One workgroup (4 waves) per 128 x 128 tile of C; wave (wm, wn) owns the 64 x 64
 // quadrant rows [wm*64, +64), columns [wn*64, +64) as 2 x 2 accumulators of 32 x 32.
 template <typename ET, int PARTS>
@@ -347,7 +354,7 @@ hipError_t GemmSubPacked(int M, int N, int K, const float* A, int lda, const flo
                        p.KB, fb, SB, static_cast<Mfma<ET>::vec*>(bp));                                            \
     {                                                                                                               \
         ProfileScope prof(ProfileKernel::TrailingGemm, 2.0 * M * N * K, stream);                                    \
-        hipLaunchKernelGGL((gemm_packed_kernel<ET, P>), grid, dim3(256), 0, stream, M, N, p.KB,                     \
+        hipLaunchKernelGGL((gemm_packed_kernel<ET, P>), grid, dim3(256), P == 3 ? kPanelRoom : 0, stream, M, N, p.KB, \
                            static_cast<const Mfma<ET>::vec*>(ap), static_cast<const Mfma<ET>::vec*>(bp), C, ldc,    \
                            tilesM, tilesN, SA, SB);                                                                 \
     }
