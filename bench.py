@@ -496,10 +496,7 @@ def uneven_batched(A, torch, h, steps=5):
         if step:
             ms_total += ev0.elapsed_time(ev1)
     ms = ms_total / steps
-    sched = np.zeros(12, np.int32)
-    assert L.aclsolverSgesvVbatched_getSchedule(plan, sched.ctypes.data) == A.SUCCESS
     L.aclsolverSgesvVbatched_destroyPlan(plan)
-    cfg_names = {1: "C2x4", 2: "C2x8", 3: "C3x8", 4: "C3x16", 5: "C4x16"}
     n = sizes.astype(np.float64)
     bytes_ = float(np.sum((2 * n * n + 2 * n * nrhs) * 4 + n * 4 + 4))
     flops = float(np.sum(2.0 / 3.0 * n ** 3 + 2 * n * n * nrhs))
@@ -515,7 +512,6 @@ def uneven_batched(A, torch, h, steps=5):
     return {"workload": "20000 FP32 systems, n_i ~ U{8..256}, A_i = N(0,1)/sqrt(n_i) + 2I, 4 RHS; getrf+getrs "
                         "through one plan, one launch per size class: n<=64 one wave per system, 65..256 one "
                         "workgroup of 2 to 4 waves per system",
-            "schedule": {f"{65 + 16 * b}..{80 + 16 * b}": cfg_names.get(int(c), str(int(c))) for b, c in enumerate(sched)},
             "ms": round(ms, 4), "solves_per_s": round(count / ms * 1e3, 1),
             "GB_per_s": round(bytes_ / ms / 1e6, 1), "hbm_frac": round(bytes_ / (ms * 1e-3) / PEAK_HBM, 4),
             "GFLOP_per_s": round(flops / ms / 1e6, 1), "max_backward_error_sample": worst,
@@ -622,8 +618,7 @@ def main():
         "panel_leaf": {"bound": "latency (sequential columns); HBM shown for scale",
                        "kernel": ("tournament-pivoting panel leaves (tree + apply launches, 32 columns each)"
                                   if args.tournament else
-                                  "partial-pivoting panel leaves (leaf_multi_kernel / leaf_getf2_kernel, one "
-                                  "launch per leaf of the recursive panel)"),
+                                  "partial-pivoting panel leaves (panel_leaf_kernel, one launch per 64 columns)"),
                        "launches": leaves, "ms_total": round(leaf_ms, 3),
                        "avg_launch_ms": round(leaf_ms / max(leaves, 1), 4),
                        "achieved": round(leaf_bytes / max(leaf_ms * 1e-3, 1e-12) / 1e9, 1), "peak": PEAK_HBM / 1e9,
