@@ -20,6 +20,7 @@ namespace ops
 {
 namespace
 {
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -609,86 +610,74 @@ __global__ __launch_bounds__(256) void trtri_unit_lower64_kernel(int K, const fl
 }
 
 // B <- T^{-1} B for unit-lower T (K x K, K <= 512) from the block inverses of
-// trtri_unit_lower64_kernel: one workgroup per 32-column strip of B, held in LDS; per
-// 64-row block b: X_b = inv(T_bb) B_b, then B_below -= T(below, b) X_b, both on FP32 MFMA
-// (32x32x2 tiles formed as products^T so that each accumulator lane holds one row).
+// trtri_unit_lower64_kernel or leaf_finish_kernel: one workgroup of eight waves per 16-column strip
+// of B, held in LDS; per 64-row block b: X_b = inv(T_bb) B_b (waves 0..3, 16 rows each), then
+// B_below -= T(below, b) X_b in tiles of 16 rows, both on FP32 MFMA (16x16x4 tiles formed as
+// products^T so that each accumulator lane holds one row). A panel's next block column has 512
+// columns: 16 wide it spreads over 32 workgroups, with a chain per block half as long (512 x 512
+// alone 85 us with 32 columns and four waves, 34 us now; beside the product of order 16384 145 and
+// 88 us on average).
 constexpr int kTrsmLuMaxK = 512;
-__global__ __launch_bounds__(256) void trsm_lu_kernel(int K, int N, const float* __restrict__ T, int ldt,
-                                                      const float* __restrict__ Linv, float* __restrict__ B, int ldb)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void trsm_lu_kernel(
+    int K, int N, const float* __restrict__ T, int64_t ldt, const float* __restrict__ Linv, float* __restrict__ B,
+    int64_t ldb)
 {
-    __shared__ float Xs[kTrsmLuMaxK][33];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c0 = blockIdx.x * 32, nc = min(32, N - c0);
-    const int Kp = (K + 63) & ~63;
-    for (int e = tid; e < 32 * Kp; e += 256)
-    {
-        const int c = e / Kp, r = e - c * Kp;
-        Xs[r][c] = (c < nc && r < K) ? B[static_cast<size_t>(c0 + c) * ldb + r] : 0.0f;
-    }
+    __shared__ float Xs[kTrsmLuMaxK][17];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ui = lane & 15, uk = lane >> 4;
+    const int nblk = (K + 63) / 64, Kp = nblk * 64;
+    const int c0 = static_cast<int>(blockIdx.x) * 16, nc = min(16, N - c0);
+    for (int c = wave; c < 16; c += 8)
+        for (int r = lane; r < Kp; r += 64) Xs[r][c] = c < nc && r < K ? B[(c0 + c) * ldb + r] : 0.0f;
     __syncthreads();
-    const int li = lane & 31, lk = lane >> 5;
-    const int nblk = Kp / 64;
-    // Operand fragments are loaded for a whole 32-row tile before its 32 MFMAs, so each tile
-    // waits for global memory once; the first tile below the block is fetched before the
-    // block's own product.
-    float lf[32];
-    auto loadTile = [&](int k0, int k1, int r0)
+    // A tile's operand is loaded whole before its MFMAs, the first one of a block before the block's
+    // own product. Blocks with rows below them are full; rows beyond K repeat the last one.
+    float lf[16];
+    auto loadTile = [&](int k0, int r0)
     {
-        const int row = r0 + li;
-        const float* Lc = T + static_cast<size_t>(k0) * ldt + row;
+        const float* const Lc = T + k0 * ldt + min(r0 + ui, K - 1);
 #pragma unroll
-        for (int t = 0; t < 32; ++t)
-        {
-            const int k = 2 * t + lk;
-            lf[t] = (row < K && k0 + k < k1) ? Lc[static_cast<size_t>(k) * ldt] : 0.0f;
-        }
+        for (int t = 0; t < 16; ++t) lf[t] = Lc[(4 * t + uk) * ldt];
     };
     for (int b = 0; b < nblk; ++b)
     {
-        const int k0 = b * 64, k1 = min(K, k0 + 64);
-        float lb[32];
-        if (wave < 2)
+        const int k0 = b * 64;
+        int r0 = k0 + 64 + wave * 16;
+        if (r0 < K) loadTile(k0, r0);
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (wave < 4)
         {
-            const float* Lb = Linv + static_cast<size_t>(b) * 4096 + wave * 32 + li;
+            const float* const Lb = Linv + static_cast<size_t>(b) * 4096 + 16 * wave + ui;
+            float lb[16];
 #pragma unroll
-            for (int t = 0; t < 32; ++t) lb[t] = Lb[(2 * t + lk) * 64];
+            for (int t = 0; t < 16; ++t) lb[t] = Lb[(4 * t + uk) * 64];
+#pragma unroll
+            for (int t = 0; t < 16; ++t)
+                if (t < 4 * (wave + 1))  // uniform: beyond lie the triangle's zeros
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[k0 + 4 * t + uk][ui], lb[t], acc, 0, 0, 0);
         }
-        int r0 = k1 + wave * 32;
-        if (r0 < K) loadTile(k0, k1, r0);
-        // X_b = inv(T_bb) B_b: waves 0 and 1 take 32 rows each.
-        f32x16 acc;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-        if (wave < 2)
-#pragma unroll
-            for (int t = 0; t < 32; ++t)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Xs[k0 + 2 * t + lk][li], lb[t], acc, 0, 0, 0);
         __syncthreads();
-        if (wave < 2)
+        if (wave < 4)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) Xs[k0 + wave * 32 + li][(v & 3) + 8 * (v >> 2) + 4 * lk] = acc[v];
+            for (int v = 0; v < 4; ++v) Xs[k0 + 16 * wave + ui][4 * uk + v] = acc[v];
         __syncthreads();
-        // Rows below the block: 32-row tiles dealt to the four waves.
         for (; r0 < K; r0 += 128)
         {
+            acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 32; ++t)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Xs[k0 + 2 * t + lk][li], lf[t], acc, 0, 0, 0);
-            const int row = r0 + li;
-            if (r0 + 128 < K) loadTile(k0, k1, r0 + 128);
+            for (int t = 0; t < 16; ++t)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[k0 + 4 * t + uk][ui], lf[t], acc, 0, 0, 0);
+            const int row = r0 + ui;
+            if (r0 + 128 < K) loadTile(k0, r0 + 128);
             if (row < K)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) Xs[row][(v & 3) + 8 * (v >> 2) + 4 * lk] -= acc[v];
+                for (int v = 0; v < 4; ++v) Xs[row][4 * uk + v] -= acc[v];
         }
         __syncthreads();
     }
-    for (int e = tid; e < 32 * Kp; e += 256)
-    {
-        const int c = e / Kp, r = e - c * Kp;
-        if (c < nc && r < K) B[static_cast<size_t>(c0 + c) * ldb + r] = Xs[r][c];
-    }
+    for (int c = wave; c < nc; c += 8)
+        for (int r = lane; r < K; r += 64) B[(c0 + c) * ldb + r] = Xs[r][c];
 }
 
 hipError_t TrsmDiag(int kb, int N, const float* T, int ldt, bool fwd, bool unit, bool transT, float* B, int ldb,
@@ -775,7 +764,8 @@ hipError_t TrsmLowerUnitApply(int K, int N, const float* T, int ldt, const float
 {
     if (K <= 0 || N <= 0) return hipSuccess;
     if (K > kTrsmLuMaxK) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(trsm_lu_kernel, dim3((N + 31) / 32), dim3(256), 0, stream, K, N, T, ldt, linv, B, ldb);
+    hipLaunchKernelGGL(trsm_lu_kernel, dim3((N + 15) / 16), dim3(512), 0, stream, K, N, T, static_cast<int64_t>(ldt),
+                       linv, B, static_cast<int64_t>(ldb));
     return hipGetLastError();
 }
 
