@@ -27,6 +27,7 @@
 #include <cstdlib>
 
 #include "internal.h"
+#include "wave.h"
 
 namespace ops
 {
@@ -181,6 +182,19 @@ __global__ __launch_bounds__(256) void matinv_gj_kernel(int n, const float* cons
     if (live && lane == 0) info[mat] = zero;
 }
 
+// Maximum over each aligned group of NL (8 or 16) lanes, left in all of them.
+template <int NL>
+__device__ inline unsigned RowGroupMax(unsigned v)
+{
+    static_assert(NL == 8 || NL == 16, "groups within a row of 16 lanes");
+    auto mx = [](unsigned a, unsigned b) { return a > b ? a : b; };
+    v = mx(v, DppU32<0xB1>(v));   // quad_perm [1,0,3,2]
+    v = mx(v, DppU32<0x4E>(v));   // quad_perm [2,3,0,1]
+    v = mx(v, DppU32<0x141>(v));  // row_half_mirror
+    if (NL == 16) v = mx(v, DppU32<0x140>(v));  // row_mirror
+    return v;
+}
+
 // The same Gauss-Jordan inverse with R rows per lane: NL lanes own one matrix (n <= NL*R),
 // lane l holding rows l*R .. l*R+R-1, so a wave carries 64/NL matrices and each pivot step's
 // search, broadcast and reciprocal are shared by R rows of multiply-adds. Pivot keys,
@@ -196,6 +210,7 @@ __global__ __launch_bounds__(256) void matinv_gj_rows_kernel(int n, const float*
     constexpr int GROUPS = 256 / NL;
     __shared__ __attribute__((aligned(16))) float s_row[GROUPS][N];
     __shared__ int s_inv[GROUPS][N];
+    __shared__ int s_ppos[GROUPS];
     const int tid = threadIdx.x;
     const int g = tid / NL, lane = tid % NL;
     const int mat = blockIdx.x * GROUPS + g;
@@ -228,38 +243,56 @@ __global__ __launch_bounds__(256) void matinv_gj_rows_kernel(int n, const float*
     for (int k = 0; k < N; ++k)
     {
         if (k >= n) continue;
-        unsigned long long best = 0ull;
-        int bi = -1;
+        // Magnitudes first, positions only on ties: 32-bit maxima are one DPP instruction a step.
+        unsigned bm = 0u;
+        int bi = 0, bp = pos[0];
 #pragma unroll
         for (int i = 0; i < R; ++i)
         {
-            const unsigned long long key =
-                (rowLive[i] && !used[i]) ? GjKey(S[i][k], (pos[i] << 8) | (lane * R + i), pos[i] == k) : 0ull;
-            bi = key > best ? i : bi;
-            best = key > best ? key : best;
+            const unsigned ab = __float_as_uint(S[i][k]) & 0x7fffffffu;
+            unsigned m = ab <= 0x7f800000u ? ab + 0x80000001u : (pos[i] == k ? 0xffffffffu : 0x80000000u);
+            m = rowLive[i] && !used[i] ? m : 0u;
+            const bool better = i > 0 && (m > bm || (m == bm && pos[i] < bp));
+            bm = i == 0 || better ? m : bm;
+            bp = better ? pos[i] : bp;
+            bi = better ? i : bi;
         }
-        const unsigned long long top = GroupMaxKey<NL>(best);
-        const int key = static_cast<int>(~static_cast<unsigned>(top & 0xffffffffull));
-        const int p = key & 0xFF;  // pivot row
-        const int ppos = key >> 8;
-        if (live && lane == 0 && ipivOut != nullptr) ipivOut[static_cast<int64_t>(mat) * n + k] = ppos + 1;
-        // LAPACK interchange of positions k and ppos.
-#pragma unroll
-        for (int i = 0; i < R; ++i)
+        const unsigned top = RowGroupMax<NL>(bm);
+        bool mine = bm == top && bm != 0u;
+        const unsigned long long hit = __ballot(mine);
+        const unsigned share = static_cast<unsigned>(hit >> (threadIdx.x & 63 & ~(NL - 1))) & ((1u << NL) - 1u);
+        if (__builtin_expect(__any(__popc(share) > 1), 0))  // uniform
         {
-            const bool isP = lane * R + i == p;
-            if (pos[i] == k) pos[i] = ppos;
-            if (isP) pos[i] = k;
+            const unsigned low = RowGroupMax<NL>(mine ? ~static_cast<unsigned>(bp) : 0u);
+            mine = mine && ~static_cast<unsigned>(bp) == low;
         }
-        // Broadcast the pivot row.
-        if (best == top && bi >= 0)
+        // Broadcast the pivot row and its position.
+        if (mine)
+        {
+            float x[N];
 #pragma unroll
-            for (int i = 0; i < R; ++i)
-                if (i == bi)
+            for (int j = 0; j < N; ++j)
+            {
+                x[j] = S[0][j];
 #pragma unroll
-                    for (int j = 0; j < N; ++j) s_row[g][j] = S[i][j];
+                for (int i = 1; i < R; ++i) x[j] = bi == i ? S[i][j] : x[j];
+            }
+#pragma unroll
+            for (int j = 0; j < N; ++j) s_row[g][j] = x[j];
+            s_ppos[g] = bp;
+        }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const int ppos = s_ppos[g];
+        if (live && lane == 0 && ipivOut != nullptr) ipivOut[static_cast<int64_t>(mat) * n + k] = ppos + 1;
+        // LAPACK interchange of positions k and ppos.
+        bool isPivot[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+        {
+            isPivot[i] = mine && bi == i;
+            pos[i] = isPivot[i] ? k : (pos[i] == k ? ppos : pos[i]);
+        }
         float u[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) u[j] = s_row[g][j];
@@ -269,7 +302,7 @@ __global__ __launch_bounds__(256) void matinv_gj_rows_kernel(int n, const float*
             if (zero == 0) zero = k + 1;
 #pragma unroll
             for (int i = 0; i < R; ++i)
-                if (lane * R + i == p) used[i] = true;
+                if (isPivot[i]) used[i] = true;
             __builtin_amdgcn_wave_barrier();
             continue;
         }
@@ -277,7 +310,7 @@ __global__ __launch_bounds__(256) void matinv_gj_rows_kernel(int n, const float*
 #pragma unroll
         for (int i = 0; i < R; ++i)
         {
-            const bool isP = lane * R + i == p;
+            const bool isP = isPivot[i];
             const float c = isP ? 0.0f : S[i][k] * rc;
 #pragma unroll
             for (int j = 0; j < N; ++j)
