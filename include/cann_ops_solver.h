@@ -185,9 +185,9 @@ extern "C"
      * matrix (n <= 128); 2 = 2 rows, 8 waves (n <= 128); 3 = 3 rows, 8 waves (n <= 192);
      * 4 = 3 rows, 16 waves (n <= 192); 5 = 4 rows, 16 waves (n <= 256). Orders <= 64 always
      * take one wave per matrix. createPlanWithSchedule takes the caller's (INVALID_VALUE for an
-     * id outside 1..5 or one whose largest order is below its bin's). createPlan needs none: orders
-     * above 64 take one workgroup of 2 to 4 waves per matrix. getSchedule reports a plan's (for
-     * createPlan's the first id that fits each bin). */
+     * id outside 1..5 or one whose largest order is below its bin's). createPlan has the first id
+     * that fits each bin, and where there are enough matrices of a class takes one workgroup of 2
+     * to 4 waves per matrix instead. getSchedule reports a plan's. */
     aclsolverStatus_t aclsolverSgesvVbatched_createPlanWithSchedule(aclsolverHandle_t handle, int batchSize,
                                                                     const int* nArray, int nrhs, const int* schedule,
                                                                     aclsolverVbatchedPlan_t* plan);

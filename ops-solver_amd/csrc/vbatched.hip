@@ -10,9 +10,10 @@
 //   C3x8  n <= 192: column-cyclic, 3 rows per lane, 8 waves per matrix, 2 per item;
 //   C3x16 n <= 192: column-cyclic, 3 rows per lane, 16 waves, 1 per item;
 //   C4x16 n <= 256: column-cyclic, 4 rows per lane, 16 waves, 1 per item.
-// Orders above 64 take vbrows.hip's kernels (one workgroup per matrix: outputs the same, 20000
-// systems of orders 1..256 in 4.8 instead of 8.2 ms) unless the plan's caller gives a schedule,
-// the configuration of each 16-wide size bin above 64: those go through the queue here.
+// Where there are enough of them, orders above 64 take vbrows.hip's kernels instead (one workgroup
+// per matrix: outputs the same, 20000 systems of orders 1..256 in 4.8 instead of 8.2 ms; the rule is
+// at CreatePlan). A plan's caller may give the configuration of each 16-wide size bin above 64:
+// then all go through the queue here.
 // The last workgroup to leave re-arms the queue, so the queue needs no reset between launches.
 //
 // Column-cyclic kernel (one matrix per workgroup): lane l of every wave holds rows
@@ -1012,16 +1013,17 @@ hipError_t VbatchedLaunch(VbatchedPlan* p, float* const* dA, float* const* dB, i
     return hipGetLastError();
 }
 
-// Items of the plan: matrices from order[first] on in decreasing order of n, each group of up to kCfgCap[cfg]
+// Items of the plan: matrices that `rows` does not take, in decreasing order of n, each group of up to kCfgCap[cfg]
 // consecutive matrices of one configuration an item (longest-processing-time order).
-static std::vector<Item> BuildItems(const std::vector<int>& ns, const std::vector<int>& order, int first,
-                                    const int* schedule)
+static std::vector<Item> BuildItems(const std::vector<int>& ns, const std::vector<int>& order,
+                                    const std::vector<char>& rows, const int* schedule)
 {
     std::vector<Item> items;
     Item open[kNumCfg];
     for (int c = 0; c < kNumCfg; ++c) open[c] = {0, 0, c, 0};
-    for (int i = first; i < static_cast<int>(order.size()); ++i)
+    for (int i = 0; i < static_cast<int>(order.size()); ++i)
     {
+        if (rows[i]) continue;
         const int n = ns[order[i]];
         const int c = n <= 64 ? kW64 : schedule[BinOf(n)];
         // Items hold consecutive entries of the order: start a new one when this
@@ -1047,7 +1049,7 @@ using namespace ops;
 namespace
 {
 // schedule: kNumBins configuration ids (1..5) for the bins 65..80, ..., 241..256, or null
-// (orders above 64 by vbrows.hip).
+// for the default ones (or vbrows.hip's kernels, by the rule below).
 aclsolverStatus_t CreatePlan(aclsolverHandle_t handle, int batchSize, const int* nArray, int nrhs,
                              const int* schedule, aclsolverVbatchedPlan_t* plan)
 {
@@ -1068,8 +1070,8 @@ aclsolverStatus_t CreatePlan(aclsolverHandle_t handle, int batchSize, const int*
     (void)hipGetDevice(&p->device);
     p->grid = H(handle)->numCUs;
     hipError_t e = hipSuccess;
-    // Without a schedule of the caller's the orders above 64 take vbrows.hip's kernels, and the
-    // schedule reported is the first configuration that fits each bin.
+    // Without a schedule of the caller's each bin has the first configuration that fits (65..128 four
+    // waves, 129..192 eight, above sixteen: also what timing each on a full device chose).
     for (int b = 0; b < kNumBins; ++b)
     {
         const int top = 64 + kBinW * (b + 1);
@@ -1078,15 +1080,32 @@ aclsolverStatus_t CreatePlan(aclsolverHandle_t handle, int batchSize, const int*
     std::vector<int> order(batchSize);
     for (int i = 0; i < batchSize; ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return ns[x] > ns[y]; });
-    int first = 0;
-    if (schedule == nullptr)
-        for (int c = 0; c < 3; ++c)
+    // The classes 193..256, 129..192 and 65..128 go to vbrows.hip where that is the faster: its
+    // workgroups come in rounds of 4, 5 and 8 a compute unit, a round takes 2.33, 2.16 and 1.75 us
+    // per order of its first matrix; an item of the queue 1.2 us per order, on the compute unit that
+    // is free. 250 systems of orders 20..200: 263 us through the queue, 882 otherwise; 1000 of
+    // 100..220: 642 and 775; 10000 of 10..120: 1010 and 843; 20000 of 1..256: 9.0 and 5.3 ms.
+    std::vector<char> rows(batchSize, 0);
+    const double perRound[3] = {2.33, 2.16, 1.75}, perItem = 1.2;
+    const int perUnit[3] = {4, 5, 8}, cap[3] = {kCfgCap[kC4x16], kCfgCap[kC3x8], kCfgCap[kC2x4]};
+    for (int c = 0, first = 0; schedule == nullptr && c < 3; ++c)
+    {
+        int last = first;
+        double byRows = 0.0, byQueue = 0.0;
+        for (; last < batchSize && ns[order[last]] > 64 * (3 - c); ++last)
+        {
+            if ((last - first) % (perUnit[c] * p->grid) == 0) byRows += perRound[c] * ns[order[last]];
+            if ((last - first) % cap[c] == 0) byQueue += perItem * ns[order[last]] / p->grid;
+        }
+        if (byRows < byQueue)
         {
             p->rowsFirst[c] = first;
-            while (first < batchSize && ns[order[first]] > 64 * (3 - c)) ++first;
-            p->rowsCount[c] = first - p->rowsFirst[c];
+            p->rowsCount[c] = last - first;
+            std::fill(rows.begin() + first, rows.begin() + last, 1);
         }
-    const std::vector<Item> items = BuildItems(ns, order, first, p->schedule);
+        first = last;
+    }
+    const std::vector<Item> items = BuildItems(ns, order, rows, p->schedule);
     std::vector<long long> pivOff(batchSize + 1, 0);
     for (int i = 0; i < batchSize; ++i)
     {
