@@ -85,8 +85,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MULTI &
     float2* const Ap = p.A + static_cast<int64_t>(c0) * lda + c0;
     const int lr = g * T + wid * 64 + lane;
     const bool valid = lr < mp;
-    // An earlier leaf of this factorization timed out: its factors are NaN already.
-    if (MULTI && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
     bool aborted = false;  // uniform over the workgroup
 
     f32x16 curR[2], curI[2], nxtR[2], nxtI[2];
@@ -133,8 +131,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MULTI &
         if (tid == 0) StoreWord(arrival + g, p.tagBase, SPREAD);
         if (wid == 0)
         {
+            // After a wait that ran out, here or in an earlier leaf: no more waits (leaf.hip).
+            const bool late = __any(__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
             bool all = false;
-            for (unsigned spins = 0; spins < p.spinLimit; ++spins)
+            for (unsigned spins = 0; spins < p.spinLimit && !late; ++spins)
             {
                 all = __all(lane >= P || LoadWord(arrival + lane) == p.tagBase);
                 if (all) break;

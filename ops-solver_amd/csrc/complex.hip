@@ -39,13 +39,15 @@ __global__ void cclear_slots_kernel(unsigned long long* slots, int words, int* e
     if (i == 0) *err = 0;
 }
 
+// The list of rows moved by a panel; empty after a wait that ran out (getrf.hip).
 __global__ __launch_bounds__(1024) void ccompact_moves_kernel(int m, int j0, const int* __restrict__ rowsrc,
-                                                              int* __restrict__ moved)
+                                                              const int* __restrict__ err, int* __restrict__ moved)
 {
     __shared__ int s_count;
     if (threadIdx.x == 0) s_count = 0;
     __syncthreads();
-    for (int r = j0 + threadIdx.x; r < m; r += blockDim.x)
+    const int hi = *err == 0 ? m : j0;
+    for (int r = j0 + threadIdx.x; r < hi; r += blockDim.x)
     {
         const int s = rowsrc[r];
         if (s != r)
@@ -488,7 +490,8 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
             if (c0 + l.wact < panelEnd) CRET(CPanelUpdate(l, linv, w.panelRows, s0));
         }
         if (pivoting && (k > 0 || panelEnd < n))
-            hipLaunchKernelGGL(ccompact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, w.moved[k & 1]);
+            hipLaunchKernelGGL(ccompact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, w.err,
+                               w.moved[k & 1]);
         return hipGetLastError();
     };
     // Applies panel k to the columns [lo, hi) (interchanges, U12 solve, trailing product)

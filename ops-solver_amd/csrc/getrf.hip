@@ -100,14 +100,17 @@ __global__ void clear_slots_kernel(unsigned long long* slots, int words, int* er
 }
 
 // Builds the list of rows moved by the whole panel (rowsrc[r] != r) and applies it to the
-// global permutation. One workgroup.
+// global permutation. One workgroup. After a wait that ran out (*err) the workgroups of a leaf
+// may disagree on the pivots, so that rowsrc need not be a permutation: the list is empty then.
 __global__ __launch_bounds__(1024) void compact_moves_kernel(int m, int j0, const int* __restrict__ rowsrc,
-                                                             int* __restrict__ moved, int* __restrict__ perm)
+                                                             const int* __restrict__ err, int* __restrict__ moved,
+                                                             int* __restrict__ perm)
 {
     __shared__ int s_count;
     if (threadIdx.x == 0) s_count = 0;
     __syncthreads();
-    for (int r = j0 + threadIdx.x; r < m; r += blockDim.x)
+    const int hi = *err == 0 ? m : j0;
+    for (int r = j0 + threadIdx.x; r < hi; r += blockDim.x)
     {
         const int s = rowsrc[r];
         if (s != r)
@@ -443,8 +446,8 @@ hipError_t RealGetrfPerm(int m, int n, float* a, int lda, int* ipiv, int* info, 
             RET_IF(Panel(a, lda, m, j0, j0 + nb, pivoting, ipiv, info, w, linv, s0));
         // The first panel's list serves the columns right of it and perm only.
         if (pivoting && (k > 0 || j0 + nb < n || permOut != nullptr))
-            hipLaunchKernelGGL(compact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, moved(k),
-                               permOut);
+            hipLaunchKernelGGL(compact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, w.err,
+                               moved(k), permOut);
         RET_IF(hipGetLastError());
         // The U12 solves of both streams use the block inverses of this panel's L11.
         if (!w.tournament) return hipSuccess;

@@ -111,8 +111,6 @@ void panel_leaf_kernel(LeafArgs p)
     const int64_t lda = p.lda;
     float* const Ap = p.A + static_cast<int64_t>(c0) * lda + c0;
     const int rbase = g * (T * RP) + wid * (64 * RP) + lane;
-    // An earlier leaf of this factorization timed out: its factors are NaN already.
-    if (MULTI && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
     bool aborted = false;  // uniform over the wave
 
     // cur: the 32-column chunk being factored, nxt the one right of it. Lane l of tile t holds
@@ -166,8 +164,12 @@ void panel_leaf_kernel(LeafArgs p)
         if (tid == 0) StoreWord(arrival + g, p.tagBase, SPREAD);
         if (wid == 0)
         {
+            // A wait of this factorization has run out already, in an earlier leaf or in a workgroup
+            // of this one that came before: no more waits, but NaN rows and a list of moves from
+            // every workgroup all the same.
+            const bool late = __any(__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
             bool all = false;
-            for (unsigned spins = 0; spins < p.spinLimit; ++spins)
+            for (unsigned spins = 0; spins < p.spinLimit && !late; ++spins)
             {
                 all = __all(lane >= P || LoadWord(arrival + lane) == p.tagBase);
                 if (all) break;

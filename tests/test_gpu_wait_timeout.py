@@ -1,0 +1,63 @@
+"""Cross-workgroup waits that run out (a poll budget of zero, set from the host, so that every
+kernel still exits): the interchange lists stay in range whatever the workspace held before, and
+memory around the arguments is left alone."""
+import contextlib
+import ctypes
+import os
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+for p in (ROOT, os.path.join(ROOT, "ops-solver_amd")):
+    if p not in sys.path:
+        sys.path.insert(0, p)
+
+import aclsolver as A  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+POISON = 0x7F7F7F7F  # as a row index far beyond any matrix
+
+
+@pytest.fixture(scope="module")
+def handle():
+    h = A.Handle()
+    yield h
+    h.close()
+
+
+@contextlib.contextmanager
+def no_polls():
+    assert A.lib().aclsolverDebugSetSpinLimit(0) == A.SUCCESS
+    try:
+        yield
+    finally:
+        A.lib().aclsolverDebugSetSpinLimit(A.DEFAULT_SPIN_LIMIT)
+
+
+@pytest.mark.parametrize("cplx,m,n", [(0, 1100, 1100), (0, 2304, 600), (0, 9000, 64), (1, 600, 600), (1, 9000, 64)])
+def test_factorization_with_a_poisoned_workspace(handle, cplx, m, n):
+    import torch
+
+    print(f"timeout cplx={cplx} m={m} n={n}", flush=True)
+    L, lda, guard = A.lib(), m + 5, 3
+    dt = torch.complex64 if cplx else torch.float32
+    a = torch.randn(n + guard, lda, dtype=dt, device="cuda")
+    before = a.clone()
+    lw = ctypes.c_int(0)
+    size, getrf = (L.aclsolverCgetrf_bufferSize, L.aclsolverCgetrf) if cplx else (L.aclsolverSgetrf_bufferSize, L.aclsolverSgetrf)
+    assert size(handle.h, m, n, A.ptr(a), lda, ctypes.byref(lw)) == A.SUCCESS
+    words = lw.value * (2 if cplx else 1)
+    work = torch.full((words + 4096,), POISON, dtype=torch.int32, device="cuda")
+    ipiv = torch.full((min(m, n),), POISON, dtype=torch.int32, device="cuda")
+    info = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+    with no_polls():
+        assert getrf(handle.h, m, n, A.ptr(a), lda, A.ptr(work), A.ptr(ipiv), A.ptr(info)) == A.SUCCESS
+        torch.cuda.synchronize()
+    assert info.item() == A.INFO_WAIT_TIMEOUT
+    piv = ipiv.cpu().numpy()
+    assert np.all((piv >= 1) & (piv <= m))
+    assert torch.isnan(torch.view_as_real(a[:64, :m]) if cplx else a[:64, :m]).all()
+    assert torch.equal(a[n:], before[n:]) and torch.equal(a[:, m:], before[:, m:])
+    assert bool((work[words:] == POISON).all())
