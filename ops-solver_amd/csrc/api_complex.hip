@@ -334,7 +334,7 @@ struct ComplexStagingRuntime
         float2* bCol = static_cast<float2*>(st.bCol);
         hipError_t e = CTransposeRM(n, n, aRow, lda, aCol, n, s);
         if (e == hipSuccess) e = CTransposeRM(n, nrhs, bRow, ldb, bCol, n, s);
-        if (e == hipSuccess) e = ComplexGetrs(trans, n, nrhs, aCol, n, st.piv, bCol, n, st.work, s, nullptr, true);
+        if (e == hipSuccess) e = ComplexGetrs(trans, n, nrhs, aCol, n, st.piv, bCol, n, st.work, s, st.wait, true);
         if (e == hipSuccess) e = CTransposeRM(nrhs, n, bCol, n, bRow, ldb, s);
         return e != hipSuccess;
     }

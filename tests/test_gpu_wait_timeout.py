@@ -61,3 +61,28 @@ def test_factorization_with_a_poisoned_workspace(handle, cplx, m, n):
     assert torch.isnan(torch.view_as_real(a[:64, :m]) if cplx else a[:64, :m]).all()
     assert torch.equal(a[n:], before[n:]) and torch.equal(a[:, m:], before[:, m:])
     assert bool((work[words:] == POISON).all())
+
+
+@pytest.mark.parametrize("cplx", [0, 1])
+@pytest.mark.parametrize("trans", [0, 1])
+def test_host_solve_reports_the_wait(handle, cplx, trans):
+    """Three blocks of 64 rows, so that a block waits for another; info stays as it was, as after
+    any failed step of the staging."""
+    print(f"host getrs cplx={cplx} trans={trans}", flush=True)
+    n = 150
+    a = np.eye(n, dtype=np.complex64 if cplx else np.float32) * 2
+    a[1:, 0] = 0.5
+    b = np.ones((n, 2), a.dtype)
+    piv = np.arange(1, n + 1, dtype=np.int32)
+    info = np.full(1, 7, np.int32)
+    getrs = A.lib().aclsolverCgetrs if cplx else A.lib().aclsolverSgetrs
+
+    def call():
+        return getrs(handle.h, trans, n, 2, a.ctypes.data, n, piv.ctypes.data, b.ctypes.data, 2, info.ctypes.data)
+
+    with no_polls():
+        assert call() != 0
+    assert info[0] == 7
+    b[:] = 1
+    assert call() == 0 and info[0] == 0
+    assert np.isfinite(b).all()
