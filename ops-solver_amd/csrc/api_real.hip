@@ -65,6 +65,7 @@ bool Fits(const void* p, size_t bytes, RangeCache* cache = nullptr)
     return off <= size && bytes <= size - off;
 }
 
+// Launched after the solve, whose report of a wait that ran out stays.
 __global__ void first_zero_diag_kernel(int n, const float* a, int lda, int* info)
 {
     __shared__ int s_first;
@@ -73,7 +74,7 @@ __global__ void first_zero_diag_kernel(int n, const float* a, int lda, int* info
     for (int k = threadIdx.x; k < n; k += blockDim.x)
         if (a[static_cast<size_t>(k) * lda + k] == 0.0f) atomicMin(&s_first, k);
     __syncthreads();
-    if (threadIdx.x == 0) *info = s_first == INT_MAX ? 0 : s_first + 1;
+    if (threadIdx.x == 0 && *info != kInfoWaitTimeout) *info = s_first == INT_MAX ? 0 : s_first + 1;
 }
 
 __global__ void set_identity_kernel(int n, float* x, int ldx)
@@ -84,9 +85,9 @@ __global__ void set_identity_kernel(int n, float* x, int ldx)
 }
 
 __global__ void copy_matrix_kernel(int rows, int cols, const float* src, int lds, float* dst, int ldd,
-                                   const int* skipIfInfo)
+                                   const int* skipIfZeroPivot)
 {
-    if (skipIfInfo != nullptr && *skipIfInfo != 0) return;
+    if (skipIfZeroPivot != nullptr && *skipIfZeroPivot > 0) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     int c = blockIdx.y;
     if (i < rows && c < cols) dst[static_cast<size_t>(c) * ldd + i] = src[static_cast<size_t>(c) * lds + i];
@@ -438,9 +439,9 @@ OPS_API aclsolverStatus_t aclsolverSgetri(aclsolverHandle_t handle, int n, float
     if (RealGetrsWorkspaceBytes(n, n) > RealGetrsStagingBytes(n, n))
         work = HandleScratch(handle, RealGetrsWorkspaceBytes(n, n));
     if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
-    hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, A, lda, devInfo);
     hipLaunchKernelGGL(set_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, X, n);
-    if (RealGetrs(0, n, n, A, lda, devIpiv, X, n, work, s) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
+    if (RealGetrs(0, n, n, A, lda, devIpiv, X, n, work, s, devInfo) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
+    hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, A, lda, devInfo);
     hipLaunchKernelGGL(copy_matrix_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, n, X, n, A, lda, devInfo);
     return Launched();
 }
@@ -525,11 +526,11 @@ OPS_API aclsolverStatus_t aclsolverSgetriBatched(aclsolverHandle_t handle, int n
     {
         const float* a = reinterpret_cast<const float*>(in[b]);
         float* c = reinterpret_cast<float*>(out[b]);
-        hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, a, lda, infoArray + b);
         hipLaunchKernelGGL(set_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, c, ldc);
         if (RealGetrs(0, n, n, a, lda, PivotArray ? PivotArray + static_cast<size_t>(b) * n : nullptr, c, ldc, work,
-                      s) != hipSuccess)
+                      s, infoArray + b) != hipSuccess)
             return ACLSOLVER_STATUS_EXECUTION_FAILED;
+        hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, a, lda, infoArray + b);
     }
     return Launched();
 }

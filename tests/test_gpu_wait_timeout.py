@@ -86,3 +86,58 @@ def test_host_solve_reports_the_wait(handle, cplx, trans):
     b[:] = 1
     assert call() == 0 and info[0] == 0
     assert np.isfinite(b).all()
+
+
+def _diagonal(n, cplx=False):
+    """Factors of 2 I with a nonzero first column of L: every block of rows waits for the first."""
+    a = np.eye(n, dtype=np.complex64 if cplx else np.float32) * 2
+    a[1:, 0] = 0.5
+    return a
+
+
+def test_getri_reports_the_wait(handle):
+    import torch
+
+    n = 150
+    lu = A.to_device_cm(_diagonal(n))
+    lw = ctypes.c_int(0)
+    assert A.lib().aclsolverSgetri_bufferSize(handle.h, n, A.ptr(lu), n, ctypes.byref(lw)) == A.SUCCESS
+    work = torch.zeros(lw.value, device="cuda")
+    info = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+
+    def call(a):
+        st = A.lib().aclsolverSgetri(handle.h, n, A.ptr(a), n, None, A.ptr(work), lw.value, A.ptr(info))
+        torch.cuda.synchronize()
+        return st, info.item()
+
+    with no_polls():
+        a = lu.clone()
+        assert call(a) == (A.SUCCESS, A.INFO_WAIT_TIMEOUT)
+        assert torch.isnan(a).any()
+    assert call(lu.clone()) == (A.SUCCESS, 0)
+    singular = lu.clone()
+    singular[99, 99] = 0  # the factors stay, as before
+    before = singular.clone()
+    assert call(singular) == (A.SUCCESS, 100) and torch.equal(singular, before)
+
+
+@pytest.mark.parametrize("cplx,n", [(0, 600), (1, 150)])
+def test_getri_batched_reports_the_wait(handle, cplx, n):
+    import torch
+
+    print(f"getri_batched cplx={cplx} n={n}", flush=True)
+    a = torch.stack([A.to_device_cm(_diagonal(n, cplx))] * 3)
+    a[1, 70, 70] = 0
+    c = torch.zeros_like(a)
+    pa, pc = (torch.tensor([t[k].data_ptr() for k in range(3)], dtype=torch.int64, device="cuda") for t in (a, c))
+    info = torch.full((3,), 7, dtype=torch.int32, device="cuda")
+    getri = A.lib().aclsolverCgetriBatched if cplx else A.lib().aclsolverSgetriBatched
+
+    def call():
+        st = getri(handle.h, n, A.ptr(pa), n, None, A.ptr(pc), n, A.ptr(info), 3)
+        torch.cuda.synchronize()
+        return st, info.tolist()
+
+    with no_polls():
+        assert call() == (A.SUCCESS, [A.INFO_WAIT_TIMEOUT] * 3)
+    assert call() == (A.SUCCESS, [0, 71, 0])
