@@ -380,9 +380,14 @@ OPS_API aclError aclsolverSgetrs(aclsolverHandle_t handle, const uint64_t trans,
 // ---------------------------------------------------------------------------------------
 // sgetri (in place, from LU): X = A^-1 solved from the factors on the identity.
 // ---------------------------------------------------------------------------------------
-static size_t GetriWorkBytes(int n)
+// X and, behind it, what the solve uses: all of the call's device memory is the caller's, so that
+// calls on one handle with streams and workspaces of their own do not meet. chain: for the
+// chained solve, which the query reports; a workspace that is too small for it but has the
+// staging size still does with the blocked solve.
+static size_t GetriWorkBytes(int n, bool chain)
 {
-    return static_cast<size_t>(n) * n * sizeof(float) + RealGetrsStagingBytes(n, n) + 256;
+    return static_cast<size_t>(n) * n * sizeof(float) + (chain ? RealGetrsWorkspaceBytes(n, n) : RealGetrsStagingBytes(n, n)) +
+           256;
 }
 
 OPS_API aclsolverStatus_t aclsolverSgetri_bufferSize(aclsolverHandle_t handle, int n, float* A, int lda, int* Lwork)
@@ -391,7 +396,7 @@ OPS_API aclsolverStatus_t aclsolverSgetri_bufferSize(aclsolverHandle_t handle, i
     if (n < 0 || n > GetriLimit(handle) || lda < std::max(1, n) || Lwork == nullptr || IsDevice(Lwork) ||
         (A != nullptr && !IsDevice(A)))
         return ACLSOLVER_STATUS_INVALID_VALUE;
-    *Lwork = n == 0 ? 0 : static_cast<int>((GetriWorkBytes(n) + 3) / 4);
+    *Lwork = n == 0 ? 0 : static_cast<int>((std::max(GetriWorkBytes(n, true), GetriWorkBytes(n, false)) + 3) / 4);
     return ACLSOLVER_STATUS_SUCCESS;
 }
 
@@ -410,7 +415,7 @@ OPS_API aclsolverStatus_t aclsolverSgetri(aclsolverHandle_t handle, int n, float
         arg = 4;
     else if (n > 0 && !IsDevice(Workspace))
         arg = 5;
-    else if (n > 0 && static_cast<size_t>(Lwork) * 4 < GetriWorkBytes(n))
+    else if (n > 0 && static_cast<size_t>(Lwork) * 4 < GetriWorkBytes(n, false))
         arg = 6;
     else if (!IsDevice(devInfo))
         arg = 7;
@@ -436,11 +441,10 @@ OPS_API aclsolverStatus_t aclsolverSgetri(aclsolverHandle_t handle, int n, float
     float* X = Workspace;
     void* work = reinterpret_cast<char*>(Workspace) + static_cast<size_t>(n) * n * sizeof(float);
     work = reinterpret_cast<char*>(work) + (256 - reinterpret_cast<uintptr_t>(work) % 256) % 256;
-    if (RealGetrsWorkspaceBytes(n, n) > RealGetrsStagingBytes(n, n))
-        work = HandleScratch(handle, RealGetrsWorkspaceBytes(n, n));
-    if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
+    const bool chain = static_cast<size_t>(Lwork) * 4 >= GetriWorkBytes(n, true);
     hipLaunchKernelGGL(set_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, X, n);
-    if (RealGetrs(0, n, n, A, lda, devIpiv, X, n, work, s, devInfo) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
+    if (RealGetrs(0, n, n, A, lda, devIpiv, X, n, work, s, devInfo, chain) != hipSuccess)
+        return ACLSOLVER_STATUS_EXECUTION_FAILED;
     hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, A, lda, devInfo);
     hipLaunchKernelGGL(copy_matrix_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, n, X, n, A, lda, devInfo);
     return Launched();

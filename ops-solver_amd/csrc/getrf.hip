@@ -714,10 +714,10 @@ hipError_t TransposeRM(int rows, int cols, const float* src, int64_t lds, float*
 }
 
 hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const int* ipiv, float* b, int ldb,
-                     void* work, hipStream_t stream, int* info)
+                     void* work, hipStream_t stream, int* info, bool chain)
 {
     if (n <= 0 || nrhs <= 0) return hipSuccess;
-    if (UseTrs(n, nrhs)) return TrsSolve(trans, n, nrhs, lu, lda, ipiv, b, ldb, b, ldb, info, work, nullptr, stream);
+    if (chain && UseTrs(n, nrhs)) return TrsSolve(trans, n, nrhs, lu, lda, ipiv, b, ldb, b, ldb, info, work, nullptr, stream);
     if (info != nullptr) FillInfo(info, 1, 0, stream);
     float* x = static_cast<float*>(work);
     int* perm = reinterpret_cast<int*>(x + static_cast<size_t>(n) * nrhs);

@@ -178,8 +178,9 @@ size_t RealGetrsWorkspaceBytes(int n, int nrhs);
 // the getri workspace query); the chained solves keep their own layout.
 size_t RealGetrsStagingBytes(int n, int nrhs);
 // info (optional, Device): set to 0, or to kInfoWaitTimeout when a bounded wait of the solve gave up.
+// chain = false: work has RealGetrsStagingBytes only and the chained solve is not taken.
 hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const int* ipiv, float* b, int ldb,
-                     void* work, hipStream_t stream, int* info = nullptr);
+                     void* work, hipStream_t stream, int* info = nullptr, bool chain = true);
 
 // ---- complex LU engine (complex_engine.hip) ----
 // ipiv (1-based interchange sequence) -> perm (perm[i] = source row of row i of P*B), one
