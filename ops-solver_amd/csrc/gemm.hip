@@ -15,12 +15,12 @@
 #include <climits>
 
 #include "lu_kernels.h"
+#include "unitlower.h"
 
 namespace ops
 {
 namespace
 {
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -561,65 +561,30 @@ __global__ __launch_bounds__(256) void trsm_diag64_kernel(int kb, int N, const f
         if (live && 16 * q + t < kb) b[16 * q + t] = x[t];
 }
 
-// Inverses of the unit-lower 64 x 64 diagonal blocks of T (K x K): workgroup b writes
-// inv(T[64b.., 64b..]) to Linv + 4096 b (column-major, ld 64; rows and columns beyond the
-// block are the identity). Column c of the inverse is the forward substitution of e_c,
-// run like trsm_diag64_kernel: a quad of lanes per column, 16 rows each.
-__global__ __launch_bounds__(256) void trtri_unit_lower64_kernel(int K, const float* __restrict__ T, int ldt,
-                                                                 float* __restrict__ Linv)
+// The solve forms (unitlower.h) of the unit-lower 64 x 64 diagonal blocks of T (K x K): workgroup
+// b writes that of T[64b.., 64b..] to forms + 4096 b, padded with the identity.
+__global__ __launch_bounds__(256) void solve_form_kernel(int K, const float* __restrict__ T, int64_t ldt,
+                                                         float* __restrict__ forms)
 {
-    __shared__ __attribute__((aligned(16))) float Ts[64][64];  // Ts[s][i] = T(i, s) of the block
-    const int k0 = blockIdx.x * 64, kb = min(64, K - k0);
-    const float* Tb = T + static_cast<size_t>(k0) * ldt + k0;
-    for (int e = threadIdx.x; e < 64 * 64; e += 256)
-    {
-        const int s2 = e >> 6, i = e & 63;
-        Ts[s2][i] = (i < kb && s2 < kb) ? Tb[static_cast<size_t>(s2) * ldt + i] : 0.0f;
-    }
+    __shared__ __align__(16) float s_l[64 * kInvStride];
+    const int k0 = blockIdx.x * 64, kb = min(64, K - k0), lane = threadIdx.x & 63;
+    const float* const Tb = T + k0 * ldt + k0;
+    for (int c = threadIdx.x >> 6; c < 64; c += 4)
+        s_l[lane * kInvStride + c] = lane > c && lane < kb ? Tb[c * ldt + lane] : 0.0f;
     __syncthreads();
-    const int col = threadIdx.x >> 2, q = threadIdx.x & 3;
-    float x[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) x[t] = (16 * q + t == col) ? 1.0f : 0.0f;
-#pragma unroll
-    for (int s2 = 0; s2 < 64; ++s2)
-    {
-        if (s2 >= kb) continue;  // uniform
-        const int o = s2 >> 4, so = s2 & 15;
-        float xs;
-        if (o == 0)
-            xs = QuadBroadcast<0x00>(x[so]);
-        else if (o == 1)
-            xs = QuadBroadcast<0x55>(x[so]);
-        else if (o == 2)
-            xs = QuadBroadcast<0xAA>(x[so]);
-        else
-            xs = QuadBroadcast<0xFF>(x[so]);
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
-        {
-            const int row = 16 * q + t;
-            const float nx = fmaf(-Ts[s2][row], xs, x[t]);
-            x[t] = (row > s2 && row < kb) ? nx : x[t];
-        }
-    }
-    float* out = Linv + static_cast<size_t>(blockIdx.x) * 4096 + col * 64 + 16 * q;
-#pragma unroll
-    for (int t = 0; t < 16; t += 4)
-        *reinterpret_cast<float4*>(out + t) = make_float4(x[t], x[t + 1], x[t + 2], x[t + 3]);
+    SolveForm64(s_l, forms + static_cast<size_t>(blockIdx.x) * 4096, threadIdx.x);
 }
 
-// B <- T^{-1} B for unit-lower T (K x K, K <= 512) from the block inverses of
-// trtri_unit_lower64_kernel or leaf_finish_kernel: one workgroup of eight waves per 16-column strip
-// of B, held in LDS; per 64-row block b: X_b = inv(T_bb) B_b (waves 0..3, 16 rows each), then
-// B_below -= T(below, b) X_b in tiles of 16 rows, both on FP32 MFMA (16x16x4 tiles formed as
-// products^T so that each accumulator lane holds one row). A panel's next block column has 512
-// columns: 16 wide it spreads over 32 workgroups, with a chain per block half as long (512 x 512
-// alone 85 us with 32 columns and four waves, 34 us now; beside the product of order 16384 145 and
-// 88 us on average).
+// B <- T^{-1} B for unit-lower T (K x K, K <= 512) from the solve forms of its diagonal blocks
+// (solve_form_kernel or leaf_finish_kernel): one workgroup of eight waves per 16-column strip of B,
+// held in LDS; per 64-row block b: X_b from its solve form (one wave: 40 products, a chain of 28),
+// then B_below -= T(below, b) X_b in tiles of 16 rows, both on FP32 MFMA (16x16x4 tiles; the second
+// formed as products^T so that each accumulator lane holds one row). A panel's next block column
+// has 512 columns: 16 wide it spreads over 32 workgroups. 512 x 512 alone 31 us (32 columns and four
+// waves 85 us); beside the product of order 16384 85 us on average.
 constexpr int kTrsmLuMaxK = 512;
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void trsm_lu_kernel(
-    int K, int N, const float* __restrict__ T, int64_t ldt, const float* __restrict__ Linv, float* __restrict__ B,
+    int K, int N, const float* __restrict__ T, int64_t ldt, const float* __restrict__ forms, float* __restrict__ B,
     int64_t ldb)
 {
     __shared__ float Xs[kTrsmLuMaxK][17];
@@ -631,51 +596,74 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void t
     for (int c = wave; c < 16; c += 8)
         for (int r = lane; r < Kp; r += 64) Xs[r][c] = c < nc && r < K ? B[(c0 + c) * ldb + r] : 0.0f;
     __syncthreads();
-    // A tile's operand is loaded whole before its MFMAs, the first one of a block before the block's
-    // own product. Blocks with rows below them are full; rows beyond K repeat the last one.
-    float lf[16];
-    auto loadTile = [&](int k0, int r0)
+    // The last wave solves the blocks and the others update the rows below them, each with its next
+    // operand loaded ahead (one wave doing both would not have the registers); they meet twice a
+    // block.
+    constexpr int UPD = 7;
+    if (wave == UPD)
     {
-        const float* const Lc = T + k0 * ldt + min(r0 + ui, K - 1);
-#pragma unroll
-        for (int t = 0; t < 16; ++t) lf[t] = Lc[(4 * t + uk) * ldt];
-    };
-    for (int b = 0; b < nblk; ++b)
-    {
-        const int k0 = b * 64;
-        int r0 = k0 + 64 + wave * 16;
-        if (r0 < K) loadTile(k0, r0);
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (wave < 4)
+        SolveOperands op;
+        LoadOperands(forms, ui, uk, op);
+        for (int b = 0; b < nblk; ++b)
         {
-            const float* const Lb = Linv + static_cast<size_t>(b) * 4096 + 16 * wave + ui;
-            float lb[16];
+            const int k0 = b * 64;
+            f32x4 x[4];
 #pragma unroll
-            for (int t = 0; t < 16; ++t) lb[t] = Lb[(4 * t + uk) * 64];
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int t = 0; t < 16; ++t)
-                if (t < 4 * (wave + 1))  // uniform: beyond lie the triangle's zeros
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[k0 + 4 * t + uk][ui], lb[t], acc, 0, 0, 0);
+                for (int r = 0; r < 4; ++r) x[t][r] = Xs[k0 + 16 * t + 4 * uk + r][ui];
+            if (__builtin_expect(SolveColumns(op, x), 1))  // uniform
+            {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) Xs[k0 + 16 * t + 4 * uk + r][ui] = x[t][r];
+            }
+            else
+            {
+                float v[16];
+#pragma unroll
+                for (int c = 0; c < 16; ++c) v[c] = Xs[k0 + lane][c];
+                SubstituteColumns(T + k0 * ldt + k0, ldt, min(64, K - k0), lane, v);
+#pragma unroll
+                for (int c = 0; c < 16; ++c) Xs[k0 + lane][c] = v[c];
+            }
+            if (b + 1 < nblk) LoadOperands(forms + static_cast<size_t>(b + 1) * 4096, ui, uk, op);
+            __syncthreads();
+            __syncthreads();
         }
-        __syncthreads();
-        if (wave < 4)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Xs[k0 + 16 * wave + ui][4 * uk + v] = acc[v];
-        __syncthreads();
-        for (; r0 < K; r0 += 128)
-        {
-            acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int t = 0; t < 16; ++t)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[k0 + 4 * t + uk][ui], lf[t], acc, 0, 0, 0);
-            const int row = r0 + ui;
-            if (r0 + 128 < K) loadTile(k0, r0 + 128);
-            if (row < K)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) Xs[row][4 * uk + v] -= acc[v];
-        }
-        __syncthreads();
     }
+    else
+        for (int b = 0; b < nblk; ++b)
+        {
+            const int k0 = b * 64;
+            int r0 = k0 + 64 + wave * 16;
+            // A tile's operand is loaded whole before its MFMAs. Blocks with rows below them are
+            // full; rows beyond K repeat the last one.
+            float lf[16];
+            auto loadTile = [&]()
+            {
+                const float* const Lc = T + k0 * ldt + min(r0 + ui, K - 1);
+#pragma unroll
+                for (int t = 0; t < 16; ++t) lf[t] = Lc[(4 * t + uk) * ldt];
+            };
+            if (r0 < K) loadTile();
+            __syncthreads();
+            while (r0 < K)
+            {
+                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int t = 0; t < 16; ++t)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Xs[k0 + 4 * t + uk][ui], lf[t], acc, 0, 0, 0);
+                const int row = r0 + ui;
+                r0 += 16 * UPD;
+                if (r0 < K) loadTile();
+                if (row < K)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) Xs[row][4 * uk + v] -= acc[v];
+            }
+            __syncthreads();
+        }
     for (int c = wave; c < nc; c += 8)
         for (int r = lane; r < K; r += 64) B[(c0 + c) * ldb + r] = Xs[r][c];
 }
@@ -752,20 +740,20 @@ hipError_t GemmSub(int M, int N, int K, const float* A, int lda, int transA, con
 
 size_t TrsmLowerUnitWorkspaceBytes(int K) { return static_cast<size_t>((K + 63) / 64) * 4096 * sizeof(float); }
 
-hipError_t TrsmLowerUnitInverse(int K, const float* T, int ldt, float* linv, hipStream_t stream)
+hipError_t TrsmLowerUnitForms(int K, const float* T, int ldt, float* forms, hipStream_t stream)
 {
     if (K <= 0 || K > kTrsmLuMaxK) return K <= 0 ? hipSuccess : hipErrorInvalidValue;
-    hipLaunchKernelGGL(trtri_unit_lower64_kernel, dim3((K + 63) / 64), dim3(256), 0, stream, K, T, ldt, linv);
+    hipLaunchKernelGGL(solve_form_kernel, dim3((K + 63) / 64), dim3(256), 0, stream, K, T, static_cast<int64_t>(ldt), forms);
     return hipGetLastError();
 }
 
-hipError_t TrsmLowerUnitApply(int K, int N, const float* T, int ldt, const float* linv, float* B, int ldb,
+hipError_t TrsmLowerUnitApply(int K, int N, const float* T, int ldt, const float* forms, float* B, int ldb,
                               hipStream_t stream)
 {
     if (K <= 0 || N <= 0) return hipSuccess;
     if (K > kTrsmLuMaxK) return hipErrorInvalidValue;
     hipLaunchKernelGGL(trsm_lu_kernel, dim3((N + 15) / 16), dim3(512), 0, stream, K, N, T, static_cast<int64_t>(ldt),
-                       linv, B, static_cast<int64_t>(ldb));
+                       forms, B, static_cast<int64_t>(ldb));
     return hipGetLastError();
 }
 

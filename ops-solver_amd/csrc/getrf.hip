@@ -45,7 +45,7 @@ constexpr int kMovedInts = 4 * NBMAX + 8;
 constexpr size_t kSlotBytes = (256 + 2ull * 128 * 64) * sizeof(unsigned long long);
 static_assert((kLeafSlotWords * 2 + kLeafMoveInts) * sizeof(int) <= kSlotBytes, "leaf words");
 constexpr int kProbeGroups = 8 * 128;  // workgroups of the placement probe
-constexpr size_t kLinvPanelBytes = (NBMAX / 64) * 4096 * sizeof(float);  // block inverses of one panel's L11
+constexpr size_t kFormPanelBytes = (NBMAX / 64) * 4096 * sizeof(float);  // solve forms of one panel's L11 (unitlower.h)
 struct Work
 {
     int* rowsrc;
@@ -57,9 +57,9 @@ struct Work
     int* leafMoves;
     int* err;
     unsigned* epoch;       // host counter: tag base of the next multi-workgroup leaf
-    float* linvNode;       // tournament panels: block inverses for their internal solves
+    float* formNode;       // tournament panels: solve forms for their internal solves
     float* panelRows;      // the same space: 64 rows of the panel columns right of a leaf (panel stream only)
-    float* linvPanel[2];   // block inverses of panel k's L11 in slot k % 2 (both streams read them)
+    float* formPanel[2];   // solve forms of panel k's L11 in slot k % 2 (both streams read them)
     void* tslu;            // scratch of the tournament leaves
     bool tournament;       // tall leaves pivot by tournament (TsluLeaf)
 };
@@ -83,11 +83,11 @@ inline Work Layout(void* base, int m)
     w.err = reinterpret_cast<int*>(q + kSlotBytes);
     w.epoch = nullptr;
     q = (q + kSlotBytes + 16 + 255) & ~static_cast<uintptr_t>(255);
-    w.linvNode = w.panelRows = reinterpret_cast<float*>(q);
-    static_assert(NBMAX * kLeafMaxWidth * sizeof(float) <= kLinvPanelBytes, "panel rows");
-    w.linvPanel[0] = reinterpret_cast<float*>(q + kLinvPanelBytes);
-    w.linvPanel[1] = reinterpret_cast<float*>(q + 2 * kLinvPanelBytes);
-    w.tslu = reinterpret_cast<void*>(q + 3 * kLinvPanelBytes);
+    w.formNode = w.panelRows = reinterpret_cast<float*>(q);
+    static_assert(NBMAX * kLeafMaxWidth * sizeof(float) <= kFormPanelBytes, "panel rows");
+    w.formPanel[0] = reinterpret_cast<float*>(q + kFormPanelBytes);
+    w.formPanel[1] = reinterpret_cast<float*>(q + 2 * kFormPanelBytes);
+    w.tslu = reinterpret_cast<void*>(q + 3 * kFormPanelBytes);
     w.tournament = false;
     return w;
 }
@@ -310,22 +310,22 @@ LeafArgs MakeLeaf(float* A, int lda, int m, int j0, int c0, int wact, int panelE
     } while (0)
 
 // The panel [j0, panelEnd) of rows [j0, m): per 64 columns one leaf, one launch that applies its
-// interchanges to the whole panel and inverts its diagonal block, and one that updates all
-// panel columns to its right. The block inverses (linv, 4096 floats per 64 columns) serve the
+// interchanges to the whole panel and prepares its diagonal block, and one that updates all
+// panel columns to its right. The solve forms (4096 floats per 64 columns) serve the
 // U12 solves of the trailing columns afterwards.
 // Right-looking by 64 columns rather than recursive: the same number of updates, each one
 // launch instead of two to four, for somewhat more traffic on the panel.
 hipError_t Panel(float* a, int lda, int m, int j0, int panelEnd, int pivoting, int* ipiv, int* info, const Work& wk,
-                 float* linv, hipStream_t stream)
+                 float* forms, hipStream_t stream)
 {
     for (int c0 = j0; c0 < panelEnd; c0 += kLeafMaxWidth)
     {
         const int wact = std::min(kLeafMaxWidth, panelEnd - c0);
         LeafArgs l = MakeLeaf(a, lda, m, j0, c0, wact, panelEnd, pivoting, ipiv, info, wk);
-        float* const inv = linv + static_cast<size_t>(c0 - j0) * kLeafMaxWidth;
+        float* const form = forms + static_cast<size_t>(c0 - j0) * kLeafMaxWidth;
         RET_IF(LeafColumns(l, wk, stream));
-        RET_IF(LeafFinish(l, inv, wk.panelRows, stream));
-        if (c0 + wact < panelEnd) RET_IF(PanelUpdate(l, inv, wk.panelRows, stream));
+        RET_IF(LeafFinish(l, form, wk.panelRows, stream));
+        if (c0 + wact < panelEnd) RET_IF(PanelUpdate(l, form, wk.panelRows, stream));
     }
     return hipSuccess;
 }
@@ -360,8 +360,8 @@ hipError_t PanelRec(float* a, int lda, int m, int j0, int panelEnd, int c0, int 
         RET_IF(TrsmBlock(h, r, L11, lda, true, true, false, B12, lda, stream));
     else
     {
-        RET_IF(TrsmLowerUnitInverse(h, L11, lda, wk.linvNode, stream));
-        RET_IF(TrsmLowerUnitApply(h, r, L11, lda, wk.linvNode, B12, lda, stream));
+        RET_IF(TrsmLowerUnitForms(h, L11, lda, wk.formNode, stream));
+        RET_IF(TrsmLowerUnitApply(h, r, L11, lda, wk.formNode, B12, lda, stream));
     }
     if (m - c0 - h > 0)
         RET_IF(GemmSub(m - c0 - h, r, h, a + static_cast<size_t>(c0) * lda + c0 + h, lda, 0,
@@ -376,7 +376,7 @@ size_t RealGetrfWorkspaceBytes(int m, int n)
 {
     (void)n;
     // The tournament leaves' scratch only where one can run (a panel taller than TsluRows).
-    return WorkInts(std::max(m, 1)) * sizeof(int) + 8 + kSlotBytes + 16 + 256 + 3 * kLinvPanelBytes +
+    return WorkInts(std::max(m, 1)) * sizeof(int) + 8 + kSlotBytes + 16 + 256 + 3 * kFormPanelBytes +
            (m > TsluRows() ? TsluScratchBytes(m) : 0);
 }
 
@@ -439,19 +439,19 @@ hipError_t RealGetrfPerm(int m, int n, float* a, int lda, int* ipiv, int* info, 
     auto panel = [&](int k) -> hipError_t
     {
         const int j0 = k * NB, nb = std::min(NB, kmax - j0);
-        float* const linv = w.linvPanel[k & 1];
+        float* const forms = w.formPanel[k & 1];
         if (w.tournament)
             RET_IF(PanelRec(a, lda, m, j0, j0 + nb, j0, nb, pivoting, ipiv, info, w, s0));
         else
-            RET_IF(Panel(a, lda, m, j0, j0 + nb, pivoting, ipiv, info, w, linv, s0));
+            RET_IF(Panel(a, lda, m, j0, j0 + nb, pivoting, ipiv, info, w, forms, s0));
         // The first panel's list serves the columns right of it and perm only.
         if (pivoting && (k > 0 || j0 + nb < n || permOut != nullptr))
             hipLaunchKernelGGL(compact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, w.err,
                                moved(k), permOut);
         RET_IF(hipGetLastError());
-        // The U12 solves of both streams use the block inverses of this panel's L11.
+        // The U12 solves of both streams use the solve forms of this panel's L11.
         if (!w.tournament) return hipSuccess;
-        return TrsmLowerUnitInverse(nb, a + static_cast<size_t>(j0) * lda + j0, lda, linv, s0);
+        return TrsmLowerUnitForms(nb, a + static_cast<size_t>(j0) * lda + j0, lda, forms, s0);
     };
     // Applies panel k to the columns [lo, hi) (interchanges, U12 solve, trailing product)
     // and, when leftSwaps, its interchanges to the columns left of the panel.
@@ -464,7 +464,7 @@ hipError_t RealGetrfPerm(int m, int n, float* a, int lda, int* ipiv, int* info, 
                                hi, moved(k));
         RET_IF(hipGetLastError());
         if (cols <= 0) return hipSuccess;
-        RET_IF(TrsmLowerUnitApply(nb, cols, a + static_cast<size_t>(j0) * lda + j0, lda, w.linvPanel[k & 1],
+        RET_IF(TrsmLowerUnitApply(nb, cols, a + static_cast<size_t>(j0) * lda + j0, lda, w.formPanel[k & 1],
                                   a + static_cast<size_t>(lo) * lda + j0, lda, st));
         if (m - pe <= 0) return hipSuccess;
         const float* L21 = a + static_cast<size_t>(j0) * lda + pe;

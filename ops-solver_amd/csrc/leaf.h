@@ -42,11 +42,11 @@ hipError_t LeafSingle(const LeafArgs& a, hipStream_t stream);
 // Up to 64 workgroups (m - c0 <= kLeafMultiRows, wact <= kLeafMaxWidth):
 hipError_t LeafMulti(const LeafArgs& a, bool cooperative, bool spread, hipStream_t stream);
 hipError_t LeafSwap(const LeafArgs& a, hipStream_t stream);
-// The same and, with it, linv (4096 floats, column-major): the inverse of the leaf's unit-lower
-// diagonal block, padded with the identity; the top 64 rows of the panel columns right of the
-// leaf go to ub (64 floats a column) instead of A.
-hipError_t LeafFinish(const LeafArgs& a, float* linv, float* ub, hipStream_t stream);
+// The same and, with it, the solve form (unitlower.h; 4096 floats, column-major) of the leaf's
+// unit-lower diagonal block, padded with the identity; the top 64 rows of the panel columns right
+// of the leaf go to ub (64 floats a column, 16-byte aligned) instead of A.
+hipError_t LeafFinish(const LeafArgs& a, float* form, float* ub, hipStream_t stream);
 // After LeafFinish of a 64-column leaf: U = inv(L11) ub into A's top rows and the update of the
 // rows below, for the panel columns right of the leaf.
-hipError_t PanelUpdate(const LeafArgs& a, const float* linv, const float* ub, hipStream_t stream);
+hipError_t PanelUpdate(const LeafArgs& a, const float* form, const float* ub, hipStream_t stream);
 }  // namespace ops

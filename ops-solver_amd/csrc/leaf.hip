@@ -36,7 +36,7 @@
 
 #include "internal.h"
 #include "lanes.h"
-#include "trtri64.h"
+#include "unitlower.h"
 #include "wave.h"
 
 namespace ops
@@ -669,17 +669,17 @@ __global__ __launch_bounds__(256) void leaf_swap_kernel(float* __restrict__ A, i
 }
 
 // What follows a leaf of 64 columns, in one launch: its interchanges on every panel column
-// and the inverse of its unit-lower 64 x 64 diagonal block. Workgroup 0 takes the leaf's own
-// columns (it needs them in place for the inverse), the others a wave per column left and
+// and the solve form of its unit-lower 64 x 64 diagonal block (unitlower.h). Workgroup 0 takes the
+// leaf's own columns (it needs them in place for that), the others a wave per column left and
 // right of it. The top 64 rows of the right columns go to ub (ld 64) instead of A: the launch
 // that turns them into U writes A while its other workgroups still read them.
 __global__ __launch_bounds__(256) void leaf_finish_kernel(float* __restrict__ A, int64_t lda, int j0, int c0, int wact,
                                                           int hi, const int2* __restrict__ moves,
-                                                          const int* __restrict__ err, float* __restrict__ linv,
+                                                          const int* __restrict__ err, float* __restrict__ form,
                                                           float* __restrict__ ub)
 {
     constexpr int W = kLeafMaxWidth;
-    __shared__ __align__(16) float s_l[W * kInvStride], s_i[W * kInvStride], s_t[32 * kInvStride];
+    __shared__ __align__(16) float s_l[W * kInvStride];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (*err != 0) return;  // after a timeout the list is not complete
     const int2 none = make_int2(-1, -1);
@@ -725,18 +725,11 @@ __global__ __launch_bounds__(256) void leaf_finish_kernel(float* __restrict__ A,
             if (m0.x >= 0) col[m0.x] = x0[k];
             if (m1.x >= 0) col[m1.x] = x1[k];
         }
-        // Unit lower; rows and columns beyond the block are the identity.
+        // Rows and columns beyond the block are the identity.
         s_l[lane * kInvStride + c] = lane > c && lane < wact ? x0[k] : 0.0f;
-        s_i[lane * kInvStride + c] = 0.0f;
     }
     __syncthreads();
-    InvertLower64<true>(s_l, s_i, s_t, tid);
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-    {
-        const int c = wave * 16 + k;
-        linv[c * W + lane] = s_i[lane * kInvStride + c];
-    }
+    SolveForm64(s_l, form, tid);
 }
 
 // The panel columns right of a finished leaf: U = inv(L11) B (B: the 64 rows of ub) and
@@ -744,16 +737,17 @@ __global__ __launch_bounds__(256) void leaf_finish_kernel(float* __restrict__ A,
 // of its 64 columns itself (40 products of 16 x 16 x 4 a wave, 0.5 us) rather than wait for a
 // launch that does; those of the first tile row store it. Bound by latency for short panels
 // and by the read and write of C for tall ones. The operands of the update are loaded before
-// U is formed, so the launch waits for memory once.
+// U is formed, so the launch waits for memory once; U's operands come in the layout of its products,
+// so the waves meet once (order 512, on average 6.8 us; 11.4 us with three barriers).
 template <int RT>
 __global__ __launch_bounds__(256) void panel_update_kernel(float* __restrict__ A, int64_t lda, int m, int c0, int hi,
-                                                           const float* __restrict__ linv, const float* __restrict__ ub)
+                                                           const float* __restrict__ form, const float* __restrict__ ub)
 {
     constexpr int W = kLeafMaxWidth;
     constexpr int BS = W + 4;
     constexpr int NT = 2 * RT / 4;    // 32 x 32 tiles per wave: 1 (RT = 2) or 2 (RT = 4)
     static_assert(RT == 2 || RT == 4, "64 or 128 rows");
-    __shared__ __align__(16) float s_b[W * BS];  // [column][row], then U in the same place
+    __shared__ __align__(16) float s_b[W * BS];  // U, [column][row]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 31, lk = lane >> 5;
     const int col0 = static_cast<int>(blockIdx.y) * W, cols = min(W, hi - (c0 + W) - col0);
@@ -762,21 +756,17 @@ __global__ __launch_bounds__(256) void panel_update_kernel(float* __restrict__ A
     // Wave: rows wr .. wr + 31 of the tile, 32-column strips ws, ws + CT, ...
     const int row = row0 + (wave % RT) * 32 + li, ws = wave / RT;
     const bool inRow = row < m;
-    // inv(L11) fragments for this wave's 16 columns of U: all 64 rows, k ascending.
+    // U, columns 16 wave .. 16 wave + 15.
     const int ui = lane & 15, uk = lane >> 4;
-    float lf[40], l21[32], cv[NT][16];
-#pragma unroll
-    for (int t = 0, x = 0; t < 4; ++t)
-#pragma unroll
-        for (int k = 0; k < 4 * (t + 1); ++k, ++x) lf[x] = linv[(4 * k + uk) * W + 16 * t + ui];
+    const float* const ubc = ub + static_cast<size_t>(col0 + 16 * wave) * W;
+    SolveOperands op;
+    LoadOperands(form, ui, uk, op);
+    f32x4 u[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-    {
-        const int c = tid >> 4, r4 = (tid & 15) * 4;
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (c + 16 * t < cols) v = *reinterpret_cast<const float4*>(ub + static_cast<size_t>(col0 + c + 16 * t) * W + r4);
-        *reinterpret_cast<float4*>(s_b + (c + 16 * t) * BS + r4) = v;
-    }
+        u[t] = 16 * wave + ui < cols ? *reinterpret_cast<const f32x4*>(ubc + ui * W + 16 * t + 4 * uk)
+                                     : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float l21[32], cv[NT][16];
     const float* lp = A + c0 * lda + row + lk * lda;
 #pragma unroll
     for (int t = 0; t < 32; ++t)
@@ -792,21 +782,20 @@ __global__ __launch_bounds__(256) void panel_update_kernel(float* __restrict__ A
             const int c = (ws + n * (2 / NT)) * 32 + (v & 3) + 8 * (v >> 2) + 4 * lk;
             cv[n][v] = inRow && c < cols ? Ct[c * lda + row] : 0.0f;
         }
-    __syncthreads();
-    // U, columns 16 wave .. 16 wave + 15: lane (ui, uk) of product t gets rows 16 t + 4 uk + r.
-    f32x4 uacc[4];
-#pragma unroll
-    for (int t = 0, x = 0; t < 4; ++t)
+    if (__builtin_expect(SolveColumns(op, u), 1))  // uniform over the wave
     {
-        uacc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int k = 0; k < 4 * (t + 1); ++k, ++x)
-            uacc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(lf[x], s_b[(16 * wave + ui) * BS + 4 * k + uk], uacc[t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) *reinterpret_cast<f32x4*>(s_b + (16 * wave + ui) * BS + 16 * t + 4 * uk) = u[t];
     }
-    __syncthreads();
+    else
+    {
+        float v[16];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-        *reinterpret_cast<f32x4*>(s_b + (16 * wave + ui) * BS + 16 * t + 4 * uk) = uacc[t];
+        for (int c = 0; c < 16; ++c) v[c] = 16 * wave + c < cols ? ubc[c * W + lane] : 0.0f;
+        SubstituteColumns(A + c0 * lda + c0, lda, W, lane, v);
+#pragma unroll
+        for (int c = 0; c < 16; ++c) s_b[(16 * wave + c) * BS + lane] = v[c];
+    }
     __syncthreads();
     if (blockIdx.x == 0)
 #pragma unroll
@@ -896,16 +885,16 @@ hipError_t LeafSwap(const LeafArgs& a, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t LeafFinish(const LeafArgs& a, float* linv, float* ub, hipStream_t stream)
+hipError_t LeafFinish(const LeafArgs& a, float* form, float* ub, hipStream_t stream)
 {
     const int others = (a.c0 - a.j0) + (a.panelEnd - a.c0 - a.wact);
     hipLaunchKernelGGL(leaf_finish_kernel, dim3(1 + (others + 3) / 4), dim3(256), 0, stream, a.A,
                        static_cast<int64_t>(a.lda), a.j0, a.c0, a.wact, a.panelEnd,
-                       reinterpret_cast<const int2*>(a.moves), a.err, linv, ub);
+                       reinterpret_cast<const int2*>(a.moves), a.err, form, ub);
     return hipGetLastError();
 }
 
-hipError_t PanelUpdate(const LeafArgs& a, const float* linv, const float* ub, hipStream_t stream)
+hipError_t PanelUpdate(const LeafArgs& a, const float* form, const float* ub, hipStream_t stream)
 {
     const int cols = a.panelEnd - a.c0 - kLeafMaxWidth, rows = a.m - a.c0 - kLeafMaxWidth;
     if (a.wact != kLeafMaxWidth) return hipErrorInvalidValue;
@@ -915,10 +904,10 @@ hipError_t PanelUpdate(const LeafArgs& a, const float* linv, const float* ub, hi
     // above, where the repeated formation of U would cost more.
     if ((rows + 63) / 64 * nc <= 512)
         hipLaunchKernelGGL(panel_update_kernel<2>, dim3(std::max(1, (rows + 63) / 64), nc), dim3(256), 0, stream, a.A,
-                           static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, linv, ub);
+                           static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, form, ub);
     else
         hipLaunchKernelGGL(panel_update_kernel<4>, dim3((rows + 127) / 128, nc), dim3(256), 0, stream, a.A,
-                           static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, linv, ub);
+                           static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, form, ub);
     return hipGetLastError();
 }
 }  // namespace ops
