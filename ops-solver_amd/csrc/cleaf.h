@@ -33,18 +33,18 @@ constexpr int kCLeafRowWord = kCLeafValueWord + 2 * 16 * kCLeafMaxGroups;
 constexpr int kCLeafRowStride = 2 * kCLeafWidth + 16;
 constexpr int kCLeafArrivalWord = kCLeafRowWord + 2 * 8 * kCLeafRowStride;
 constexpr int kCLeafSlotWords = kCLeafArrivalWord + kCLeafMaxGroups;
-constexpr size_t kCInverseBlock = 2 * 64 * 64;  // floats per diagonal block: real part, then imaginary part
+constexpr size_t kCFormBlock = 2 * 64 * 64;  // floats per diagonal block: real part, then imaginary part
 
 hipError_t CLeafColumns(const CLeafArgs& a, bool spread, hipStream_t stream);
-// The leaf's interchanges on the whole panel; the inverse of its unit-lower diagonal block to
-// linv (kCInverseBlock floats, column-major, padded with the identity); the top 64 rows of the
+// The leaf's interchanges on the whole panel; the solve form of its unit-lower diagonal
+// block to form (kCFormBlock floats: unitlower.h's, real parts, then imaginary parts); the top 64 rows of the
 // panel columns right of it to ub (64 complex a column) instead of A.
-hipError_t CLeafFinish(const CLeafArgs& a, float* linv, float2* ub, hipStream_t stream);
+hipError_t CLeafFinish(const CLeafArgs& a, float* form, float2* ub, hipStream_t stream);
 // After CLeafFinish of a 64-column leaf: U = inv(L11) ub into A's top rows, and the update of the
 // rows below, for the panel columns right of the leaf.
-hipError_t CPanelUpdate(const CLeafArgs& a, const float* linv, const float2* ub, hipStream_t stream);
-// B <- L^{-1} B for the unit-lower K x K block T (K <= 512) and N columns, from the inverses of
-// T's 64 x 64 diagonal blocks.
-hipError_t CTrsmLowerUnit(int K, int N, const float2* T, int ldt, const float* linv, float2* B, int ldb,
+hipError_t CPanelUpdate(const CLeafArgs& a, const float* form, const float2* ub, hipStream_t stream);
+// B <- L^{-1} B for the unit-lower K x K block T (K <= 512) and N columns, from the solve forms
+// of T's 64 x 64 diagonal blocks.
+hipError_t CTrsmLowerUnit(int K, int N, const float2* T, int ldt, const float* forms, float2* B, int ldb,
                           hipStream_t stream);
 }  // namespace ops

@@ -17,7 +17,7 @@
 #include "complex_math.h"
 #include "internal.h"
 #include "lanes.h"
-#include "trtri64.h"
+#include "unitlower.h"
 #include "wave.h"
 
 namespace ops
@@ -540,86 +540,138 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(MULTI &
     }
 }
 
-// D (16 x 16 at d) = sign * A (16 x K) * B (K x 16), complex, real and imaginary parts kC apart.
+// unitlower.h's solve form of a unit-lower block, real parts, then imaginary parts 4096 floats
+// further; s: the block's strictly lower triangle row-major in LDS, imaginary parts kC further.
+// Growth in the norm |re| + |im|; 256: 768 diagonal blocks each of complex Gaussian, uniform and
+// small-integer matrices with partial pivoting have 113, 132 and 131 at most.
 constexpr int kC = 64 * kInvStride;
-template <int K>
-__device__ inline void CProduct16(const float* a, const float* b, float* d, float sign, int lane)
-{
-    f32x4 re = {0.0f, 0.0f, 0.0f, 0.0f}, im = re;
-    const int i = lane & 15, k0 = lane >> 4;
-#pragma unroll
-    for (int k = 0; k < K; k += 4)
-    {
-        const float ar = a[i * kInvStride + k + k0], ai = a[kC + i * kInvStride + k + k0];
-        const float* const bp = b + (k + k0) * kInvStride + i;
-        const float br = bp[0], bi = bp[kC];
-        re = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, br, re, 0, 0, 0);
-        im = __builtin_amdgcn_mfma_f32_16x16x4f32(ar, bi, im, 0, 0, 0);
-        re = __builtin_amdgcn_mfma_f32_16x16x4f32(-ai, bi, re, 0, 0, 0);
-        im = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, br, im, 0, 0, 0);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-    {
-        d[(4 * k0 + r) * kInvStride + i] = sign * re[r];
-        d[kC + (4 * k0 + r) * kInvStride + i] = sign * im[r];
-    }
-}
-
-// trtri64.h's InvertLower64 for a unit-lower complex block in place (real parts, and imaginary
-// parts kC floats further): a block is read for the last time before its inverse goes there, and
-// the intermediate product lies in the upper right quarter. A third of the LDS of separate
-// arrays, which every workgroup of the launch would reserve (104 KB of them waited for whole
-// compute units beside the trailing product: 50 us a launch at order 8192, now 20).
-__device__ inline void CInvertUnitLower64(float* s, int tid)
+constexpr float kCInverseGrowth = 256.0f;
+__device__ inline void CSolveForm64(const float* s, float* __restrict__ form, int tid)
 {
     const int lane = tid & 63, wave = tid >> 6;
-    float* const t = s + 32;
-    if (wave == 0)
-    {
-        const int b = lane & 48;
-        float2 x[16];
+    if ((lane >> 4) != wave)
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
+        for (int k = 0; k < 16; ++k)
         {
-            float2 v = make_float2(i == (lane & 15) ? 1.0f : 0.0f, 0.0f);
-            const float* const row = s + (b + i) * kInvStride + b;
-#pragma unroll
-            for (int k = 0; k < i; ++k) v = SubMul(v, make_float2(row[k], row[kC + k]), x[k]);
-            x[i] = v;
+            const int c = 16 * wave + k, at = lane * kInvStride + c;
+            const bool low = (lane >> 4) > wave;
+            if (c != 63 || lane != 0) form[c * 64 + lane] = low ? -s[at] : 0.0f;
+            form[4096 + c * 64 + lane] = low ? -s[kC + at] : 0.0f;
         }
+    if (wave != 0) return;
+    const int b = lane & 48;
+    float2 x[16];
+    float grow[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
+    for (int i = 0; i < 16; ++i)
+    {
+        float2 v = make_float2(i == (lane & 15) ? 1.0f : 0.0f, 0.0f);
+        const float* const row = s + (b + i) * kInvStride + b;
+#pragma unroll
+        for (int k = 0; k < i; ++k)
         {
-            s[(b + i) * kInvStride + lane] = x[i].x;
-            s[kC + (b + i) * kInvStride + lane] = x[i].y;
+            const float2 l = make_float2(row[k], row[kC + k]);
+            v = SubMul(v, l, x[k]);
+            grow[k & 3] = fmaf(fabsf(l.x) + fabsf(l.y), fabsf(x[k].x) + fabsf(x[k].y), grow[k & 3]);
+        }
+        x[i] = v;
+        grow[3] += fabsf(v.x) + fabsf(v.y);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+    {
+        const bool low = i > (lane & 15);
+        form[lane * 64 + b + i] = low ? x[i].x : 0.0f;
+        form[4096 + lane * 64 + b + i] = low ? x[i].y : 0.0f;
+    }
+    const bool fine = (grow[0] + grow[1]) + (grow[2] + grow[3]) <= kCInverseGrowth;
+    const bool all = __all(fine);
+    if (lane == 0) form[kSubstituteFlag] = all ? 0.0f : 1.0f;
+}
+
+struct CSolveOperands
+{
+    float re[40], im[40];
+    float substitute;
+};
+__device__ inline void LoadOperands(const float* __restrict__ form, int ui, int uk, CSolveOperands& o)
+{
+#pragma unroll
+    for (int t = 0, x = 0; t < 4; ++t)
+#pragma unroll
+        for (int d = t; d < 4; ++d)
+#pragma unroll
+            for (int s = 0; s < 4; ++s, ++x)
+            {
+                const int at = (16 * t + 4 * uk + s) * 64 + 16 * d + ui;
+                o.re[x] = form[at];
+                o.im[x] = form[4096 + at];
+            }
+    o.substitute = form[kSubstituteFlag];
+}
+
+// unitlower.h's SolveColumns on pairs of real products.
+__device__ inline bool CSolveColumns(const CSolveOperands& o, f32x4 (&re)[4], f32x4 (&im)[4])
+{
+    bool fine = o.substitute == 0.0f;
+    auto add = [&](int x, float br, float bi, f32x4& r, f32x4& i)
+    {
+        r = __builtin_amdgcn_mfma_f32_16x16x4f32(o.re[x], br, r, 0, 0, 0);
+        i = __builtin_amdgcn_mfma_f32_16x16x4f32(o.re[x], bi, i, 0, 0, 0);
+        r = __builtin_amdgcn_mfma_f32_16x16x4f32(-o.im[x], bi, r, 0, 0, 0);
+        i = __builtin_amdgcn_mfma_f32_16x16x4f32(o.im[x], br, i, 0, 0, 0);
+    };
+    f32x4 sr[4], si[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sr[t] = si[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0, x = 0; t < 4; ++t)
+    {
+        if (t > 0)
+        {
+            re[t] = re[t] + sr[t];
+            im[t] = im[t] + si[t];
+        }
+        f32x4 ur = {0.0f, 0.0f, 0.0f, 0.0f}, ux = ur;
+#pragma unroll
+        for (int s = 0; s < 4; ++s, ++x) add(x, re[t][s], im[t][s], ur, ux);
+        re[t] = re[t] + ur;
+        im[t] = im[t] + ux;
+#pragma unroll
+        for (int d = t + 1; d < 4; ++d)
+#pragma unroll
+            for (int s = 0; s < 4; ++s, ++x) add(x, re[t][s], im[t][s], sr[d], si[d]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fine = fine && fabsf(re[t][r]) <= FLT_MAX && fabsf(im[t][r]) <= FLT_MAX;
+    }
+    return __all(fine);
+}
+
+__device__ inline void SubstituteColumns(const float2* __restrict__ T, int64_t ldt, int size, int lane, float2 (&v)[16])
+{
+#pragma unroll 1
+    for (int k = 0; k + 1 < size; ++k)
+    {
+        const bool below = lane > k && lane < size;
+        const float2 l = below ? T[k * ldt + lane] : make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+        {
+            const float2 y = SubMul(v[c], l, make_float2(ReadLane(v[c].x, k), ReadLane(v[c].y, k)));
+            if (below) v[c] = y;
         }
     }
-    __syncthreads();
-    if (wave < 2)
-        CProduct16<16>(s + (32 * wave + 16) * kInvStride + 32 * wave, s + 32 * wave * kInvStride + 32 * wave,
-                       t + 16 * wave * kInvStride, 1.0f, lane);
-    __syncthreads();
-    if (wave < 2)
-        CProduct16<16>(s + (32 * wave + 16) * kInvStride + 32 * wave + 16, t + 16 * wave * kInvStride,
-                       s + (32 * wave + 16) * kInvStride + 32 * wave, -1.0f, lane);
-    __syncthreads();
-    const int qr = 16 * (wave >> 1), qc = 16 * (wave & 1);
-    CProduct16<32>(s + (32 + qr) * kInvStride, s + qc, t + qr * kInvStride + qc, 1.0f, lane);
-    __syncthreads();
-    CProduct16<32>(s + (32 + qr) * kInvStride + 32, t + qc, s + (32 + qr) * kInvStride + qc, -1.0f, lane);
-    __syncthreads();
 }
 
 // leaf.hip's leaf_finish_kernel for complex columns.
 __global__ __launch_bounds__(256) void cleaf_finish_kernel(float2* __restrict__ A, int64_t lda, int j0, int c0, int wact,
                                                            int hi, const int2* __restrict__ moves,
-                                                           const int* __restrict__ err, float* __restrict__ linv,
+                                                           const int* __restrict__ err, float* __restrict__ form,
                                                            float2* __restrict__ ub)
 {
     __builtin_amdgcn_s_setprio(3);  // before the trailing product's waves on the same SIMD
     constexpr int W = kCLeafWidth;
-    __shared__ __align__(16) float s_l[2 * kC];  // the block, then its inverse
+    __shared__ __align__(16) float s_l[2 * kC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (*err != 0) return;  // after a timeout the list is not complete
     const int2 none = make_int2(-1, -1);
@@ -670,48 +722,19 @@ __global__ __launch_bounds__(256) void cleaf_finish_kernel(float2* __restrict__ 
         s_l[kC + lane * kInvStride + c] = in ? x0[k].y : 0.0f;
     }
     __syncthreads();
-    CInvertUnitLower64(s_l, tid);
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-    {
-        const int c = wave * 16 + k;
-        linv[c * W + lane] = lane >= c ? s_l[lane * kInvStride + c] : 0.0f;
-        linv[4096 + c * W + lane] = lane >= c ? s_l[kC + lane * kInvStride + c] : 0.0f;
-    }
+    CSolveForm64(s_l, form, tid);
 }
 
-// One 16-column strip (wave) of U = inv(L11) B, 64 rows: B at sr / si in LDS as [column][row].
-__device__ inline void FormU(const float* __restrict__ linv, const float* sr, const float* si, int BS, int wave, int ui,
-                             int uk, f32x4 (&re)[4], f32x4 (&im)[4])
-{
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-    {
-        re[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        im[t] = re[t];
-#pragma unroll
-        for (int k = 0; k < 4 * (t + 1); ++k)
-        {
-            const int at = (4 * k + uk) * 64 + 16 * t + ui;
-            const float lr = linv[at], li = linv[4096 + at];
-            const float br = sr[(16 * wave + ui) * BS + 4 * k + uk], bi = si[(16 * wave + ui) * BS + 4 * k + uk];
-            re[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(lr, br, re[t], 0, 0, 0);
-            im[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(lr, bi, im[t], 0, 0, 0);
-            re[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(-li, bi, re[t], 0, 0, 0);
-            im[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(li, br, im[t], 0, 0, 0);
-        }
-    }
-}
-
-// leaf.hip's panel_update_kernel for complex columns: 64 x 64 tiles of C, one 32 x 32 tile a wave.
+// leaf.hip's panel_update_kernel for complex columns: 64 x 64 tiles of C, one 32 x 32 tile a wave
+// (order 512, on average 15 us; 23 us with the product read back from LDS and operands in the loop).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void cpanel_update_kernel(
-    float2* __restrict__ A, int64_t lda, int m, int c0, int hi, const float* __restrict__ linv,
+    float2* __restrict__ A, int64_t lda, int m, int c0, int hi, const float* __restrict__ form,
     const float2* __restrict__ ub)
 {
     __builtin_amdgcn_s_setprio(3);  // before the trailing product's waves on the same SIMD
     constexpr int W = kCLeafWidth;
     constexpr int BS = W + 4;
-    __shared__ __align__(16) float s_r[W * BS], s_i[W * BS];  // [column][row] of B, then of U
+    __shared__ __align__(16) float s_r[W * BS], s_i[W * BS];  // [column][row] of U
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 31, lk = lane >> 5, ui = lane & 15, uk = lane >> 4;
     const int col0 = static_cast<int>(blockIdx.y) * W, cols = min(W, hi - (c0 + W) - col0);
@@ -719,6 +742,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     float2* const Ct = A + (c0 + W + col0) * lda;
     const int row = row0 + (wave & 1) * 32 + li, strip = (wave >> 1) * 32;
     const bool inRow = row < m;
+    const float2* const ubc = ub + static_cast<size_t>(col0 + 16 * wave) * W;
+    CSolveOperands op;
+    LoadOperands(form, ui, uk, op);
+    f32x4 re[4], im[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const float2 v = 16 * wave + ui < cols ? ubc[ui * W + 16 * t + 4 * uk + r] : make_float2(0.0f, 0.0f);
+            re[t][r] = v.x;
+            im[t][r] = v.y;
+        }
     float2 l21[32];
     const float2* lp = A + c0 * lda + row + lk * lda;
 #pragma unroll
@@ -727,24 +763,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
         l21[t] = inRow ? *lp : make_float2(0.0f, 0.0f);
         lp += 2 * lda;
     }
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
+    if (__builtin_expect(CSolveColumns(op, re, im), 1))  // uniform over the wave
     {
-        const int c = (tid >> 6) + 4 * t;
-        float2 v = make_float2(0.0f, 0.0f);
-        if (c < cols) v = ub[static_cast<size_t>(col0 + c) * W + lane];
-        s_r[c * BS + lane] = v.x;
-        s_i[c * BS + lane] = v.y;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+        {
+            *reinterpret_cast<f32x4*>(s_r + (16 * wave + ui) * BS + 16 * t + 4 * uk) = re[t];
+            *reinterpret_cast<f32x4*>(s_i + (16 * wave + ui) * BS + 16 * t + 4 * uk) = im[t];
+        }
     }
-    __syncthreads();
-    f32x4 re[4], im[4];
-    FormU(linv, s_r, s_i, BS, wave, ui, uk, re, im);
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
+    else
     {
-        *reinterpret_cast<f32x4*>(s_r + (16 * wave + ui) * BS + 16 * t + 4 * uk) = re[t];
-        *reinterpret_cast<f32x4*>(s_i + (16 * wave + ui) * BS + 16 * t + 4 * uk) = im[t];
+        float2 v[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) v[c] = 16 * wave + c < cols ? ubc[c * W + lane] : make_float2(0.0f, 0.0f);
+        SubstituteColumns(A + c0 * lda + c0, lda, W, lane, v);
+#pragma unroll
+        for (int c = 0; c < 16; ++c)
+        {
+            s_r[(16 * wave + c) * BS + lane] = v[c].x;
+            s_i[(16 * wave + c) * BS + lane] = v[c].y;
+        }
     }
     __syncthreads();
     if (blockIdx.x == 0)
@@ -779,13 +818,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 }
 
 // B <- L^{-1} B, one workgroup of eight waves per 16 columns held in LDS (up to 512 rows, parts
-// apart): per 64-row block X_b = inv(L_bb) B_b (waves 0..3), then the rows below -= L X_b in
-// tiles of 16 rows. The critical path calls it with 512 columns, so width is what spreads it:
-// 512 x 512 takes 32 workgroups and 85 us (160 us with 32 columns and four waves). Against one
-// substitution launch and one product per 64 rows before: 31 us each at 8 blocks of 64.
+// apart), as gemm.hip's trsm_lu_kernel: one wave solves the 64-row blocks from their solve forms,
+// seven subtract L X_b from the rows below in tiles of 16. The critical path calls it with 512
+// columns, so width is what spreads it: 512 x 512 takes 32 workgroups and 75 us alone (32
+// columns and four waves 160 us).
 constexpr int kCXStride = 17;
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void ctrsm_lu_kernel(
-    int K, int N, const float2* __restrict__ T, int64_t ldt, const float* __restrict__ linv, float2* __restrict__ B,
+    int K, int N, const float2* __restrict__ T, int64_t ldt, const float* __restrict__ forms, float2* __restrict__ B,
     int64_t ldb)
 {
     extern __shared__ __align__(16) float s_mem[];  // Kp rows of stride 17, real, then imaginary
@@ -804,79 +843,98 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void c
             xi[r * kCXStride + c] = v.y;
         }
     __syncthreads();
-    float2 lf[16];
-    auto loadTile = [&](int k0, int r0)
+    // They meet twice a block.
+    constexpr int UPD = 7;
+    if (wave == UPD)
     {
-        // Rows beyond K repeat the last one, columns beyond K (zero rows of X) likewise.
-        const float2* const Lc = T + k0 * ldt + min(r0 + ui, K - 1);
-        const int last = min(64, K - k0) - 1;
-#pragma unroll
-        for (int t = 0; t < 16; ++t) lf[t] = Lc[min(4 * t + uk, last) * ldt];
-    };
-    for (int b = 0; b < nblk; ++b)
-    {
-        const int k0 = b * 64;
-        int r0 = k0 + 64 + wave * 16;
-        if (r0 < K) loadTile(k0, r0);
-        f32x4 re = {0.0f, 0.0f, 0.0f, 0.0f}, im = re;
-        if (wave < 4)
+        CSolveOperands op;
+        LoadOperands(forms, ui, uk, op);
+        for (int b = 0; b < nblk; ++b)
         {
-            const float* const Lb = linv + static_cast<size_t>(b) * kCInverseBlock + 16 * wave + ui;
-            float lr[16], lx[16];
+            const int k0 = b * 64;
+            f32x4 re[4], im[4];
 #pragma unroll
-            for (int t = 0; t < 16; ++t)
-            {
-                lr[t] = Lb[(4 * t + uk) * 64];
-                lx[t] = Lb[4096 + (4 * t + uk) * 64];
-            }
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int t = 0; t < 16; ++t)
-            {
-                if (t >= 4 * (wave + 1)) continue;  // uniform: zeros of the triangle
-                const int at = (k0 + 4 * t + uk) * kCXStride + ui;
-                const float br = xr[at], bi = xi[at];
-                re = __builtin_amdgcn_mfma_f32_16x16x4f32(br, lr[t], re, 0, 0, 0);
-                im = __builtin_amdgcn_mfma_f32_16x16x4f32(bi, lr[t], im, 0, 0, 0);
-                re = __builtin_amdgcn_mfma_f32_16x16x4f32(-bi, lx[t], re, 0, 0, 0);
-                im = __builtin_amdgcn_mfma_f32_16x16x4f32(br, lx[t], im, 0, 0, 0);
-            }
-        }
-        __syncthreads();
-        if (wave < 4)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-            {
-                const int at = (k0 + 16 * wave + ui) * kCXStride + 4 * uk + r;
-                xr[at] = re[r];
-                xi[at] = im[r];
-            }
-        __syncthreads();
-        for (; r0 < K; r0 += 128)
-        {
-            f32x4 ar = {0.0f, 0.0f, 0.0f, 0.0f}, ai = ar;
-#pragma unroll
-            for (int t = 0; t < 16; ++t)
-            {
-                const int at = (k0 + 4 * t + uk) * kCXStride + ui;
-                const float ur = xr[at], ux = xi[at];
-                ar = __builtin_amdgcn_mfma_f32_16x16x4f32(ur, lf[t].x, ar, 0, 0, 0);
-                ai = __builtin_amdgcn_mfma_f32_16x16x4f32(ux, lf[t].x, ai, 0, 0, 0);
-                ar = __builtin_amdgcn_mfma_f32_16x16x4f32(-ux, lf[t].y, ar, 0, 0, 0);
-                ai = __builtin_amdgcn_mfma_f32_16x16x4f32(ur, lf[t].y, ai, 0, 0, 0);
-            }
-            const int row = r0 + ui;
-            if (r0 + 128 < K) loadTile(k0, r0 + 128);
-            if (row < K)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
+                for (int r = 0; r < 4; ++r)
                 {
-                    const int at = row * kCXStride + 4 * uk + v;
-                    xr[at] -= ar[v];
-                    xi[at] -= ai[v];
+                    const int at = (k0 + 16 * t + 4 * uk + r) * kCXStride + ui;
+                    re[t][r] = xr[at];
+                    im[t][r] = xi[at];
                 }
+            if (__builtin_expect(CSolveColumns(op, re, im), 1))  // uniform
+            {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                    {
+                        const int at = (k0 + 16 * t + 4 * uk + r) * kCXStride + ui;
+                        xr[at] = re[t][r];
+                        xi[at] = im[t][r];
+                    }
+            }
+            else
+            {
+                float2 v[16];
+#pragma unroll
+                for (int c = 0; c < 16; ++c)
+                    v[c] = make_float2(xr[(k0 + lane) * kCXStride + c], xi[(k0 + lane) * kCXStride + c]);
+                SubstituteColumns(T + k0 * ldt + k0, ldt, min(64, K - k0), lane, v);
+#pragma unroll
+                for (int c = 0; c < 16; ++c)
+                {
+                    xr[(k0 + lane) * kCXStride + c] = v[c].x;
+                    xi[(k0 + lane) * kCXStride + c] = v[c].y;
+                }
+            }
+            if (b + 1 < nblk) LoadOperands(forms + static_cast<size_t>(b + 1) * kCFormBlock, ui, uk, op);
+            __syncthreads();
+            __syncthreads();
         }
-        __syncthreads();
     }
+    else
+        for (int b = 0; b < nblk; ++b)
+        {
+            const int k0 = b * 64;
+            int r0 = k0 + 64 + wave * 16;
+            // Blocks with rows below them are full; rows beyond K repeat the last one.
+            float2 lf[16];
+            auto loadTile = [&]()
+            {
+                const float2* const Lc = T + k0 * ldt + min(r0 + ui, K - 1);
+#pragma unroll
+                for (int t = 0; t < 16; ++t) lf[t] = Lc[(4 * t + uk) * ldt];
+            };
+            if (r0 < K) loadTile();
+            __syncthreads();
+            while (r0 < K)
+            {
+                f32x4 ar = {0.0f, 0.0f, 0.0f, 0.0f}, ai = ar;
+#pragma unroll
+                for (int t = 0; t < 16; ++t)
+                {
+                    const int at = (k0 + 4 * t + uk) * kCXStride + ui;
+                    const float ur = xr[at], ux = xi[at];
+                    ar = __builtin_amdgcn_mfma_f32_16x16x4f32(ur, lf[t].x, ar, 0, 0, 0);
+                    ai = __builtin_amdgcn_mfma_f32_16x16x4f32(ux, lf[t].x, ai, 0, 0, 0);
+                    ar = __builtin_amdgcn_mfma_f32_16x16x4f32(-ux, lf[t].y, ar, 0, 0, 0);
+                    ai = __builtin_amdgcn_mfma_f32_16x16x4f32(ur, lf[t].y, ai, 0, 0, 0);
+                }
+                const int row = r0 + ui;
+                r0 += 16 * UPD;
+                if (r0 < K) loadTile();
+                if (row < K)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                    {
+                        const int at = row * kCXStride + 4 * uk + v;
+                        xr[at] -= ar[v];
+                        xi[at] -= ai[v];
+                    }
+            }
+            __syncthreads();
+        }
     for (int c = wave; c < nc; c += 8)
         for (int r = lane; r < K; r += 64)
             B[(c0 + c) * ldb + r] = make_float2(xr[r * kCXStride + c], xi[r * kCXStride + c]);
@@ -913,33 +971,33 @@ hipError_t CLeafColumns(const CLeafArgs& a, bool spread, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t CLeafFinish(const CLeafArgs& a, float* linv, float2* ub, hipStream_t stream)
+hipError_t CLeafFinish(const CLeafArgs& a, float* form, float2* ub, hipStream_t stream)
 {
     const int others = (a.c0 - a.j0) + (a.panelEnd - a.c0 - a.wact);
     hipLaunchKernelGGL(cleaf_finish_kernel, dim3(1 + (others + 3) / 4), dim3(256), 0, stream, a.A,
                        static_cast<int64_t>(a.lda), a.j0, a.c0, a.wact, a.panelEnd,
-                       reinterpret_cast<const int2*>(a.moves), a.err, linv, ub);
+                       reinterpret_cast<const int2*>(a.moves), a.err, form, ub);
     return hipGetLastError();
 }
 
-hipError_t CPanelUpdate(const CLeafArgs& a, const float* linv, const float2* ub, hipStream_t stream)
+hipError_t CPanelUpdate(const CLeafArgs& a, const float* form, const float2* ub, hipStream_t stream)
 {
     const int cols = a.panelEnd - a.c0 - kCLeafWidth, rows = a.m - a.c0 - kCLeafWidth;
     if (a.wact != kCLeafWidth) return hipErrorInvalidValue;
     if (cols <= 0) return hipSuccess;
     hipLaunchKernelGGL(cpanel_update_kernel, dim3(std::max(1, (rows + 63) / 64), (cols + 63) / 64), dim3(256), 0, stream,
-                       a.A, static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, linv, ub);
+                       a.A, static_cast<int64_t>(a.lda), a.m, a.c0, a.panelEnd, form, ub);
     return hipGetLastError();
 }
 
-hipError_t CTrsmLowerUnit(int K, int N, const float2* T, int ldt, const float* linv, float2* B, int ldb,
+hipError_t CTrsmLowerUnit(int K, int N, const float2* T, int ldt, const float* forms, float2* B, int ldb,
                           hipStream_t stream)
 {
     if (K <= 0 || N <= 0) return hipSuccess;
     if (K > 512) return hipErrorInvalidValue;
     const size_t lds = static_cast<size_t>((K + 63) / 64) * 64 * kCXStride * 2 * sizeof(float);
     hipLaunchKernelGGL(ctrsm_lu_kernel, dim3((N + 15) / 16), dim3(512), lds, stream, K, N, T, static_cast<int64_t>(ldt),
-                       linv, B, static_cast<int64_t>(ldb));
+                       forms, B, static_cast<int64_t>(ldb));
     return hipGetLastError();
 }
 }  // namespace ops

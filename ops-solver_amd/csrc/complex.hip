@@ -376,7 +376,7 @@ hipError_t CTrsmBlock(int K, int N, const float2* T, int ldt, bool lower, bool u
 // Workspace: ints [0, m) row sources, two moved-row lists of 4 CNB + 8 (panel k uses list
 // k % 2, so the look-ahead panel can build its list while the previous one is still being
 // applied), the leaf's moved rows; then, 8-byte aligned, the exchange words of the
-// multi-workgroup leaves, the rows a leaf's update takes, two panels' diagonal-block inverses and
+// multi-workgroup leaves, the rows a leaf's update takes, two panels' solve forms (unitlower.h) and
 // the timeout flag.
 constexpr int kCMovedInts = 4 * CNB + 8;
 inline int CPanelBlocks(int m) { return (std::min(m, CNB) + 63) / 64; }
@@ -387,14 +387,14 @@ struct CWork
     int* moves;
     unsigned long long* slots;
     float2* panelRows;
-    float* linv[2];
+    float* forms[2];
     int* err;
 };
 inline size_t CWorkInts(int m) { return static_cast<size_t>(m) + 2 * kCMovedInts + 4 * kCLeafWidth + 2; }
 inline size_t CWorkWords(int m)  // 8-byte words behind the ints
 {
     const size_t blocks = static_cast<size_t>(CPanelBlocks(m));
-    return kCLeafSlotWords + blocks * 64 * 64 + 2 * blocks * (kCInverseBlock / 2) + 1;
+    return kCLeafSlotWords + blocks * 64 * 64 + 2 * blocks * (kCFormBlock / 2) + 1;
 }
 CWork CLayout(void* base, int m)
 {
@@ -403,9 +403,9 @@ CWork CLayout(void* base, int m)
     uintptr_t q = (reinterpret_cast<uintptr_t>(base) + 7) & ~static_cast<uintptr_t>(7);
     w.slots = reinterpret_cast<unsigned long long*>(q);
     w.panelRows = reinterpret_cast<float2*>(w.slots + kCLeafSlotWords);
-    w.linv[0] = reinterpret_cast<float*>(w.panelRows + blocks * 64 * 64);
-    w.linv[1] = w.linv[0] + blocks * kCInverseBlock;
-    w.err = reinterpret_cast<int*>(w.linv[1] + blocks * kCInverseBlock);
+    w.forms[0] = reinterpret_cast<float*>(w.panelRows + blocks * 64 * 64);
+    w.forms[1] = w.forms[0] + blocks * kCFormBlock;
+    w.err = reinterpret_cast<int*>(w.forms[1] + blocks * kCFormBlock);
     w.moves = w.err + 2;
     w.moved[0] = w.moves + 4 * kCLeafWidth;
     w.moved[1] = w.moved[0] + kCMovedInts;
@@ -458,7 +458,7 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
     }
 
     // Panel k: per 64 columns one leaf, one launch that applies its interchanges to the whole
-    // panel and inverts its diagonal block, one that updates the panel columns to its right;
+    // panel and prepares its diagonal block, one that updates the panel columns to its right;
     // then the list of the panel's interchanges.
     auto panel = [&](int k) -> hipError_t
     {
@@ -484,10 +484,10 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
             l.tagBase = static_cast<unsigned>(c0 + kCLeafWidth);
             l.err = w.err;
             l.spinLimit = SpinLimit();
-            float* const linv = w.linv[k & 1] + static_cast<size_t>((c0 - j0) / 64) * kCInverseBlock;
+            float* const form = w.forms[k & 1] + static_cast<size_t>((c0 - j0) / 64) * kCFormBlock;
             CRET(CLeafColumns(l, LeafSpread(), s0));
-            CRET(CLeafFinish(l, linv, w.panelRows, s0));
-            if (c0 + l.wact < panelEnd) CRET(CPanelUpdate(l, linv, w.panelRows, s0));
+            CRET(CLeafFinish(l, form, w.panelRows, s0));
+            if (c0 + l.wact < panelEnd) CRET(CPanelUpdate(l, form, w.panelRows, s0));
         }
         if (pivoting && (k > 0 || panelEnd < n))
             hipLaunchKernelGGL(ccompact_moves_kernel, dim3(1), dim3(1024), 0, s0, m, j0, w.rowsrc, w.err,
@@ -505,7 +505,7 @@ hipError_t ComplexGetrf(int m, int n, float2* a, int lda, int* ipiv, int* info, 
                                hi, w.moved[k & 1]);
         CRET(hipGetLastError());
         if (cols <= 0) return hipSuccess;
-        CRET(CTrsmLowerUnit(nb, cols, a + static_cast<size_t>(j0) * lda + j0, lda, w.linv[k & 1],
+        CRET(CTrsmLowerUnit(nb, cols, a + static_cast<size_t>(j0) * lda + j0, lda, w.forms[k & 1],
                             a + static_cast<size_t>(lo) * lda + j0, lda, st));
         if (m - pe <= 0) return hipSuccess;
         ProfileScope prof(ProfileKernel::ComplexGemm, 8.0 * (m - pe) * cols * nb, st);

@@ -16,7 +16,7 @@ import aclsolver as A  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 EPS = 2.0 ** -24
-KINDS = [np.float32]
+KINDS = [np.float32, np.complex64]
 
 
 @pytest.fixture(scope="module")
