@@ -9,7 +9,11 @@
 // Tickets hand out the blocks in dependency order: the block with the lowest unfinished ticket
 // never waits for a workgroup that has not started. With the inverse in FP64 the block solve
 // rounds once; an FP32 inverse, applied once or with a step of refinement in FP32, erred more
-// than the substitution it replaces (Gaussian systems of order 64 to 4096, against 64 bits).
+// than the substitution it replaces (Gaussian systems of order 64 to 4096, against 64 bits). The
+// solve's backward error is that of a substitution in FP32 as long as Growth64 stays far below
+// 2^53 / 2^24; blocks above 2^20 (a zero or tiny pivot, multipliers of one sign) are substituted.
+// Factors of Gaussian, uniform and graded matrices of orders up to 2500 have 2^12 at most. It costs
+// 0.6 us of the preparation's 13 us at order 64.
 //
 // What bounds it: the chain, one device-wide trip, two products and a few barriers per 64
 // rows. 64 rows: the longest block whose inverse four waves apply from registers.
@@ -20,6 +24,7 @@
 #include <climits>
 
 #include "internal.h"
+#include "lanes.h"
 #include "permute.h"
 #include "trtri64.h"
 
@@ -44,11 +49,55 @@ struct Trs
     int* info;
     unsigned long long* pub;  // X words: [block][strip][row][column], 64 rows, strips of 16 CG columns
     double* inv;              // inverses of the diagonal blocks of op(L), op(U): row-major 64 x 64
-    int* bad;                 // per diagonal block: its inverse is not finite (2 nb ints)
+    int* bad;                 // per diagonal block: its inverse is too large to be used (2 nb ints)
     int* perm;
     unsigned* ticket;         // [2]
     unsigned spinLimit;
 };
+
+// (|E| |X| d)_i / d_i, d_i the largest entry of row i of E, for a block E and its inverse X: the
+// factor by which a solve with X may exceed the backward error |E| |x| of a substitution, in units
+// of X's own rounding. In two steps around the inversion by a workgroup of four waves, each followed
+// by a barrier of the caller's: first partial maxima of the rows, then their maxima; then the sums.
+// e: |E(lane, 16 wave + k)|; s_x: X, or X^T if flip, row-major; s_g: scratch of kGrowthScratch.
+// Each lane returns the factor of row `lane`.
+constexpr double kInverseGrowth64 = 1 << 20;
+constexpr int kGrowthScratch = 10 * 64;
+__device__ inline void PartialMaxima(const float (&e)[16], double* s_g, int tid)
+{
+    float part = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) part = fmaxf(part, e[k]);
+    s_g[tid] = part;
+}
+__device__ inline void RowMaxima(double* s_g, int tid)
+{
+    const int lane = tid & 63;
+    if ((tid >> 6) == 3)  // the wave with the least to do in the inversion
+        s_g[256 + lane] = fmax(fmax(s_g[lane], s_g[64 + lane]), fmax(s_g[128 + lane], s_g[192 + lane]));
+}
+__device__ inline double Growth64(const float (&e)[16], const double* s_x, double* s_g, bool flip, int tid)
+{
+    const int lane = tid & 63, wave = tid >> 6;
+    const double* const s_d = s_g + 4 * 64;
+    double* const s_w = s_g + 5 * 64;
+    double* const s_p = s_g + 6 * 64;
+    const double* const x = s_x + (flip ? lane : lane * kInvStride);
+    const int step = flip ? kInvStride : 1;
+    double part = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) part = fma(fabs(x[(16 * wave + k) * step]), s_d[16 * wave + k], part);
+    s_p[tid] = part;
+    __syncthreads();
+    if (wave == 0) s_w[lane] = (s_p[lane] + s_p[64 + lane]) + (s_p[128 + lane] + s_p[192 + lane]);
+    __syncthreads();
+    part = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) part = fma(static_cast<double>(e[k]), s_w[16 * wave + k], part);
+    s_g[tid] = part;
+    __syncthreads();
+    return ((s_g[lane] + s_g[64 + lane]) + (s_g[128 + lane] + s_g[192 + lane])) / s_d[lane];
+}
 
 // Preparation, by workgroup: 2 nb diagonal blocks inverted, the permutation (256 positions
 // each), the publication words cleared.
@@ -69,20 +118,32 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
         double* const s_l = s_mem;
         double* const s_i = s_mem + 64 * kInvStride;
         double* const s_t = s_i + 64 * kInvStride;
+        double* const s_g = s_t + 32 * kInvStride;
         const float* const T = p.lu + static_cast<size_t>(k0) * p.lda + k0;
         // Lower: the block; upper: its transpose. Rows beyond the block are the identity.
+        float e[16];  // op(T) by rows, for Growth64
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
             const int c = wave * 16 + k;
-            const float v = lane < kb && c < kb ? T[static_cast<size_t>(c) * p.lda + lane] : (lane == c ? 1.0f : 0.0f);
-            if (!upper)
-                s_l[lane * kInvStride + c] = lane > c ? v : 0.0;
-            else
-                s_l[c * kInvStride + lane] = lane <= c ? v : 0.0;
+            float v = lane < kb && c < kb ? T[static_cast<size_t>(c) * p.lda + lane] : 0.0f;
+            if (lane == c && (!upper || lane >= kb)) v = 1.0f;
+            if (upper ? lane > c : lane < c) v = 0.0f;
+            s_l[upper ? c * kInvStride + lane : lane * kInvStride + c] = v;
             s_i[lane * kInvStride + c] = 0.0;
+            e[k] = fabsf(v);
         }
+        if (p.trans != 0)  // uniform
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+            {
+                const int r = wave * 16 + k;
+                const bool in = lane < kb && r < kb && (upper ? r <= lane : r > lane);
+                e[k] = in ? fabsf(T[static_cast<size_t>(lane) * p.lda + r]) : (r == lane && (!upper || r >= kb) ? 1.0f : 0.0f);
+            }
+        PartialMaxima(e, s_g, tid);
         __syncthreads();
+        RowMaxima(s_g, tid);
         if (upper)
             InvertLower64<false>(s_l, s_i, s_t, tid);
         else
@@ -99,12 +160,9 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
             fine = fine && fabs(v) <= FLT_MAX;
             out[r * 64 + lane] = v;
         }
-        if (!__syncthreads_and(fine))
-        {
-            if (tid == 0) p.bad[b] = 1;
-        }
-        else if (tid == 0)
-            p.bad[b] = 0;
+        const double grow = Growth64(e, s_i, s_g, flip, tid);
+        fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
+        if (tid == 0) p.bad[b] = fine ? 0 : 1;
         return;
     }
     b -= 2 * nb;
@@ -318,30 +376,31 @@ __global__ __launch_bounds__(256) void trs_chain_kernel(Trs p, int nb, int strip
     }
     else
     {
-        // A zero pivot (or an inverse beyond the range): plain substitution, as LAPACK's.
+        // A zero pivot, or an inverse that is too large: plain substitution, as LAPACK's. Lane: row,
+        // NS / 4 columns a wave.
+        constexpr int PC = NS / 4;
+        const int64_t ld = p.lda;
+        const float* const T = p.lu + r0 * ld + r0;
+        float v[PC];
+#pragma unroll
+        for (int c = 0; c < PC; ++c) v[c] = s_r[lane * S + PC * wave + c];
+#pragma unroll 1
         for (int e = 0; e < 64; ++e)
         {
             const int k = BACK ? 63 - e : e;
             if (r0 + k >= p.n) continue;  // uniform
-            const float d = p.lu[static_cast<size_t>(r0 + k) * p.lda + r0 + k];
-            __syncthreads();
-            for (int at = tid; at < 64 * NS; at += 256)
+            const bool rest = (BACK ? lane < k : lane > k) && r0 + lane < p.n;
+            const float t = rest ? T[TRANS ? lane * ld + k : k * ld + lane] : 0.0f, d = T[k * ld + k];
+#pragma unroll
+            for (int c = 0; c < PC; ++c)
             {
-                const int r = at / NS, c = at - r * NS;
-                if (r == k) s_y[k * S + c] = UPPER ? s_r[k * S + c] / d : s_r[k * S + c];
-            }
-            __syncthreads();
-            for (int at = tid; at < 64 * NS; at += 256)
-            {
-                const int r = at / NS, c = at - r * NS;
-                if (r0 + r < p.n && (BACK ? r < k : r > k))
-                {
-                    const float t = TRANS ? p.lu[static_cast<size_t>(r0 + r) * p.lda + r0 + k]
-                                          : p.lu[static_cast<size_t>(r0 + k) * p.lda + r0 + r];
-                    s_r[r * S + c] = fmaf(-t, s_y[k * S + c], s_r[r * S + c]);
-                }
+                float x = ReadLane(v[c], k);
+                if (UPPER) x = x / d;
+                v[c] = rest ? fmaf(-t, x, v[c]) : (lane == k ? x : v[c]);
             }
         }
+#pragma unroll
+        for (int c = 0; c < PC; ++c) s_y[lane * S + PC * wave + c] = v[c];
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < CG; ++c) x0[c] = *reinterpret_cast<const f32x4*>(s_y + (16 * wave + li) * S + 16 * c + 4 * g);
@@ -438,7 +497,7 @@ hipError_t TrsSolve(int trans, int n, int nrhs, const float* lu, int lda, const 
     p.spinLimit = SpinLimit();
     const int np = ipiv != nullptr ? (n + 255) / 256 : 0;
     const int nz = static_cast<int>(std::min<size_t>((words + 1023) / 1024, 1024));
-    const size_t ldsBytes = std::max<size_t>((2 * 64 + 32) * kInvStride * sizeof(double), ipiv ? ((n + 3) & ~3) * sizeof(int) : 0);
+    const size_t ldsBytes = std::max<size_t>(((2 * 64 + 32) * kInvStride + kGrowthScratch) * sizeof(double), ipiv ? ((n + 3) & ~3) * sizeof(int) : 0);
     hipLaunchKernelGGL(trs_prep_kernel, dim3(2 * nb + np + nz), dim3(256), ldsBytes, stream, p, nb, np, words);
     if (trans == 0)
         cg == 1 ? Chains<false, 1>(p, nb, strips, stream) : Chains<false, 4>(p, nb, strips, stream);
