@@ -3,8 +3,9 @@
 // trans N / T / C).
 //
 // One launch per triangle, a workgroup per 64 rows and 16 right-hand sides; FP32 products with
-// the solved blocks, FP64 inverses of the diagonal blocks, blocks handed out by ticket in
-// dependency order, solved rows published as tagged words. Bound by the chain: one device-wide
+// the solved blocks, FP64 inverses of the diagonal blocks (or substitution where trs.hip's measure of
+// their growth says so), blocks handed out by ticket in dependency order, solved rows published as
+// tagged words. Bound by the chain: one device-wide
 // trip, two products and a few barriers per 64 rows, 8 us a block and triangle (n = 8192, one
 // right-hand side: 2.1 ms; 10.5 ms as two launches per block).
 #include "ctrs.h"
@@ -15,6 +16,7 @@
 
 #include "complex_math.h"
 #include "internal.h"
+#include "lanes.h"
 #include "permute.h"
 #include "trtri64.h"
 
@@ -40,7 +42,7 @@ struct CTrs
     int* info;
     unsigned long long* pub;  // [block][strip][part][row][column]
     double* inv;              // inverses of the diagonal blocks of op(L), op(U): row-major, parts 4096 apart
-    int* bad;                 // per diagonal block: its inverse is not finite (2 nb ints)
+    int* bad;                 // per diagonal block: its inverse is too large to be used (2 nb ints)
     int* perm;
     unsigned* ticket;         // [2]
     unsigned spinLimit;
@@ -122,6 +124,48 @@ __device__ inline void ZInvertLower64(double* s, int tid)
     __syncthreads();
 }
 
+// trs.hip's growth of an inverse in the norm |re| + |im|; s_x: X, or X^T if flip, lower triangular
+// with parts kZ apart.
+constexpr double kInverseGrowth64 = 1 << 20;
+constexpr int kGrowthScratch = 10 * 64;
+__device__ inline void PartialMaxima(const float (&e)[16], double* s_g, int tid)
+{
+    float part = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) part = fmaxf(part, e[k]);
+    s_g[tid] = part;
+}
+__device__ inline void RowMaxima(double* s_g, int tid)
+{
+    const int lane = tid & 63;
+    if ((tid >> 6) == 3)
+        s_g[256 + lane] = fmax(fmax(s_g[lane], s_g[64 + lane]), fmax(s_g[128 + lane], s_g[192 + lane]));
+}
+__device__ inline double ZGrowth64(const float (&e)[16], const double* s_x, double* s_g, bool flip, int tid)
+{
+    const int lane = tid & 63, wave = tid >> 6;
+    const double* const s_d = s_g + 4 * 64;
+    double* const s_w = s_g + 5 * 64;
+    double* const s_p = s_g + 6 * 64;
+    double part = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+    {
+        const int j = 16 * wave + k, at = flip ? j * kInvStride + lane : lane * kInvStride + j;
+        if (flip ? j >= lane : lane >= j) part = fma(fabs(s_x[at]) + fabs(s_x[kZ + at]), s_d[j], part);
+    }
+    s_p[tid] = part;
+    __syncthreads();
+    if (wave == 0) s_w[lane] = (s_p[lane] + s_p[64 + lane]) + (s_p[128 + lane] + s_p[192 + lane]);
+    __syncthreads();
+    part = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) part = fma(static_cast<double>(e[k]), s_w[16 * wave + k], part);
+    s_g[tid] = part;
+    __syncthreads();
+    return ((s_g[lane] + s_g[64 + lane]) + (s_g[128 + lane] + s_g[192 + lane])) / s_d[lane];
+}
+
 // Preparation, by workgroup: 2 nb diagonal blocks inverted, the permutation (256 positions
 // each), the publication words cleared.
 __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, size_t words)
@@ -135,19 +179,33 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
         const bool upper = b >= nb;
         const int k0 = (upper ? b - nb : b) * NBK, kb = min(NBK, p.n - k0);
         const float2* const T = p.lu + static_cast<size_t>(k0) * p.lda + k0;
+        double* const s_g = s_mem + 2 * kZ;
         // Lower: the block; upper: its transpose. Rows beyond the block are the identity.
+        float e[16];  // |op(T)| by rows, for ZGrowth64
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
             const int c = wave * 16 + k;
-            const float2 v = lane < kb && c < kb ? T[static_cast<size_t>(c) * p.lda + lane]
-                                                 : make_float2(lane == c ? 1.0f : 0.0f, 0.0f);
-            const bool in = upper ? lane <= c : lane > c;
+            float2 v = lane < kb && c < kb ? T[static_cast<size_t>(c) * p.lda + lane] : make_float2(0.0f, 0.0f);
+            if (lane == c && (!upper || lane >= kb)) v = make_float2(1.0f, 0.0f);
+            if (upper ? lane > c : lane < c) v = make_float2(0.0f, 0.0f);
             const int at = upper ? c * kInvStride + lane : lane * kInvStride + c;
-            s_mem[at] = in ? v.x : 0.0;
-            s_mem[kZ + at] = in ? v.y : 0.0;
+            s_mem[at] = v.x;
+            s_mem[kZ + at] = v.y;
+            e[k] = fabsf(v.x) + fabsf(v.y);
         }
+        if (p.trans != 0)  // uniform
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+            {
+                const int r = wave * 16 + k;
+                const bool in = lane < kb && r < kb && (upper ? r <= lane : r > lane);
+                const float2 v = in ? T[static_cast<size_t>(lane) * p.lda + r] : make_float2(0.0f, 0.0f);
+                e[k] = r == lane && (!upper || r >= kb) ? 1.0f : fabsf(v.x) + fabsf(v.y);
+            }
+        PartialMaxima(e, s_g, tid);
         __syncthreads();
+        RowMaxima(s_g, tid);
         if (upper)
             ZInvertLower64<false>(s_mem, tid);
         else
@@ -167,7 +225,8 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
             out[r * 64 + lane] = x;
             out[4096 + r * 64 + lane] = p.trans == 2 ? -y : y;
         }
-        fine = __syncthreads_and(fine);
+        const double grow = ZGrowth64(e, s_mem, s_g, flip, tid);
+        fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
         if (tid == 0) p.bad[b] = fine ? 0 : 1;
         return;
     }
@@ -364,40 +423,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
     }
     else
     {
-        // A zero pivot (or an inverse beyond the range): plain substitution, as LAPACK's.
+        // A zero pivot, or an inverse that is too large: plain substitution, as LAPACK's. Lane: row,
+        // four columns a wave.
+        const int64_t ld = p.lda;
+        const float2* const T = p.lu + r0 * ld + r0;
+        float2 v[NS / 4];
+#pragma unroll
+        for (int c = 0; c < NS / 4; ++c)
+        {
+            const int at = lane * S + NS / 4 * wave + c;
+            v[c] = make_float2(s_r[at], s_r[64 * S + at]);
+        }
+#pragma unroll 1
         for (int e = 0; e < 64; ++e)
         {
             const int k = BACK ? 63 - e : e;
             if (r0 + k >= p.n) continue;  // uniform
-            float2 d = p.lu[static_cast<size_t>(r0 + k) * p.lda + r0 + k];
+            const bool rest = (BACK ? lane < k : lane > k) && r0 + lane < p.n;
+            float2 d = T[k * ld + k], t = rest ? T[TRANS ? lane * ld + k : k * ld + lane] : make_float2(0.0f, 0.0f);
             d.y *= conj;
-            __syncthreads();
-            for (int at = tid; at < 64 * NS; at += 256)
+            t.y *= conj;
+#pragma unroll
+            for (int c = 0; c < NS / 4; ++c)
             {
-                const int r = at / NS, c = at - r * NS;
-                if (r == k)
-                {
-                    float2 v = make_float2(s_r[k * S + c], s_r[64 * S + k * S + c]);
-                    if (UPPER) v = Mul64(v, Recip64(d));
-                    s_y[k * S + c] = v.x;
-                    s_y[64 * S + k * S + c] = v.y;
-                }
+                float2 x = make_float2(ReadLane(v[c].x, k), ReadLane(v[c].y, k));
+                if (UPPER) x = Mul64(x, Recip64(d));
+                const float2 y = SubMul(v[c], t, x);
+                v[c] = rest ? y : (lane == k ? x : v[c]);
             }
-            __syncthreads();
-            for (int at = tid; at < 64 * NS; at += 256)
-            {
-                const int r = at / NS, c = at - r * NS;
-                if (r0 + r < p.n && (BACK ? r < k : r > k))
-                {
-                    float2 t = TRANS ? p.lu[static_cast<size_t>(r0 + r) * p.lda + r0 + k]
-                                     : p.lu[static_cast<size_t>(r0 + k) * p.lda + r0 + r];
-                    t.y *= conj;
-                    const float2 v = SubMul(make_float2(s_r[r * S + c], s_r[64 * S + r * S + c]), t,
-                                            make_float2(s_y[k * S + c], s_y[64 * S + k * S + c]));
-                    s_r[r * S + c] = v.x;
-                    s_r[64 * S + r * S + c] = v.y;
-                }
-            }
+        }
+#pragma unroll
+        for (int c = 0; c < NS / 4; ++c)
+        {
+            const int at = lane * S + NS / 4 * wave + c;
+            s_y[at] = v[c].x;
+            s_y[64 * S + at] = v[c].y;
         }
         __syncthreads();
         x0 = *reinterpret_cast<const f32x4*>(s_y + (16 * wave + li) * S + 4 * g);
@@ -483,7 +543,7 @@ hipError_t CTrsSolve(int trans, int n, int nrhs, const float2* lu, int lda, cons
     p.spinLimit = SpinLimit();
     const int np = ipiv != nullptr ? (n + 255) / 256 : 0;
     const int nz = static_cast<int>(std::min<size_t>((words + 1023) / 1024, 1024));
-    const size_t ldsBytes = std::max<size_t>(2 * kZ * sizeof(double), ipiv ? ((n + 3) & ~3) * sizeof(int) : 0);
+    const size_t ldsBytes = std::max<size_t>((2 * kZ + kGrowthScratch) * sizeof(double), ipiv ? ((n + 3) & ~3) * sizeof(int) : 0);
     hipLaunchKernelGGL(ctrs_prep_kernel, dim3(2 * nb + np + nz), dim3(256), ldsBytes, stream, p, nb, np, words);
     if (trans == 0)
         CChains<false>(p, nb, strips, stream);

@@ -14,7 +14,7 @@ for p in (ROOT, os.path.join(ROOT, "ops-solver_amd")):
 import aclsolver as A  # noqa: E402
 
 pytestmark = pytest.mark.gpu
-KINDS = [np.float32]
+KINDS = [np.float32, np.complex64]
 
 
 @pytest.fixture(scope="module")
