@@ -5,10 +5,9 @@
 // panel, swap+TRSM, trailing product per block). The MI355X design:
 //   * panel: a sequence of register-resident leaf factorizations (leaf.hip) of up to 64
 //     columns, one workgroup or, for tall panels, several.
-//   * the panel is halved recursively down to leaves; the interchanges of a leaf (a
-//     gather/scatter of the <= 128 moved rows) are applied to the other panel columns, and
-//     every split solves the right half's top rows with the left half's L11
-//     and updates the rest of the right half with one MFMA product.
+//   * the panel is right-looking by 64 columns: after a leaf, one launch applies its interchanges
+//     (a gather/scatter of the <= 128 moved rows) to all panel columns, and one solves for U
+//     and updates the columns right of it. With tournament pivoting it is halved recursively.
 //   * after the panel, the composed interchanges of all NB pivots are applied to every
 //     column outside the panel (one coalesced gather/scatter per column), then the NB x NB
 //     unit-lower TRSM on the U12 block and the MFMA trailing update A22 -= L21 * U12.
@@ -584,19 +583,24 @@ int SolveBlock(int n) { return n >= 4096 ? 256 : 128; }
 
 namespace
 {
-// Chained substitutions (trs.hip) or, for many right-hand sides of a large system, blocked
-// ones, whose 128 x 128 products then outrun the chain's; also where the chain's padding to 64
-// rows would waste memory, and for the few problems that the no-allocation entry point takes
-// and whose chain does not fit its array (it promises the results of the allocating one).
+// Chained substitutions (trs.hip) or, for many right-hand sides of a large system, blocked ones.
+// Microseconds, blocked and chained: n = 100, 1 rhs 72 and 24, 8192 rhs 101 and 55; n = 1000, 33 rhs 842
+// and 251, 8192 1252 and 500; n = 4096, 33 rhs 3740 and 1039, 2048 4989 and 1615, 8192 8638 and 5103
+// (transposed 10769 and 5374); n = 16384, 256 rhs 20061 and 5544. Up to 4096 the chain won at every
+// number of right-hand sides, above it was measured to 256. Blocked also where the chain's
+// padding to 64 rows would waste memory, and for the few problems that the no-allocation entry
+// point takes and whose chain does not fit its array (it promises the results of the
+// allocating one).
 bool UseTrs(int n, int nrhs)
 {
     if (n > 4096 && nrhs > 256) return false;
     if (n < 16 && nrhs > 1024) return false;
     return RealGetrsStagingBytes(n, nrhs) > ACLSOLVER_NOALLOC_SCRATCH_BYTES ||
-           TrsWorkspaceBytes(n, nrhs, true) <= kNoAllocArrayBytes;
+           TrsWorkspaceBytes(n, nrhs) <= kNoAllocArrayBytes;
 }
 }  // namespace
 
+// The term of the former chained solve of one right-hand side stays: the size is documented.
 size_t RealGetrsStagingBytes(int n, int nrhs)
 {
     const size_t vectors =
@@ -606,7 +610,7 @@ size_t RealGetrsStagingBytes(int n, int nrhs)
 
 size_t RealGetrsWorkspaceBytes(int n, int nrhs)
 {
-    return UseTrs(n, nrhs) ? TrsWorkspaceBytes(n, nrhs, true) : RealGetrsStagingBytes(n, nrhs);
+    return UseTrs(n, nrhs) ? TrsWorkspaceBytes(n, nrhs) : RealGetrsStagingBytes(n, nrhs);
 }
 
 // Triangular solves on a column-major n x nrhs block X (ldx) with packed LU factors.
@@ -717,7 +721,7 @@ hipError_t RealGetrs(int trans, int n, int nrhs, const float* lu, int lda, const
                      void* work, hipStream_t stream, int* info, bool chain)
 {
     if (n <= 0 || nrhs <= 0) return hipSuccess;
-    if (chain && UseTrs(n, nrhs)) return TrsSolve(trans, n, nrhs, lu, lda, ipiv, b, ldb, b, ldb, info, work, nullptr, stream);
+    if (chain && UseTrs(n, nrhs)) return TrsSolve(trans, n, nrhs, lu, lda, ipiv, b, ldb, info, work, stream);
     if (info != nullptr) FillInfo(info, 1, 0, stream);
     float* x = static_cast<float*>(work);
     int* perm = reinterpret_cast<int*>(x + static_cast<size_t>(n) * nrhs);

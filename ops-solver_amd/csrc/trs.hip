@@ -41,10 +41,9 @@ __device__ inline unsigned long long LoadWord(const unsigned long long* p)
 
 struct Trs
 {
-    int trans, n, nrhs, lda, lds, ldb;
+    int trans, n, nrhs, lda, ldb;
     const float* lu;
     const int* ipiv;
-    const float* src;  // null: the identity
     float* B;
     int* info;
     unsigned long long* pub;  // X words: [block][strip][row][column], 64 rows, strips of 16 CG columns
@@ -282,8 +281,7 @@ __global__ __launch_bounds__(256) void trs_chain_kernel(Trs p, int nb, int strip
                 if (SECOND)
                     v = __uint_as_float(static_cast<unsigned>(mine[col]));
                 else if (inRow && c0 + col < p.nrhs)
-                    v = p.src == nullptr ? (from == c0 + col ? 1.0f : 0.0f)
-                                         : p.src[static_cast<size_t>(c0 + col) * p.lds + from];
+                    v = p.B[static_cast<size_t>(c0 + col) * p.ldb + from];
                 rhs[c][r] = v;
             }
     }
@@ -449,23 +447,22 @@ void Chains(const Trs& p, int nb, int strips, hipStream_t stream)
 }
 
 size_t Up(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
-}  // namespace
-
-size_t TrsPublicationBytes(int n, int nrhs)
+size_t PublicationWords(int n, int nrhs)
 {
     const int ns = 16 * GroupsPerStrip(nrhs);
-    return static_cast<size_t>((n + NBK - 1) / NBK) * NBK * ((nrhs + ns - 1) / ns * ns) * sizeof(unsigned long long);
+    return static_cast<size_t>((n + NBK - 1) / NBK) * NBK * ((nrhs + ns - 1) / ns * ns);
 }
+}  // namespace
 
-size_t TrsWorkspaceBytes(int n, int nrhs, bool withPublication)
+size_t TrsWorkspaceBytes(int n, int nrhs)
 {
     const size_t nb = (n + NBK - 1) / NBK;
     return Up(2 * nb * 4096 * sizeof(double)) + Up(2 * nb * sizeof(int)) + Up(n * sizeof(int)) + 256 +
-           (withPublication ? Up(TrsPublicationBytes(n, nrhs)) : 0) + 256;
+           Up(PublicationWords(n, nrhs) * 8) + 256;
 }
 
-hipError_t TrsSolve(int trans, int n, int nrhs, const float* lu, int lda, const int* ipiv, const float* src, int lds,
-                    float* B, int ldb, int* info, void* work, void* pub, hipStream_t stream)
+hipError_t TrsSolve(int trans, int n, int nrhs, const float* lu, int lda, const int* ipiv, float* B, int ldb, int* info,
+                    void* work, hipStream_t stream)
 {
     if (n <= 0 || nrhs <= 0) return hipSuccess;
     if (n > kEngineMaxOrder) return hipErrorInvalidValue;
@@ -481,19 +478,17 @@ hipError_t TrsSolve(int trans, int n, int nrhs, const float* lu, int lda, const 
     p.n = n;
     p.nrhs = nrhs;
     p.lda = lda;
-    p.lds = lds;
     p.ldb = ldb;
     p.lu = lu;
     p.ipiv = ipiv;
-    p.src = src;
     p.B = B;
     p.info = info;
     p.inv = reinterpret_cast<double*>(take(static_cast<size_t>(2 * nb) * 4096 * sizeof(double)));
     p.bad = reinterpret_cast<int*>(take(static_cast<size_t>(2 * nb) * sizeof(int)));
     p.perm = reinterpret_cast<int*>(take(static_cast<size_t>(n) * sizeof(int)));
     p.ticket = reinterpret_cast<unsigned*>(take(256));
-    const size_t words = TrsPublicationBytes(n, nrhs) / sizeof(unsigned long long);
-    p.pub = reinterpret_cast<unsigned long long*>(pub != nullptr ? pub : take(words * sizeof(unsigned long long)));
+    const size_t words = PublicationWords(n, nrhs);
+    p.pub = reinterpret_cast<unsigned long long*>(take(words * sizeof(unsigned long long)));
     p.spinLimit = SpinLimit();
     const int np = ipiv != nullptr ? (n + 255) / 256 : 0;
     const int nz = static_cast<int>(std::min<size_t>((words + 1023) / 1024, 1024));
