@@ -3,8 +3,7 @@
 // trans N / T / C).
 //
 // One launch per triangle, a workgroup per 64 rows and 16 right-hand sides; FP32 products with
-// the solved blocks, FP64 inverses of the diagonal blocks (or substitution where trs.hip's measure of
-// their growth says so), blocks handed out by ticket in dependency order, solved rows published as
+// the solved blocks, FP64 inverses of the diagonal blocks (or substitution where growth.h says so), blocks handed out by ticket in dependency order, solved rows published as
 // tagged words. Bound by the chain: one device-wide
 // trip, two products and a few barriers per 64 rows, 8 us a block and triangle (n = 8192, one
 // right-hand side: 2.1 ms; 10.5 ms as two launches per block).
@@ -15,6 +14,7 @@
 #include <climits>
 
 #include "complex_math.h"
+#include "growth.h"
 #include "internal.h"
 #include "lanes.h"
 #include "permute.h"
@@ -124,48 +124,6 @@ __device__ inline void ZInvertLower64(double* s, int tid)
     __syncthreads();
 }
 
-// trs.hip's growth of an inverse in the norm |re| + |im|; s_x: X, or X^T if flip, lower triangular
-// with parts kZ apart.
-constexpr double kInverseGrowth64 = 1 << 20;
-constexpr int kGrowthScratch = 10 * 64;
-__device__ inline void PartialMaxima(const float (&e)[16], double* s_g, int tid)
-{
-    float part = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) part = fmaxf(part, e[k]);
-    s_g[tid] = part;
-}
-__device__ inline void RowMaxima(double* s_g, int tid)
-{
-    const int lane = tid & 63;
-    if ((tid >> 6) == 3)
-        s_g[256 + lane] = fmax(fmax(s_g[lane], s_g[64 + lane]), fmax(s_g[128 + lane], s_g[192 + lane]));
-}
-__device__ inline double ZGrowth64(const float (&e)[16], const double* s_x, double* s_g, bool flip, int tid)
-{
-    const int lane = tid & 63, wave = tid >> 6;
-    const double* const s_d = s_g + 4 * 64;
-    double* const s_w = s_g + 5 * 64;
-    double* const s_p = s_g + 6 * 64;
-    double part = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-    {
-        const int j = 16 * wave + k, at = flip ? j * kInvStride + lane : lane * kInvStride + j;
-        if (flip ? j >= lane : lane >= j) part = fma(fabs(s_x[at]) + fabs(s_x[kZ + at]), s_d[j], part);
-    }
-    s_p[tid] = part;
-    __syncthreads();
-    if (wave == 0) s_w[lane] = (s_p[lane] + s_p[64 + lane]) + (s_p[128 + lane] + s_p[192 + lane]);
-    __syncthreads();
-    part = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) part = fma(static_cast<double>(e[k]), s_w[16 * wave + k], part);
-    s_g[tid] = part;
-    __syncthreads();
-    return ((s_g[lane] + s_g[64 + lane]) + (s_g[128 + lane] + s_g[192 + lane])) / s_d[lane];
-}
-
 // Preparation, by workgroup: 2 nb diagonal blocks inverted, the permutation (256 positions
 // each), the publication words cleared.
 __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, size_t words)
@@ -181,7 +139,7 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
         const float2* const T = p.lu + static_cast<size_t>(k0) * p.lda + k0;
         double* const s_g = s_mem + 2 * kZ;
         // Lower: the block; upper: its transpose. Rows beyond the block are the identity.
-        float e[16];  // |op(T)| by rows, for ZGrowth64
+        float e[16];  // |re| + |im| of op(T) by rows, for Growth64
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
@@ -225,7 +183,12 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
             out[r * 64 + lane] = x;
             out[4096 + r * 64 + lane] = p.trans == 2 ? -y : y;
         }
-        const double grow = ZGrowth64(e, s_mem, s_g, flip, tid);
+        auto size = [&](int j)
+        {
+            const int at = flip ? j * kInvStride + lane : lane * kInvStride + j;
+            return (flip ? j >= lane : lane >= j) ? fabs(s_mem[at]) + fabs(s_mem[kZ + at]) : 0.0;
+        };
+        const double grow = Growth64(e, size, s_g, tid);
         fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
         if (tid == 0) p.bad[b] = fine ? 0 : 1;
         return;

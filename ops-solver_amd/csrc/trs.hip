@@ -23,6 +23,7 @@
 #include <cfloat>
 #include <climits>
 
+#include "growth.h"
 #include "internal.h"
 #include "lanes.h"
 #include "permute.h"
@@ -53,50 +54,6 @@ struct Trs
     unsigned* ticket;         // [2]
     unsigned spinLimit;
 };
-
-// (|E| |X| d)_i / d_i, d_i the largest entry of row i of E, for a block E and its inverse X: the
-// factor by which a solve with X may exceed the backward error |E| |x| of a substitution, in units
-// of X's own rounding. In two steps around the inversion by a workgroup of four waves, each followed
-// by a barrier of the caller's: first partial maxima of the rows, then their maxima; then the sums.
-// e: |E(lane, 16 wave + k)|; s_x: X, or X^T if flip, row-major; s_g: scratch of kGrowthScratch.
-// Each lane returns the factor of row `lane`.
-constexpr double kInverseGrowth64 = 1 << 20;
-constexpr int kGrowthScratch = 10 * 64;
-__device__ inline void PartialMaxima(const float (&e)[16], double* s_g, int tid)
-{
-    float part = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) part = fmaxf(part, e[k]);
-    s_g[tid] = part;
-}
-__device__ inline void RowMaxima(double* s_g, int tid)
-{
-    const int lane = tid & 63;
-    if ((tid >> 6) == 3)  // the wave with the least to do in the inversion
-        s_g[256 + lane] = fmax(fmax(s_g[lane], s_g[64 + lane]), fmax(s_g[128 + lane], s_g[192 + lane]));
-}
-__device__ inline double Growth64(const float (&e)[16], const double* s_x, double* s_g, bool flip, int tid)
-{
-    const int lane = tid & 63, wave = tid >> 6;
-    const double* const s_d = s_g + 4 * 64;
-    double* const s_w = s_g + 5 * 64;
-    double* const s_p = s_g + 6 * 64;
-    const double* const x = s_x + (flip ? lane : lane * kInvStride);
-    const int step = flip ? kInvStride : 1;
-    double part = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) part = fma(fabs(x[(16 * wave + k) * step]), s_d[16 * wave + k], part);
-    s_p[tid] = part;
-    __syncthreads();
-    if (wave == 0) s_w[lane] = (s_p[lane] + s_p[64 + lane]) + (s_p[128 + lane] + s_p[192 + lane]);
-    __syncthreads();
-    part = 0.0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) part = fma(static_cast<double>(e[k]), s_w[16 * wave + k], part);
-    s_g[tid] = part;
-    __syncthreads();
-    return ((s_g[lane] + s_g[64 + lane]) + (s_g[128 + lane] + s_g[192 + lane])) / s_d[lane];
-}
 
 // Preparation, by workgroup: 2 nb diagonal blocks inverted, the permutation (256 positions
 // each), the publication words cleared.
@@ -159,7 +116,9 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
             fine = fine && fabs(v) <= FLT_MAX;
             out[r * 64 + lane] = v;
         }
-        const double grow = Growth64(e, s_i, s_g, flip, tid);
+        const double* const x = s_i + (flip ? lane : lane * kInvStride);
+        const int step = flip ? kInvStride : 1;
+        const double grow = Growth64(e, [&](int j) { return fabs(x[j * step]); }, s_g, tid);
         fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
         if (tid == 0) p.bad[b] = fine ? 0 : 1;
         return;
