@@ -193,15 +193,25 @@ int CheckArrays(aclsolverHandle_t h, int n, const void* aArr, int lda, const voi
     return 0;
 }
 
+// Scratch of `own` bytes and, behind them, ComplexGetrs's: the chained solve's, or the smaller one of
+// the blocked solve where the device has no room for that.
+char* SolveScratch(aclsolverHandle_t h, size_t own, int n, int nrhs, bool* chain)
+{
+    void* work = HandleScratch(h, own + ComplexGetrsWorkspaceBytes(n, nrhs, true));
+    *chain = work != nullptr;
+    if (work == nullptr) work = HandleScratch(h, own + ComplexGetrsWorkspaceBytes(n, nrhs, false));
+    return static_cast<char*>(work);
+}
+
 // Factor-and-solve inverse of one matrix into C (used beyond the register kernels' orders).
 aclsolverStatus_t InverseByFactor(aclsolverHandle_t h, int n, const float2* a, int lda, const int* pivIn, bool factor,
                                   float2* c, int ldc, int* info)
 {
     hipStream_t s = Stream(h);
     const size_t luBytes = static_cast<size_t>(n) * n * sizeof(float2);
-    const size_t need = luBytes + static_cast<size_t>(n) * sizeof(int) + ComplexGetrfWorkspaceBytes(n, n) +
-                        ComplexGetrsWorkspaceBytes(n, n, true) + 1024;
-    char* base = static_cast<char*>(HandleScratch(h, need));
+    const size_t own = luBytes + static_cast<size_t>(n) * sizeof(int) + ComplexGetrfWorkspaceBytes(n, n) + 1024;
+    bool chain = true;
+    char* base = SolveScratch(h, own, n, n, &chain);
     if (base == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
     float2* lu = reinterpret_cast<float2*>(base);
     int* piv = reinterpret_cast<int*>(base + luBytes);
@@ -217,7 +227,7 @@ aclsolverStatus_t InverseByFactor(aclsolverHandle_t h, int n, const float2* a, i
     else
         hipLaunchKernelGGL(c_first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, lu, n, info);
     hipLaunchKernelGGL(c_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, c, ldc);
-    if (ComplexGetrs(0, n, n, lu, n, p, c, ldc, sw, s, info, true) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
+    if (ComplexGetrs(0, n, n, lu, n, p, c, ldc, sw, s, info, chain) != hipSuccess) return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();
 }
 }  // namespace
@@ -292,10 +302,11 @@ OPS_API aclsolverStatus_t aclsolverCgetrsDevice(aclsolverHandle_t handle, int tr
     hipStream_t s = Stream(handle);
     FillInfo(devInfo, 1, 0, s);
     if (n == 0 || nrhs == 0) return Launched();
-    void* work = HandleScratch(handle, ComplexGetrsWorkspaceBytes(n, nrhs, true));
+    bool chain = true;
+    void* work = SolveScratch(handle, 0, n, nrhs, &chain);
     if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
     if (ComplexGetrs(trans, n, nrhs, reinterpret_cast<const float2*>(dA), lda, devIpiv, reinterpret_cast<float2*>(dB),
-                     ldb, work, s, devInfo, true) != hipSuccess)
+                     ldb, work, s, devInfo, chain) != hipSuccess)
         return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();
 }

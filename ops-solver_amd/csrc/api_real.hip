@@ -282,6 +282,18 @@ OPS_API aclsolverStatus_t aclsolverSgetrfTournament(aclsolverHandle_t handle, in
 // ---------------------------------------------------------------------------------------
 // Device column-major getrs (EXTENSION)
 // ---------------------------------------------------------------------------------------
+namespace
+{
+// Scratch for RealGetrs: the chained solve's, or the smaller one of the blocked solve where the
+// device has no room for that.
+void* SolveScratch(aclsolverHandle_t h, int n, int nrhs, bool* chain)
+{
+    void* const work = HandleScratch(h, RealGetrsWorkspaceBytes(n, nrhs));
+    *chain = work != nullptr;
+    return work != nullptr ? work : HandleScratch(h, RealGetrsStagingBytes(n, nrhs));
+}
+}  // namespace
+
 OPS_API aclsolverStatus_t aclsolverSgetrsDevice(aclsolverHandle_t handle, int trans, int n, int nrhs, const float* dA,
                                                 int lda, const int* devIpiv, float* dB, int ldb, int* devInfo)
 {
@@ -307,13 +319,14 @@ OPS_API aclsolverStatus_t aclsolverSgetrsDevice(aclsolverHandle_t handle, int tr
         arg = 9;
     if (arg) return Invalid(handle, devInfo, 1, arg);
     hipStream_t s = Stream(handle);
-    void* work = n > 0 && nrhs > 0 ? HandleScratch(handle, RealGetrsWorkspaceBytes(n, nrhs)) : nullptr;
+    bool chain = true;
+    void* work = n > 0 && nrhs > 0 ? SolveScratch(handle, n, nrhs, &chain) : nullptr;
     if (work == nullptr)
     {
         FillInfo(devInfo, 1, 0, s);
         return n == 0 || nrhs == 0 ? Launched() : ACLSOLVER_STATUS_ALLOC_FAILED;
     }
-    if (RealGetrs(trans, n, nrhs, dA, lda, devIpiv, dB, ldb, work, s, devInfo) != hipSuccess)
+    if (RealGetrs(trans, n, nrhs, dA, lda, devIpiv, dB, ldb, work, s, devInfo, chain) != hipSuccess)
         return ACLSOLVER_STATUS_EXECUTION_FAILED;
     return Launched();
 }
@@ -524,7 +537,8 @@ OPS_API aclsolverStatus_t aclsolverSgetriBatched(aclsolverHandle_t handle, int n
         hipMemcpyAsync(out.data(), Carray, sizeof(uintptr_t) * batchSize, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return ACLSOLVER_STATUS_EXECUTION_FAILED;
-    void* work = HandleScratch(handle, RealGetrsWorkspaceBytes(n, n));
+    bool chain = true;
+    void* work = SolveScratch(handle, n, n, &chain);
     if (work == nullptr) return ACLSOLVER_STATUS_ALLOC_FAILED;
     for (int b = 0; b < batchSize; ++b)
     {
@@ -532,7 +546,7 @@ OPS_API aclsolverStatus_t aclsolverSgetriBatched(aclsolverHandle_t handle, int n
         float* c = reinterpret_cast<float*>(out[b]);
         hipLaunchKernelGGL(set_identity_kernel, dim3((n + 255) / 256, n), dim3(256), 0, s, n, c, ldc);
         if (RealGetrs(0, n, n, a, lda, PivotArray ? PivotArray + static_cast<size_t>(b) * n : nullptr, c, ldc, work,
-                      s, infoArray + b) != hipSuccess)
+                      s, infoArray + b, chain) != hipSuccess)
             return ACLSOLVER_STATUS_EXECUTION_FAILED;
         hipLaunchKernelGGL(first_zero_diag_kernel, dim3(1), dim3(256), 0, s, n, a, lda, infoArray + b);
     }
