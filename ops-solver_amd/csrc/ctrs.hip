@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
         const float2* const T = p.lu + static_cast<size_t>(k0) * p.lda + k0;
         double* const s_g = s_mem + 2 * kZ;
         // Lower: the block; upper: its transpose. Rows beyond the block are the identity.
-        float e[16];  // |re| + |im| of op(T) by rows, for Growth64
+        float part = 0.0f;
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
@@ -150,28 +150,35 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
             const int at = upper ? c * kInvStride + lane : lane * kInvStride + c;
             s_mem[at] = v.x;
             s_mem[kZ + at] = v.y;
-            e[k] = fabsf(v.x) + fabsf(v.y);
+            part = fmaxf(part, fabsf(v.x) + fabsf(v.y));
         }
+        // The maxima (|re| + |im|) of op(T)'s rows: T's own from the registers, its columns from LDS
+        // (before the inversion, which works in place).
+        const bool flip = upper != (p.trans != 0);
+        const int step = flip ? kInvStride : 1, first = flip ? lane : lane * kInvStride;
         if (p.trans != 0)  // uniform
+        {
+            __syncthreads();
+            part = 0.0f;
 #pragma unroll
             for (int k = 0; k < 16; ++k)
             {
-                const int r = wave * 16 + k;
-                const bool in = lane < kb && r < kb && (upper ? r <= lane : r > lane);
-                const float2 v = in ? T[static_cast<size_t>(lane) * p.lda + r] : make_float2(0.0f, 0.0f);
-                e[k] = r == lane && (!upper || r >= kb) ? 1.0f : fabsf(v.x) + fabsf(v.y);
+                const int at = first + (16 * wave + k) * step;
+                part = fmaxf(part, static_cast<float>(fabs(s_mem[at]) + fabs(s_mem[kZ + at])));
             }
-        PartialMaxima(e, s_g, tid);
+        }
+        s_g[tid] = part;
         __syncthreads();
-        RowMaxima(s_g, tid);
+        if (wave == 3)
+            RowMaxima(s_g)[lane] = fmax(fmax(s_g[lane], s_g[64 + lane]), fmax(s_g[128 + lane], s_g[192 + lane]));
         if (upper)
             ZInvertLower64<false>(s_mem, tid);
         else
             ZInvertLower64<true>(s_mem, tid);
         // Row-major inverse of op(T): L^-1 and (U^T)^-1 as they are, the other two transposed.
         double* const out = p.inv + static_cast<size_t>(b) * 8192;
-        const bool flip = upper != (p.trans != 0);
-        bool fine = true;
+        const double d = RowMaxima(s_g)[lane];
+        bool fine = true, small = true;
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
@@ -180,16 +187,29 @@ __global__ __launch_bounds__(256) void ctrs_prep_kernel(CTrs p, int nb, int np, 
             const bool in = flip ? lane >= r : r >= lane;
             const double x = in ? s_mem[at] : 0.0, y = in ? s_mem[kZ + at] : 0.0;
             fine = fine && fabs(x) <= FLT_MAX && fabs(y) <= FLT_MAX;
+            small = small && (fabs(x) + fabs(y)) * d <= kSmallInverse;
             out[r * 64 + lane] = x;
             out[4096 + r * 64 + lane] = p.trans == 2 ? -y : y;
         }
-        auto size = [&](int j)
+        if (!__syncthreads_and(fine && small))
         {
-            const int at = flip ? j * kInvStride + lane : lane * kInvStride + j;
-            return (flip ? j >= lane : lane >= j) ? fabs(s_mem[at]) + fabs(s_mem[kZ + at]) : 0.0;
-        };
-        const double grow = Growth64(e, size, s_g, tid);
-        fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
+            float e[16];  // op(T) by rows, again from memory
+#pragma unroll
+            for (int k = 0; k < 16; ++k)
+            {
+                const int r = p.trans ? wave * 16 + k : lane, c = p.trans ? lane : wave * 16 + k;
+                const bool in = r < kb && c < kb && (upper ? r <= c : r > c);
+                const float2 v = in ? T[static_cast<size_t>(c) * p.lda + r] : make_float2(0.0f, 0.0f);
+                e[k] = r == c && (!upper || r >= kb) ? 1.0f : fabsf(v.x) + fabsf(v.y);
+            }
+            auto size = [&](int j)
+            {
+                const int at = first + j * step;
+                return (flip ? j >= lane : lane >= j) ? fabs(s_mem[at]) + fabs(s_mem[kZ + at]) : 0.0;
+            };
+            const double grow = Growth64(e, size, s_g, tid);
+            fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
+        }
         if (tid == 0) p.bad[b] = fine ? 0 : 1;
         return;
     }

@@ -6,32 +6,22 @@ namespace ops
 {
 namespace
 {
-// (|E| |X| d)_i / d_i, d_i the largest entry of row i of E, for a block E and its inverse X: the
-// factor by which a solve with X may exceed the backward error |E| |x| of a substitution, in units
-// of X's own rounding. In two steps around the inversion by a workgroup of four waves, each followed
-// by a barrier of the caller's or the inversion's: first partial maxima of the rows, then their
-// maxima; then the sums. e: |E(lane, 16 wave + k)|; s_g: scratch of kGrowthScratch doubles.
+// The factor of row i is (|E| |X| d)_i / d_i, d_i the largest entry of row i of E, for a block E and
+// its inverse X: by so much may a solve with X exceed the backward error |E| |x| of a substitution, in
+// units of X's own rounding. Entries |X_jk| d_k <= kSmallInverse bound it by 64^2 times that
+// (|E_ij| <= d_i), so that it is computed for the odd block only.
 constexpr double kInverseGrowth64 = 1 << 20;
-constexpr int kGrowthScratch = 10 * 64;
-__device__ inline void PartialMaxima(const float (&e)[16], double* s_g, int tid)
-{
-    float part = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) part = fmaxf(part, e[k]);
-    s_g[tid] = part;
-}
-__device__ inline void RowMaxima(double* s_g, int tid)
-{
-    const int lane = tid & 63;
-    if ((tid >> 6) == 3)  // the wave with the least to do in the inversion
-        s_g[256 + lane] = fmax(fmax(s_g[lane], s_g[64 + lane]), fmax(s_g[128 + lane], s_g[192 + lane]));
-}
-// x(j): |X(lane, j)|. Returns the factor of row `lane`.
+constexpr double kSmallInverse = 1 << 8;
+constexpr int kGrowthScratch = 10 * 64;  // doubles; d lies in the fifth 64
+__device__ inline double* RowMaxima(double* s_g) { return s_g + 4 * 64; }
+
+// By a workgroup of four waves. e: |E(lane, 16 wave + k)|, x(j): |X(lane, j)|; d in place. Returns the
+// factor of row `lane`.
 template <typename F>
 __device__ inline double Growth64(const float (&e)[16], F x, double* s_g, int tid)
 {
     const int lane = tid & 63, wave = tid >> 6;
-    const double* const s_d = s_g + 4 * 64;
+    const double* const s_d = RowMaxima(s_g);
     double* const s_w = s_g + 5 * 64;
     double* const s_p = s_g + 6 * 64;
     double part = 0.0;

@@ -12,8 +12,7 @@
 // than the substitution it replaces (Gaussian systems of order 64 to 4096, against 64 bits). The
 // solve's backward error is that of a substitution in FP32 as long as Growth64 stays far below
 // 2^53 / 2^24; blocks above 2^20 (a zero or tiny pivot, multipliers of one sign) are substituted.
-// Factors of Gaussian, uniform and graded matrices of orders up to 2500 have 2^12 at most. It costs
-// 0.6 us of the preparation's 13 us at order 64.
+// Factors of Gaussian, uniform and graded matrices of orders up to 2500 have 2^12 at most.
 //
 // What bounds it: the chain, one device-wide trip, two products and a few barriers per 64
 // rows. 64 rows: the longest block whose inverse four waves apply from registers.
@@ -77,7 +76,6 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
         double* const s_g = s_t + 32 * kInvStride;
         const float* const T = p.lu + static_cast<size_t>(k0) * p.lda + k0;
         // Lower: the block; upper: its transpose. Rows beyond the block are the identity.
-        float e[16];  // op(T) by rows, for Growth64
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
@@ -87,39 +85,46 @@ __global__ __launch_bounds__(256) void trs_prep_kernel(Trs p, int nb, int np, si
             if (upper ? lane > c : lane < c) v = 0.0f;
             s_l[upper ? c * kInvStride + lane : lane * kInvStride + c] = v;
             s_i[lane * kInvStride + c] = 0.0;
-            e[k] = fabsf(v);
         }
-        if (p.trans != 0)  // uniform
-#pragma unroll
-            for (int k = 0; k < 16; ++k)
-            {
-                const int r = wave * 16 + k;
-                const bool in = lane < kb && r < kb && (upper ? r <= lane : r > lane);
-                e[k] = in ? fabsf(T[static_cast<size_t>(lane) * p.lda + r]) : (r == lane && (!upper || r >= kb) ? 1.0f : 0.0f);
-            }
-        PartialMaxima(e, s_g, tid);
         __syncthreads();
-        RowMaxima(s_g, tid);
+        // s_l is op(T) or, if flip, its transpose. The rows' maxima, in halves, beside the first phase
+        // of the inversion, which these two waves have no part in.
+        const bool flip = upper != (p.trans != 0);
+        const int step = flip ? kInvStride : 1, first = flip ? lane : lane * kInvStride;
+        if (wave >= 2)
+        {
+            double d = 0.0;
+#pragma unroll
+            for (int j = 0; j < 32; ++j) d = fmax(d, fabs(s_l[first + (32 * (wave - 2) + j) * step]));
+            s_g[64 * (wave - 2) + lane] = d;
+        }
         if (upper)
             InvertLower64<false>(s_l, s_i, s_t, tid);
         else
             InvertLower64<true>(s_l, s_i, s_t, tid);
         // Row-major inverse of op(T): L^-1 and (U^T)^-1 as they are, the other two transposed.
         double* const out = p.inv + static_cast<size_t>(b) * 4096;
-        const bool flip = upper != (p.trans != 0);
-        bool fine = true;
+        const double d = fmax(s_g[lane], s_g[64 + lane]);
+        bool fine = true, small = true;
 #pragma unroll
         for (int k = 0; k < 16; ++k)
         {
             const int r = wave * 16 + k;
             const double v = flip ? s_i[lane * kInvStride + r] : s_i[r * kInvStride + lane];
             fine = fine && fabs(v) <= FLT_MAX;
+            small = small && fabs(v) * d <= kSmallInverse;
             out[r * 64 + lane] = v;
         }
-        const double* const x = s_i + (flip ? lane : lane * kInvStride);
-        const int step = flip ? kInvStride : 1;
-        const double grow = Growth64(e, [&](int j) { return fabs(x[j * step]); }, s_g, tid);
-        fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
+        if (!__syncthreads_and(fine && small))
+        {
+            float e[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) e[k] = fabs(s_l[first + (16 * wave + k) * step]);
+            RowMaxima(s_g)[lane] = d;
+            __syncthreads();
+            const double grow = Growth64(e, [&](int j) { return fabs(s_i[first + j * step]); }, s_g, tid);
+            fine = __syncthreads_and(fine && grow <= kInverseGrowth64);
+        }
         if (tid == 0) p.bad[b] = fine ? 0 : 1;
         return;
     }
