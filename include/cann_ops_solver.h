@@ -110,8 +110,10 @@ extern "C"
     /* ---- EXTENSION without a counterpart in the reference: a solve that allocates nothing ----
      * For callers that cannot allocate device memory (code under stream/graph capture, tight
      * serving loops, harnesses that forbid hipMalloc): the same computation and results as
-     * aclsolverSgetrsDevice, with its staging (4*n*nrhs + 20*n bytes plus alignment) in a
-     * fixed per-GPU device array of ACLSOLVER_NOALLOC_SCRATCH_BYTES instead of handle scratch.
+     * aclsolverSgetrsDevice, in a fixed per-GPU device array of 36 MiB (reserved when the library
+     * is loaded) instead of handle scratch. It takes problems of which 4*n*nrhs + 20*n bytes (plus
+     * alignment) fit ACLSOLVER_NOALLOC_SCRATCH_BYTES; the rest of the array holds the chained
+     * solve's block inverses and published words.
      * Larger problems return INVALID_VALUE with devInfo = -2 (n alone too large) or -3
      * (n*nrhs too large). Every call on one GPU shares the array: calls that overlap on one
      * GPU (two streams or threads) race on it. */

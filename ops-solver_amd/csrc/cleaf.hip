@@ -821,7 +821,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
 // apart), as gemm.hip's trsm_lu_kernel: one wave solves the 64-row blocks from their solve forms,
 // seven subtract L X_b from the rows below in tiles of 16. The critical path calls it with 512
 // columns, so width is what spreads it: 512 x 512 takes 32 workgroups and 75 us alone (32
-// columns and four waves 160 us).
+// columns and four waves 160 us), 122 us on average beside the product of order 8192.
 constexpr int kCXStride = 17;
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void ctrsm_lu_kernel(
     int K, int N, const float2* __restrict__ T, int64_t ldt, const float* __restrict__ forms, float2* __restrict__ B,

@@ -11,9 +11,10 @@
 //   C3x16 n <= 192: column-cyclic, 3 rows per lane, 16 waves, 1 per item;
 //   C4x16 n <= 256: column-cyclic, 4 rows per lane, 16 waves, 1 per item.
 // Where there are enough of them, orders above 64 take vbrows.hip's kernels instead (one workgroup
-// per matrix: outputs the same, 20000 systems of orders 1..256 in 4.8 instead of 8.2 ms; the rule is
-// at CreatePlan). A plan's caller may give the configuration of each 16-wide size bin above 64:
-// then all go through the queue here.
+// per matrix; results the same up to rounding; the rule is at CreatePlan): 20000 systems of orders
+// 1..256 in 4.8 instead of 8.2 ms, 5.3 instead of 9.0 with the copies that restore their inputs. A
+// plan's caller may give the configuration of each 16-wide size bin above 64: then all go through
+// the queue here.
 // The last workgroup to leave re-arms the queue, so the queue needs no reset between launches.
 //
 // Column-cyclic kernel (one matrix per workgroup): lane l of every wave holds rows
@@ -1083,7 +1084,7 @@ aclsolverStatus_t CreatePlan(aclsolverHandle_t handle, int batchSize, const int*
     // The classes 193..256, 129..192 and 65..128 go to vbrows.hip where that is the faster: its
     // workgroups come in rounds of 4, 5 and 8 a compute unit, a round takes 2.33, 2.16 and 1.75 us
     // per order of its first matrix; an item of the queue 1.2 us per order, on the compute unit that
-    // is free. 250 systems of orders 20..200: 263 us through the queue, 882 otherwise; 1000 of
+    // is free. With input copies, 250 systems of orders 20..200: 263 us through the queue, 882 otherwise; 1000 of
     // 100..220: 642 and 775; 10000 of 10..120: 1010 and 843; 20000 of 1..256: 9.0 and 5.3 ms.
     std::vector<char> rows(batchSize, 0);
     const double perRound[3] = {2.33, 2.16, 1.75}, perItem = 1.2;
