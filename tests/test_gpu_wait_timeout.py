@@ -141,3 +141,26 @@ def test_getri_batched_reports_the_wait(handle, cplx, n):
     with no_polls():
         assert call() == (A.SUCCESS, [A.INFO_WAIT_TIMEOUT] * 3)
     assert call() == (A.SUCCESS, [0, 71, 0])
+
+
+@pytest.mark.parametrize("cplx", [0, 1])
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("nrhs", [1, 40])
+def test_device_solve_reports_the_wait(handle, cplx, trans, nrhs):
+    import torch
+
+    print(f"device getrs cplx={cplx} trans={trans} nrhs={nrhs}", flush=True)
+    n = 150
+    lu = A.to_device_cm(_diagonal(n, cplx))
+    info = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+    getrs = A.lib().aclsolverCgetrsDevice if cplx else A.lib().aclsolverSgetrsDevice
+
+    def call():
+        b = torch.ones(nrhs, n, dtype=lu.dtype, device="cuda")
+        st = getrs(handle.h, trans, n, nrhs, A.ptr(lu), n, None, A.ptr(b), n, A.ptr(info))
+        torch.cuda.synchronize()
+        return st, info.item(), bool(torch.isnan(torch.view_as_real(b) if cplx else b).any())
+
+    with no_polls():
+        assert call() == (A.SUCCESS, A.INFO_WAIT_TIMEOUT, True)
+    assert call() == (A.SUCCESS, 0, False)
