@@ -650,16 +650,20 @@ __device__ inline bool CSolveColumns(const CSolveOperands& o, f32x4 (&re)[4], f3
 __device__ inline void SubstituteColumns(const float2* __restrict__ T, int64_t ldt, int size, int lane, float2 (&v)[16])
 {
 #pragma unroll 1
-    for (int k = 0; k + 1 < size; ++k)
+    for (int k0 = 0; k0 < size; k0 += 8)
     {
-        const bool below = lane > k && lane < size;
-        const float2 l = below ? T[k * ldt + lane] : make_float2(0.0f, 0.0f);
+        float2 l[8];
 #pragma unroll
-        for (int c = 0; c < 16; ++c)
-        {
-            const float2 y = SubMul(v[c], l, make_float2(ReadLane(v[c].x, k), ReadLane(v[c].y, k)));
-            if (below) v[c] = y;
-        }
+        for (int e = 0; e < 8; ++e)
+            l[e] = lane > k0 + e && lane < size ? T[(k0 + e) * ldt + lane] : make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+            {
+                const float2 y = SubMul(v[c], l[e], make_float2(ReadLane(v[c].x, k0 + e), ReadLane(v[c].y, k0 + e)));
+                if (lane > k0 + e && lane < size) v[c] = y;
+            }
     }
 }
 

@@ -417,22 +417,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void c
             const int at = lane * S + NS / 4 * wave + c;
             v[c] = make_float2(s_r[at], s_r[64 * S + at]);
         }
+        // Eight columns' entries at a time, as in trs.hip.
+        const int last = p.n - 1 - r0;
 #pragma unroll 1
-        for (int e = 0; e < 64; ++e)
+        for (int e0 = 0; e0 < 64; e0 += 8)
         {
-            const int k = BACK ? 63 - e : e;
-            if (r0 + k >= p.n) continue;  // uniform
-            const bool rest = (BACK ? lane < k : lane > k) && r0 + lane < p.n;
-            float2 d = T[k * ld + k], t = rest ? T[TRANS ? lane * ld + k : k * ld + lane] : make_float2(0.0f, 0.0f);
-            d.y *= conj;
-            t.y *= conj;
+            float2 t[8], d[8];
 #pragma unroll
-            for (int c = 0; c < NS / 4; ++c)
+            for (int e = 0; e < 8; ++e)
             {
-                float2 x = make_float2(ReadLane(v[c].x, k), ReadLane(v[c].y, k));
-                if (UPPER) x = Mul64(x, Recip64(d));
-                const float2 y = SubMul(v[c], t, x);
-                v[c] = rest ? y : (lane == k ? x : v[c]);
+                const int k = BACK ? 63 - e0 - e : e0 + e;
+                const bool rest = (BACK ? lane < k : lane > k) && max(lane, k) <= last;
+                t[e] = rest ? T[TRANS ? lane * ld + k : k * ld + lane] : make_float2(0.0f, 0.0f);
+                d[e] = T[min(k, last) * ld + min(k, last)];
+                t[e].y *= conj;
+                d[e].y *= conj;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+            {
+                const int k = BACK ? 63 - e0 - e : e0 + e;
+                const bool rest = (BACK ? lane < k : lane > k) && max(lane, k) <= last;
+                const double2 r = Recip64(d[e]);
+#pragma unroll
+                for (int c = 0; c < NS / 4; ++c)
+                {
+                    float2 x = make_float2(ReadLane(v[c].x, k), ReadLane(v[c].y, k));
+                    if (UPPER) x = Mul64(x, r);
+                    const float2 y = SubMul(v[c], t[e], x);
+                    v[c] = rest ? y : (lane == k ? x : v[c]);
+                }
             }
         }
 #pragma unroll

@@ -346,19 +346,33 @@ __global__ __launch_bounds__(256) void trs_chain_kernel(Trs p, int nb, int strip
         float v[PC];
 #pragma unroll
         for (int c = 0; c < PC; ++c) v[c] = s_r[lane * S + PC * wave + c];
+        // Eight columns' entries at a time (their loads in flight together); those beyond the order
+        // change nothing.
+        const int last = p.n - 1 - r0;
 #pragma unroll 1
-        for (int e = 0; e < 64; ++e)
+        for (int e0 = 0; e0 < 64; e0 += 8)
         {
-            const int k = BACK ? 63 - e : e;
-            if (r0 + k >= p.n) continue;  // uniform
-            const bool rest = (BACK ? lane < k : lane > k) && r0 + lane < p.n;
-            const float t = rest ? T[TRANS ? lane * ld + k : k * ld + lane] : 0.0f, d = T[k * ld + k];
+            float t[8], d[8];
 #pragma unroll
-            for (int c = 0; c < PC; ++c)
+            for (int e = 0; e < 8; ++e)
             {
-                float x = ReadLane(v[c], k);
-                if (UPPER) x = x / d;
-                v[c] = rest ? fmaf(-t, x, v[c]) : (lane == k ? x : v[c]);
+                const int k = BACK ? 63 - e0 - e : e0 + e;
+                const bool rest = (BACK ? lane < k : lane > k) && max(lane, k) <= last;
+                t[e] = rest ? T[TRANS ? lane * ld + k : k * ld + lane] : 0.0f;
+                d[e] = T[min(k, last) * ld + min(k, last)];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+            {
+                const int k = BACK ? 63 - e0 - e : e0 + e;
+                const bool rest = (BACK ? lane < k : lane > k) && max(lane, k) <= last;
+#pragma unroll
+                for (int c = 0; c < PC; ++c)
+                {
+                    float x = ReadLane(v[c], k);
+                    if (UPPER) x = x / d[e];
+                    v[c] = rest ? fmaf(-t[e], x, v[c]) : (lane == k ? x : v[c]);
+                }
             }
         }
 #pragma unroll

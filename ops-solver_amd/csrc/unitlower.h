@@ -116,20 +116,23 @@ __device__ inline bool SolveColumns(const SolveOperands& o, f32x4 (&b)[4])
 }
 
 // The same by substitution for 16 columns of one wave, lane: row. T: the block in memory, rows and
-// columns from `size` on are the identity. 64 columns about 6 us, rarely taken.
+// columns from `size` on are the identity. Rarely taken; eight columns of T in flight together.
 __device__ inline void SubstituteColumns(const float* __restrict__ T, int64_t ldt, int size, int lane, float (&v)[16])
 {
 #pragma unroll 1
-    for (int k = 0; k + 1 < size; ++k)
+    for (int k0 = 0; k0 < size; k0 += 8)
     {
-        const bool below = lane > k && lane < size;
-        const float l = below ? T[k * ldt + lane] : 0.0f;
+        float l[8];
 #pragma unroll
-        for (int c = 0; c < 16; ++c)
-        {
-            const float x = ReadLane(v[c], k);
-            v[c] = below ? fmaf(-l, x, v[c]) : v[c];
-        }
+        for (int e = 0; e < 8; ++e) l[e] = lane > k0 + e && lane < size ? T[(k0 + e) * ldt + lane] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+            {
+                const float x = ReadLane(v[c], k0 + e);
+                v[c] = lane > k0 + e && lane < size ? fmaf(-l[e], x, v[c]) : v[c];
+            }
     }
 }
 }  // namespace
